@@ -150,79 +150,184 @@ __global__ __launch_bounds__(kUThreads) void conv_mfma_kernel(
 
 // ---------------------------------------------------------------------------
 // Weight gradient on matrix cores: dW[tap][co][ci] += sum_p gy[p][co] x[p+tap][ci]
-// (x read through upsampling when UPS).  Each workgroup accumulates its own
-// fp32 slot of ``part`` over a strided set of tiles; ``reduce`` sums slots.
+// (x read through upsampling when UPS): M = 16 output channels, N = 16 input
+// channels, K = 32 pixels of a row.
+//
+// The pixels are the contraction, so each tile (64 x 4 pixels, x with a one
+// pixel halo) is transposed into LDS as [channel][row][column]: an A fragment
+// is one 16-byte read, and one 16-byte and one 4-byte read give the B
+// fragments of all three taps of a row (the window shifted by 0, 1, 2
+// pixels with v_alignbit).  The channel pitches put the 16 channels of a
+// fragment read on different banks.  The 4 / RS waves of a row group share
+// out the (co, ci) block pairs, PW each, with the nine tap accumulators in
+// registers over all tiles of the block; with one or two pairs the rows are
+// split over RS groups instead and summed in LDS at the end.  Every block
+// writes its own fp32 slot of ``part`` once; reduce_slots_kernel sums them.
+// Bound: reading x and gy (16 channels: 16.8 MB at 512^2, ~3 us) and the
+// transposing LDS writes.  Measured: 16 -> 16 channels at 512^2 11 us, 48 -> 48
+// at 128^2 16 us (112 us each with 64 blocks gathering the fragments two bytes
+// at a time and adding every tile to the slot in memory).
 // ---------------------------------------------------------------------------
-template <bool UPS>
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kWXRow = 72, kWXPitch = (kUTh + 2) * kWXRow + 8;  // x: elements per row / channel
+constexpr int kWGPitch = kUTh * kUTw + 24;                      // gy: elements per channel
+
+// 4 pixels x 4 channels (one uint2 of channels per pixel) -> 4 uint2 of pixels.
+__device__ __forceinline__ void transpose4(const uint2 (&p)[4], uint2 (&c)[4]) {
+  c[0] = make_uint2((p[0].x & 0xffffu) | (p[1].x << 16), (p[2].x & 0xffffu) | (p[3].x << 16));
+  c[1] = make_uint2((p[0].x >> 16) | (p[1].x & 0xffff0000u),
+                    (p[2].x >> 16) | (p[3].x & 0xffff0000u));
+  c[2] = make_uint2((p[0].y & 0xffffu) | (p[1].y << 16), (p[2].y & 0xffffu) | (p[3].y << 16));
+  c[3] = make_uint2((p[0].y >> 16) | (p[1].y & 0xffff0000u),
+                    (p[2].y >> 16) | (p[3].y & 0xffff0000u));
+}
+
+template <int PW, int RS, bool UPS>
 __global__ __launch_bounds__(kUThreads) void conv_bwdw_mfma_kernel(
     const uint16_t* __restrict__ x, int Cin, const uint16_t* __restrict__ gy, int Cout,
     float* __restrict__ part, int H, int W, int tiles_x, int ntiles) {
-  extern __shared__ uint16_t smem[];
-  const int SW = kUTw + 2;
-  uint16_t* sx = smem;                                    // (TH+2) x SW x Cin
-  uint16_t* sg = smem + (int64_t)(kUTh + 2) * SW * Cin;   // TH x TW x Cout
-  const int COB = Cout / 16, CIB = Cin / 16;
-  const int nblk = 9 * COB * CIB;
-  float* mine = part + (int64_t)blockIdx.x * 9 * Cout * Cin;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  extern __shared__ __align__(16) uint16_t smem[];
+  uint16_t* sx = smem;                           // [Cin][TH + 2][kWXRow]
+  uint16_t* sg = smem + (int64_t)Cin * kWXPitch;  // [Cout][TH][TW]
+  constexpr int NWP = 4 / RS, ROWS = kUTh / RS;
+  const int COB = Cout / 16, CIB = Cin / 16, NP = COB * CIB;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wp = wave % NWP, rs = wave / NWP;
   const int lrow = lane & 15, lgrp = lane >> 4;
   const int Wx = UPS ? W / 2 : W;
+  f32x4 acc[PW][9];
+#pragma unroll
+  for (int k = 0; k < PW; ++k)
+#pragma unroll
+    for (int q = 0; q < 9; ++q) acc[k][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const int i0 = (t % tiles_x) * kUTw, j0 = (t / tiles_x) * kUTh;
     __syncthreads();
     const int c4x = Cin / 4;
-    for (int k = tid; k < (kUTh + 2) * SW * c4x; k += kUThreads) {
-      const int pix = k / c4x, c4 = k % c4x;
-      const int ry = pix / SW, rx = pix % SW;
-      const int gyy = j0 - 1 + ry, gxx = i0 - 1 + rx;
-      uint2 v = make_uint2(0u, 0u);
-      if (gyy >= 0 && gyy < H && gxx >= 0 && gxx < W) {
-        const int sy = UPS ? (gyy >> 1) : gyy, sxx = UPS ? (gxx >> 1) : gxx;
-        v = *reinterpret_cast<const uint2*>(x + ((int64_t)sy * Wx + sxx) * Cin + 4 * c4);
+    for (int k = tid; k < (kUTh + 2) * 17 * c4x; k += kUThreads) {
+      const int c4 = k % c4x, u = k / c4x, g = u % 17, ry = u / 17;
+      const int gyy = j0 - 1 + ry;
+      uint2 px[4], ch[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int gxx = i0 - 1 + 4 * g + e;
+        px[e] = make_uint2(0u, 0u);
+        if (gyy >= 0 && gyy < H && gxx >= 0 && gxx < W) {
+          const int sy = UPS ? (gyy >> 1) : gyy, sxx = UPS ? (gxx >> 1) : gxx;
+          px[e] = *reinterpret_cast<const uint2*>(x + ((int64_t)sy * Wx + sxx) * Cin + 4 * c4);
+        }
       }
-      *reinterpret_cast<uint2*>(sx + (int64_t)pix * Cin + 4 * c4) = v;
+      transpose4(px, ch);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        *reinterpret_cast<uint2*>(sx + (4 * c4 + e) * kWXPitch + ry * kWXRow + 4 * g) = ch[e];
     }
     const int c4g = Cout / 4;
-    for (int k = tid; k < kUTh * kUTw * c4g; k += kUThreads) {
-      const int pix = k / c4g, c4 = k % c4g;
-      const int ry = pix / kUTw, rx = pix % kUTw;
-      const int gyy = j0 + ry, gxx = i0 + rx;
-      uint2 v = make_uint2(0u, 0u);
-      if (gyy < H && gxx < W)
-        v = *reinterpret_cast<const uint2*>(gy + ((int64_t)gyy * W + gxx) * Cout + 4 * c4);
-      *reinterpret_cast<uint2*>(sg + (int64_t)pix * Cout + 4 * c4) = v;
+    for (int k = tid; k < kUTh * (kUTw / 4) * c4g; k += kUThreads) {
+      const int c4 = k % c4g, u = k / c4g, g = u % (kUTw / 4), ry = u / (kUTw / 4);
+      const int gyy = j0 + ry;
+      uint2 px[4], ch[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int gxx = i0 + 4 * g + e;
+        px[e] = (gyy < H && gxx < W) ? *reinterpret_cast<const uint2*>(
+                                           gy + ((int64_t)gyy * W + gxx) * Cout + 4 * c4)
+                                     : make_uint2(0u, 0u);
+      }
+      transpose4(px, ch);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        *reinterpret_cast<uint2*>(sg + (4 * c4 + e) * kWGPitch + ry * kUTw + 4 * g) = ch[e];
     }
     __syncthreads();
-    for (int b = wave; b < nblk; b += 4) {
-      const int cib = b % CIB, cob = (b / CIB) % COB, tap = b / (CIB * COB);
-      const int ky = tap / 3, kx = tap % 3;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      for (int kb = 0; kb < (kUTh * kUTw) / 16; ++kb) {
-        bf16x4 a, bb;
+    for (int rk = 0; rk < 2 * ROWS; ++rk) {
+      const int r = rs * ROWS + (rk >> 1), col = 32 * (rk & 1) + 8 * lgrp;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int pix = kb * 16 + 4 * lgrp + i;
-          const int ry = pix / kUTw, rx = pix % kUTw;
-          a[i] = (short)sg[(int64_t)pix * Cout + cob * 16 + lrow];
-          bb[i] = (short)sx[((int64_t)(ry + ky) * SW + rx + kx) * Cin + cib * 16 + lrow];
+      for (int k = 0; k < PW; ++k) {
+        const int p = wp + NWP * k;
+        if (p < NP) {
+          const int cob = p / CIB, cib = p - cob * CIB;
+          const bf16x8 a =
+              *reinterpret_cast<const bf16x8*>(sg + (cob * 16 + lrow) * kWGPitch + r * kUTw + col);
+#pragma unroll
+          for (int ky = 0; ky < 3; ++ky) {
+            const uint16_t* b =
+                sx + (cib * 16 + lrow) * kWXPitch + (r + ky) * kWXRow + col;
+            const uint4 lo = *reinterpret_cast<const uint4*>(b);
+            const uint32_t hi = *reinterpret_cast<const uint32_t*>(b + 8);
+            const uint4 b1 = make_uint4(__builtin_amdgcn_alignbit(lo.y, lo.x, 16),
+                                        __builtin_amdgcn_alignbit(lo.z, lo.y, 16),
+                                        __builtin_amdgcn_alignbit(lo.w, lo.z, 16),
+                                        __builtin_amdgcn_alignbit(hi, lo.w, 16));
+            const uint4 b2 = make_uint4(lo.y, lo.z, lo.w, hi);
+            acc[k][3 * ky] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a, __builtin_bit_cast(bf16x8, lo), acc[k][3 * ky], 0, 0, 0);
+            acc[k][3 * ky + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a, __builtin_bit_cast(bf16x8, b1), acc[k][3 * ky + 1], 0, 0, 0);
+            acc[k][3 * ky + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a, __builtin_bit_cast(bf16x8, b2), acc[k][3 * ky + 2], 0, 0, 0);
+          }
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, acc, 0, 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int co = cob * 16 + 4 * lgrp + i, ci = cib * 16 + lrow;
-        mine[((int64_t)tap * Cout + co) * Cin + ci] += acc[i];
       }
     }
   }
+  if constexpr (RS > 1) {
+    f32x4* sr = reinterpret_cast<f32x4*>(smem);  // [(RS - 1) * NWP][PW * 9][64]
+    __syncthreads();
+    if (rs > 0) {
+#pragma unroll
+      for (int k = 0; k < PW; ++k)
+#pragma unroll
+        for (int q = 0; q < 9; ++q)
+          sr[(((rs - 1) * NWP + wp) * PW * 9 + k * 9 + q) * 64 + lane] = acc[k][q];
+    }
+    __syncthreads();
+    if (rs > 0) return;
+    for (int o = 0; o < RS - 1; ++o)
+#pragma unroll
+      for (int k = 0; k < PW; ++k)
+#pragma unroll
+        for (int q = 0; q < 9; ++q)
+          acc[k][q] += sr[((o * NWP + wp) * PW * 9 + k * 9 + q) * 64 + lane];
+  }
+  float* mine = part + (int64_t)blockIdx.x * 9 * Cout * Cin;
+#pragma unroll
+  for (int k = 0; k < PW; ++k) {
+    const int p = wp + NWP * k;
+    if (p >= NP) continue;
+    const int cob = p / CIB, cib = p - cob * CIB;
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        mine[((int64_t)q * Cout + cob * 16 + 4 * lgrp + i) * Cin + cib * 16 + lrow] = acc[k][q][i];
+  }
 }
 
-__global__ void reduce_slots_kernel(const float* __restrict__ part, int nslot, int n,
-                                    float* __restrict__ out, int accumulate) {
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int g = 0; g < nslot; ++g) s += part[(int64_t)g * n + e];
-    out[e] = accumulate ? out[e] + s : s;
+// out[e] (+)= sum over slots of part[g][e], 64 elements a block: 16 wavefronts
+// take every 16th slot (independent loads in flight; with one thread per
+// element the 64 slots were a 15 us chain), then sum in LDS in wave order.
+constexpr int kRedWaves = 16;
+__global__ __launch_bounds__(64 * kRedWaves) void reduce_slots_kernel(
+    const float* __restrict__ part, int nslot, int n, float* __restrict__ out, int accumulate) {
+  __shared__ float red[kRedWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int e = blockIdx.x * 64 + lane;
+  float s = 0.f;
+  if (e < n) {
+#pragma unroll 8
+    for (int g = wave; g < nslot; g += kRedWaves) s += part[(int64_t)g * n + e];
+  }
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && e < n) {
+    float v = 0.f;
+#pragma unroll
+    for (int k = 0; k < kRedWaves; ++k) v += red[k][lane];
+    out[e] = accumulate ? out[e] + v : v;
   }
 }
 
@@ -291,7 +396,8 @@ __global__ void conv_last_kernel(const uint16_t* __restrict__ d, const float* __
   y[(int64_t)j * ld_y + i] = (TO)s;
 }
 
-// g_d[q][c] = (d[q][c] > 0) * sum_tap w[tap][c] gy[q - tap]
+// g_d[q][c] = (d[q][c] > 0) * sum_tap w[tap][c] gy[q - tap]; 8 channels per
+// 16-byte load and store (one channel at a time: 24 us at 512^2, 16 channels).
 __global__ void conv_last_bwd_data_kernel(const float* __restrict__ gy, const float* __restrict__ w,
                                           int C, const uint16_t* __restrict__ d,
                                           uint16_t* __restrict__ gd, int H, int W) {
@@ -304,46 +410,90 @@ __global__ void conv_last_bwd_data_kernel(const float* __restrict__ gy, const fl
     g[t] = (y >= 0 && y < H && x >= 0 && x < W) ? gy[(int64_t)y * W + x] : 0.f;
   }
   const int64_t q = (int64_t)j * W + i;
-  for (int c = 0; c < C; ++c) {
-    float s = 0.f;
+  for (int c8 = 0; c8 < C; c8 += 8) {
+    const uint4 dv = *reinterpret_cast<const uint4*>(d + q * C + c8);
+    const uint32_t du[4] = {dv.x, dv.y, dv.z, dv.w};
+    uint32_t pk[4];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) s += w[t * C + c] * g[t];
-    gd[q * C + c] = f2bf(bf2f(d[q * C + c]) > 0.f ? s : 0.f);
+    for (int h = 0; h < 4; ++h) {
+      float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+      for (int t = 0; t < 9; ++t) {
+        s0 += w[t * C + c8 + 2 * h] * g[t];
+        s1 += w[t * C + c8 + 2 * h + 1] * g[t];
+      }
+      s0 = bf2f((uint16_t)(du[h] & 0xffffu)) > 0.f ? s0 : 0.f;
+      s1 = bf2f((uint16_t)(du[h] >> 16)) > 0.f ? s1 : 0.f;
+      pk[h] = (uint32_t)f2bf(s0) | ((uint32_t)f2bf(s1) << 16);
+    }
+    *reinterpret_cast<uint4*>(gd + q * C + c8) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
   }
 }
 
-// Per-block partial sums of dW[tap][c] = sum_p a[p] * b[p + tap][c] (a fp32
-// single channel, b bf16 C channels) or, with swap, sum_p a[p][c] b[p + tap]
-// (a bf16 C channels, b fp32 single channel).  part: [nblk][9*C].
+// Per-block partial sums of the one-channel layers' weight gradients, FP32:
+// dW[tap][c] = sum_q sc[q][c] s1[q - sgn tap] (sgn = +1: s1 is the gradient of
+// the output layer and sc its input; sgn = -1: s1 is the input field and sc
+// the gradient of the first layer).  A thread owns 8 channels of every
+// (256 * 8 / C)-th pixel of its block: one 16-byte load of sc and nine of s1
+// feed its 72 register sums, where one pass over both fields per (tap, c)
+// took 846 us at 512^2 with 16 channels (now 34 us).  part: [nblk][9 * C].
 __global__ __launch_bounds__(256) void edge_bwdw_kernel(const float* __restrict__ s1,
-                                                         const uint16_t* __restrict__ sc, int C,
-                                                         int swap, float* __restrict__ part,
-                                                         int H, int W) {
-  __shared__ float red[256];
-  const int tid = threadIdx.x;
+                                                        const uint16_t* __restrict__ sc, int C,
+                                                        int sgn, float* __restrict__ part, int H,
+                                                        int W) {
+  __shared__ float red[4][9 * 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int cg = C / 8;  // threads per pixel: 2, 4, 6 or 8
+  const int ppw = 64 / cg;  // pixels per wavefront pass (6 groups: 10, four lanes idle)
+  const int c8 = lane % cg, pl = lane / cg;
   const int64_t N = (int64_t)H * W;
   const int64_t per = (N + gridDim.x - 1) / gridDim.x;
   const int64_t p0 = (int64_t)blockIdx.x * per, p1 = min(N, p0 + per);
-  for (int e = 0; e < 9 * C; ++e) {
-    const int t = e / C, c = e % C;
-    const int dy = t / 3 - 1, dx = t % 3 - 1;
-    float acc = 0.f;
-    for (int64_t p = p0 + tid; p < p1; p += 256) {
-      const int j = (int)(p / W), i = (int)(p % W);
-      const int y = j + dy, x = i + dx;
-      if (y < 0 || y >= H || x < 0 || x >= W) continue;
-      const int64_t q = (int64_t)y * W + x;
-      acc += swap ? bf2f(sc[p * C + c]) * s1[q] : s1[p] * bf2f(sc[q * C + c]);
+  float acc[9][8];
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int h = 0; h < 8; ++h) acc[t][h] = 0.f;
+  if (pl < ppw) {
+    for (int64_t p = p0 + wave * ppw + pl; p < p1; p += 4 * ppw) {
+      const int j = (int)((uint32_t)p / (uint32_t)W), i = (int)((uint32_t)p % (uint32_t)W);
+      const uint4 v = *reinterpret_cast<const uint4*>(sc + p * C + 8 * c8);
+      const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+      float f[8];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        f[2 * h] = bf2f((uint16_t)(u[h] & 0xffffu));
+        f[2 * h + 1] = bf2f((uint16_t)(u[h] >> 16));
+      }
+#pragma unroll
+      for (int t = 0; t < 9; ++t) {
+        const int y = j - sgn * (t / 3 - 1), x = i - sgn * (t % 3 - 1);
+        const bool in = y >= 0 && y < H && x >= 0 && x < W;
+        const float g = in ? s1[(int64_t)y * W + x] : 0.f;
+#pragma unroll
+        for (int h = 0; h < 8; ++h) acc[t][h] += g * f[h];
+      }
     }
-    red[tid] = acc;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if (tid < s) red[tid] += red[tid + s];
-      __syncthreads();
-    }
-    if (tid == 0) part[(int64_t)blockIdx.x * 9 * C + e] = red[0];
-    __syncthreads();
   }
+  // Sum over the lanes of one channel group (stride cg; power-of-two groups
+  // by butterflies, six groups through their first lanes).
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int h = 0; h < 8; ++h) {
+      float s = acc[t][h];
+      if (cg != 6) {
+        for (int o = 32; o >= cg; o >>= 1) s += __shfl_xor(s, o);
+      } else {
+        float r = s;
+        for (int k = 1; k < 10; ++k) r += __shfl(s, min(lane + 6 * k, 63));
+        s = r;
+      }
+      if (lane < cg) red[wave][t * C + 8 * c8 + h] = s;
+    }
+  __syncthreads();
+  for (int e = tid; e < 9 * C; e += 256)
+    part[(int64_t)blockIdx.x * 9 * C + e] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
 }
 
 // ---------------------------------------------------------------------------
@@ -613,24 +763,39 @@ static int unet_forward(UNet& N, int H, int W, hipStream_t s, bool last = true) 
   return kOk;
 }
 
+// Blocks of a weight-gradient launch: two per CU (each writes a slot that the
+// reduction reads back, so more only add traffic).
+constexpr int kBwdwBlocks = 512;
+
+template <int PW, int RS, bool UPS>
+static void launch_bwdw(UNet& N, const Layer& Ly, const uint16_t* x, const uint16_t* gyt, int G,
+                        int H, int W, int tx, int nt, hipStream_t s) {
+  const size_t stage = ((size_t)Ly.cin * kWXPitch + (size_t)Ly.cout * kWGPitch) * sizeof(uint16_t);
+  const size_t sums = (size_t)(RS - 1) * (4 / RS) * PW * 9 * 64 * sizeof(f32x4);
+  hipLaunchKernelGGL((conv_bwdw_mfma_kernel<PW, RS, UPS>), dim3(G), dim3(kUThreads),
+                     std::max(stage, sums), s, x, Ly.cin, gyt, Ly.cout, N.part, H, W, tx, nt);
+}
+
 static int bwdw_launch(UNet& N, int li, const uint16_t* x, const uint16_t* gyt, bool ups, int H,
                        int W, hipStream_t s) {
   const Layer& Ly = N.layers[li];
   const int tx = cdiv(W, kUTw), ty = cdiv(H, kUTh), nt = tx * ty;
-  const int G = std::min(nt, 64);
   const size_t n = (size_t)9 * Ly.cout * Ly.cin;
-  FVX_CHECK_ARG((size_t)G * n <= N.part_elems, "gradient scratch too small");
-  FVX_HIP(hipMemsetAsync(N.part, 0, (size_t)G * n * sizeof(float), s));
-  const size_t lds = ((size_t)(kUTh + 2) * (kUTw + 2) * Ly.cin + (size_t)kUTh * kUTw * Ly.cout) *
-                     sizeof(uint16_t);
-  if (ups)
-    hipLaunchKernelGGL(conv_bwdw_mfma_kernel<true>, dim3(G), dim3(kUThreads), lds, s, x, Ly.cin,
-                       gyt, Ly.cout, N.part, H, W, tx, nt);
-  else
-    hipLaunchKernelGGL(conv_bwdw_mfma_kernel<false>, dim3(G), dim3(kUThreads), lds, s, x, Ly.cin,
-                       gyt, Ly.cout, N.part, H, W, tx, nt);
-  hipLaunchKernelGGL(reduce_slots_kernel, g1((int64_t)n), dim3(256), 0, s, N.part, G, (int)n,
-                     N.g + Ly.off, 1);
+  const int G = (int)std::min<size_t>(std::min(nt, kBwdwBlocks), N.part_elems / n);
+  FVX_CHECK_ARG(G >= 1, "gradient scratch too small");
+  const int np = (Ly.cout / 16) * (Ly.cin / 16);  // (co, ci) block pairs, 1 .. 16
+#define FVX_BWDW(PW, RS)                                                          \
+  (ups ? launch_bwdw<PW, RS, true>(N, Ly, x, gyt, G, H, W, tx, nt, s)             \
+       : launch_bwdw<PW, RS, false>(N, Ly, x, gyt, G, H, W, tx, nt, s))
+  if (np == 1) FVX_BWDW(1, 4);
+  else if (np == 2) FVX_BWDW(1, 2);
+  else if (np <= 4) FVX_BWDW(1, 1);
+  else if (np <= 8) FVX_BWDW(2, 1);
+  else if (np <= 12) FVX_BWDW(3, 1);
+  else FVX_BWDW(4, 1);
+#undef FVX_BWDW
+  hipLaunchKernelGGL(reduce_slots_kernel, dim3(cdiv((int)n, 64)), dim3(64 * kRedWaves), 0, s,
+                     N.part, G, (int)n, N.g + Ly.off, 1);
   FVX_LAUNCH_CHECK();
   return kOk;
 }
@@ -638,12 +803,13 @@ static int bwdw_launch(UNet& N, int li, const uint16_t* x, const uint16_t* gyt, 
 static int edge_bwdw(UNet& N, int li, const float* s1, const uint16_t* sc, int C, bool swap,
                      int H, int W, hipStream_t s) {
   const Layer& Ly = N.layers[li];
-  const int G = 64;
+  const int64_t px = (int64_t)H * W;
+  const int G = (int)std::min<int64_t>((px + 255) / 256, kBwdwBlocks);
   const size_t n = (size_t)9 * C;
-  hipLaunchKernelGGL(edge_bwdw_kernel, dim3(G), dim3(256), 0, s, s1, sc, C, swap ? 1 : 0, N.part,
+  hipLaunchKernelGGL(edge_bwdw_kernel, dim3(G), dim3(256), 0, s, s1, sc, C, swap ? -1 : 1, N.part,
                      H, W);
-  hipLaunchKernelGGL(reduce_slots_kernel, g1((int64_t)n), dim3(256), 0, s, N.part, G, (int)n,
-                     N.g + Ly.off, 1);
+  hipLaunchKernelGGL(reduce_slots_kernel, dim3(cdiv((int)n, 64)), dim3(64 * kRedWaves), 0, s,
+                     N.part, G, (int)n, N.g + Ly.off, 1);
   FVX_LAUNCH_CHECK();
   return kOk;
 }
@@ -796,10 +962,18 @@ int fvx_unet_create(int nlev, const int* channels, int H, int W, void** out) {
   rc |= dev_alloc(*N, &N->loss, 1);
   if (!rc) {
     const int big = 160 * 1024;
-    (void)hipFuncSetAttribute((const void*)conv_bwdw_mfma_kernel<true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, big);
-    (void)hipFuncSetAttribute((const void*)conv_bwdw_mfma_kernel<false>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, big);
+#define FVX_BWDW_LDS(PW, RS)                                                          \
+  (void)hipFuncSetAttribute((const void*)conv_bwdw_mfma_kernel<PW, RS, true>,         \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, big);         \
+  (void)hipFuncSetAttribute((const void*)conv_bwdw_mfma_kernel<PW, RS, false>,        \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, big)
+    FVX_BWDW_LDS(1, 4);
+    FVX_BWDW_LDS(1, 2);
+    FVX_BWDW_LDS(1, 1);
+    FVX_BWDW_LDS(2, 1);
+    FVX_BWDW_LDS(3, 1);
+    FVX_BWDW_LDS(4, 1);
+#undef FVX_BWDW_LDS
     hipError_t e = hipMemset(N->g, 0, off * sizeof(float));
     if (e == hipSuccess) e = hipMemset(N->m, 0, off * sizeof(float));
     if (e == hipSuccess) e = hipMemset(N->v, 0, off * sizeof(float));

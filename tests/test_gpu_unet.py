@@ -83,3 +83,27 @@ def test_training_reduces_loss():
     for _ in range(60):
         l1 = net.train_step(xb, eb, 1e-3)
     assert l1 < 0.5 * l0, (l0, l1)
+
+
+@pytest.mark.parametrize("channels", [(16,), (32,), (48,), (64,), (16, 32), (32, 64), (64, 48)])
+@pytest.mark.parametrize("H,W", [(6, 62), (10, 130)])
+def test_weight_gradients_at_tile_edges(channels, H, W):
+    """Every (co, ci) block split of the weight-gradient kernel and both
+    one-channel layers on fields that end inside a 64 x 4 tile.  Each stored
+    tensor on the way to a gradient may differ from the oracle's by one bf16
+    ulp (2^-8 relative); there are 4 per level, so the Frobenius distance is
+    within 4 * levels * 2^-8.  A tile edge read wrongly moves it by > 0.1."""
+    need_gpu()
+    net = Lm.UNet(channels, H, W, seed=3)
+    Wt = {k: (v if k in ("e0a", "out") else Lm.to_bf16(v).astype(np.float64))
+          for k, v in net.get_weights().items()}
+    rng = np.random.default_rng(4)
+    x = Lm.to_bf16(rng.standard_normal((H, W))).astype(np.float64)
+    gy = Lm.to_bf16(rng.standard_normal((H, W))).astype(np.float64)
+    _, cache = U.forward(Wt, x, channels, bf16=True)
+    ref = U.backward(Wt, cache, gy, channels, bf16=True)
+    got = net.grads(torch.tensor(x, device="cuda"), torch.tensor(gy, device="cuda"))
+    tol = 4 * len(channels) * 2.0**-8
+    for k in ref:
+        err = np.linalg.norm(got[k] - ref[k]) / np.linalg.norm(ref[k])
+        assert err <= tol, (k, err)
