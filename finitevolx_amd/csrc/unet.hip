@@ -7,9 +7,9 @@
 // the 1-channel input / output handled by dedicated FP32 kernels.  Convs with
 // Cin, Cout multiples of 16 are implicit GEMMs on
 // v_mfma_f32_16x16x16_bf16: M = Cout, N = 16 pixels of a row, K = 16
-// input channels of one tap; a workgroup (4 waves) owns a 64 x 4 pixel tile
-// whose input (+1 halo, optionally read through nearest upsampling) is
-// staged in LDS; weights are pre-packed into per-lane MFMA fragments.
+// input channels of one tap; a workgroup owns a tile of 4 rows whose input
+// (+1 halo, optionally read through nearest upsampling) is staged in LDS;
+// weights are pre-packed into per-lane MFMA fragments.
 
 #include <cmath>
 #include <cstring>
@@ -61,89 +61,117 @@ __global__ void pack_weights_kernel(const float* __restrict__ w, uint16_t* __res
 
 // ---------------------------------------------------------------------------
 // 3x3 conv on matrix cores.  out = epi(sum_tap W x), epi: + skip, relu,
-// * (maskt > 0).  UPS: x is (H/2, W/2) and read through nearest upsampling.
+// * (maskt > 0).  ups: x is (H/2, W/2) and read through nearest upsampling.
+//
+// A workgroup owns a tile of 16 NB x 4 pixels; its COB * RG waves take one
+// block of 16 output channels and 4 / RG rows each.  The layers hold too little
+// work to be bound by anything but latency (64 -> 64 channels at 64^2: 36
+// matrix instructions per SIMD), so a launch is arranged as one round of
+// loads: every wave requests its 9 CIB weight fragments (each reused on its
+// rows x NB pixel blocks) and its share of the input tile together, then the
+// tile goes to LDS (pixel pitch Cin + 8: the 16 pixels of a fragment read lie
+// on different banks) and the matrix instructions run from registers and LDS.
+// NB = 1 where NB = 4 would leave CUs idle (conv_launch).  Measured: 64 -> 64
+// channels at 64^2 7.8 us, 48 -> 48 at 128^2 6.7 us, 16 -> 16 at 512^2 9.9 us
+// (one wave per row with the weights fetched between the matrix instructions:
+// 31.5, 23.8 and 14.5 us).
 // ---------------------------------------------------------------------------
-template <int COB, bool UPS>
-__global__ __launch_bounds__(kUThreads) void conv_mfma_kernel(
-    const uint16_t* __restrict__ x, int Cin, const bf16x4* __restrict__ wp,
-    uint16_t* __restrict__ out, const uint16_t* __restrict__ skip,
-    const uint16_t* __restrict__ maskt, int relu, int H, int W, int tiles_x, int ntiles,
-    const int* __restrict__ guard) {
+constexpr int conv_row_groups(int cob) { return cob == 1 ? 4 : cob == 2 ? 2 : 1; }
+constexpr int conv_threads(int cob) { return 64 * cob * conv_row_groups(cob); }
+
+template <int COB, int CIB, int NB>
+__global__ __launch_bounds__(conv_threads(COB)) void conv_mfma_kernel(
+    const uint16_t* __restrict__ x, const bf16x4* __restrict__ wp, uint16_t* __restrict__ out,
+    const uint16_t* __restrict__ skip, const uint16_t* __restrict__ maskt, int relu, int ups, int H,
+    int W, int tiles_x, int ntiles, const int* __restrict__ guard) {
   if (guard && *guard) return;
-  extern __shared__ uint16_t sx[];
-  constexpr int Cout = COB * 16;
-  const int CIB = Cin / 16;
-  const int SW = kUTw + 2;
+  constexpr int RG = conv_row_groups(COB), RPW = kUTh / RG, NT = conv_threads(COB);
+  constexpr int Cin = CIB * 16, Cout = COB * 16, SW = 16 * NB + 2, PITCH = Cin + 8;
+  constexpr int CPP = Cin / 8;  // 16-byte chunks per pixel
+  constexpr int NCH = (kUTh + 2) * SW * CPP, PER = (NCH + NT - 1) / NT;
+  __shared__ __align__(16) uint16_t sx[(kUTh + 2) * SW * PITCH];
   const int t = xcd_swizzle(blockIdx.x, ntiles);
-  const int i0 = (t % tiles_x) * kUTw, j0 = (t / tiles_x) * kUTh;
-  const int tid = threadIdx.x;
-  const int Hx = UPS ? H / 2 : H, Wx = UPS ? W / 2 : W;
-  const int c4n = Cin / 4;
-  const int nchunk = (kUTh + 2) * SW * c4n;
-  for (int k = tid; k < nchunk; k += kUThreads) {
-    const int pix = k / c4n, c4 = k % c4n;
-    const int ry = pix / SW, rx = pix % SW;
-    const int gy = j0 - 1 + ry, gx = i0 - 1 + rx;
-    uint2 v = make_uint2(0u, 0u);
-    if (gy >= 0 && gy < H && gx >= 0 && gx < W) {
-      const int sy = UPS ? (gy >> 1) : gy, sxx = UPS ? (gx >> 1) : gx;
-      v = *reinterpret_cast<const uint2*>(x + ((int64_t)sy * Wx + sxx) * Cin + 4 * c4);
-    }
-    *reinterpret_cast<uint2*>(sx + (int64_t)pix * Cin + 4 * c4) = v;
+  const int i0 = (t % tiles_x) * (16 * NB), j0 = (t / tiles_x) * kUTh;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cob = wave % COB, r0 = (wave / COB) * RPW;
+  const int lrow = lane & 15, lgrp = lane >> 4;
+  const int Wx = W >> ups;
+
+  bf16x4 afrag[9][CIB];
+#pragma unroll
+  for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+    for (int cib = 0; cib < CIB; ++cib)
+      afrag[tap][cib] = wp[((tap * COB + cob) * CIB + cib) * 64 + lane];
+  uint4 st[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = tid + k * NT, pix = c / CPP, c8 = c % CPP;
+    const int gy = j0 - 1 + pix / SW, gx = i0 - 1 + pix % SW;
+    st[k] = make_uint4(0u, 0u, 0u, 0u);
+    if (c < NCH && gy >= 0 && gy < H && gx >= 0 && gx < W)
+      st[k] = *reinterpret_cast<const uint4*>(
+          x + ((int64_t)(gy >> ups) * Wx + (gx >> ups)) * Cin + 8 * c8);
   }
-  (void)Hx;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = tid + k * NT;
+    if (c < NCH) *reinterpret_cast<uint4*>(sx + (c / CPP) * PITCH + 8 * (c % CPP)) = st[k];
+  }
   __syncthreads();
 
-  const int wave = tid >> 6, lane = tid & 63;
-  const int lrow = lane & 15, lgrp = lane >> 4;
-  f32x4 acc[COB][4];
+  f32x4 acc[RPW][NB];
 #pragma unroll
-  for (int a = 0; a < COB; ++a)
+  for (int r = 0; r < RPW; ++r)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int nb = 0; nb < NB; ++nb) acc[r][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+    for (int cib = 0; cib < CIB; ++cib)
+#pragma unroll
+      for (int r = 0; r < RPW; ++r)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const int pix = (r0 + r + tap / 3) * SW + nb * 16 + lrow + tap % 3;
+          const bf16x4 b =
+              *reinterpret_cast<const bf16x4*>(sx + pix * PITCH + cib * 16 + 4 * lgrp);
+          acc[r][nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(afrag[tap][cib], b, acc[r][nb], 0,
+                                                                 0, 0);
+        }
 
-  for (int tap = 0; tap < 9; ++tap) {
-    const int ky = tap / 3, kx = tap % 3;
-    for (int cib = 0; cib < CIB; ++cib) {
-      bf16x4 bfrag[4];
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        const int col = nb * 16 + lrow;
-        const int64_t off = ((int64_t)(wave + ky) * SW + (col + kx)) * Cin + cib * 16 + 4 * lgrp;
-        bfrag[nb] = *reinterpret_cast<const bf16x4*>(sx + off);
+  for (int r = 0; r < RPW; ++r) {
+    const int gy = j0 + r0 + r;
+    if (gy >= H) continue;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int gx = i0 + nb * 16 + lrow;
+      if (gx >= W) continue;
+      const int64_t o = ((int64_t)gy * W + gx) * Cout + cob * 16 + 4 * lgrp;
+      float v[4] = {acc[r][nb][0], acc[r][nb][1], acc[r][nb][2], acc[r][nb][3]};
+      if (skip) {
+        const uint2 k = *reinterpret_cast<const uint2*>(skip + o);
+        v[0] += bf2f((uint16_t)(k.x & 0xffffu));
+        v[1] += bf2f((uint16_t)(k.x >> 16));
+        v[2] += bf2f((uint16_t)(k.y & 0xffffu));
+        v[3] += bf2f((uint16_t)(k.y >> 16));
       }
+      if (relu) {
 #pragma unroll
-      for (int cob = 0; cob < COB; ++cob) {
-        const bf16x4 afrag = wp[((tap * COB + cob) * CIB + cib) * 64 + lane];
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
-          acc[cob][nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(afrag, bfrag[nb], acc[cob][nb],
-                                                                   0, 0, 0);
+        for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.f);
       }
-    }
-  }
-
-  const int gy = j0 + wave;
-  if (gy >= H) return;
-#pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
-    const int gx = i0 + nb * 16 + lrow;
-    if (gx >= W) continue;
-    const int64_t p = (int64_t)gy * W + gx;
-#pragma unroll
-    for (int cob = 0; cob < COB; ++cob) {
-      const int c0 = cob * 16 + 4 * lgrp;
-      uint16_t o4[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v = acc[cob][nb][i];
-        if (skip) v += bf2f(skip[p * Cout + c0 + i]);
-        if (relu) v = fmaxf(v, 0.f);
-        if (maskt) v = (bf2f(maskt[p * Cout + c0 + i]) > 0.f) ? v : 0.f;
-        o4[i] = f2bf(v);
+      if (maskt) {
+        const uint2 k = *reinterpret_cast<const uint2*>(maskt + o);
+        v[0] = bf2f((uint16_t)(k.x & 0xffffu)) > 0.f ? v[0] : 0.f;
+        v[1] = bf2f((uint16_t)(k.x >> 16)) > 0.f ? v[1] : 0.f;
+        v[2] = bf2f((uint16_t)(k.y & 0xffffu)) > 0.f ? v[2] : 0.f;
+        v[3] = bf2f((uint16_t)(k.y >> 16)) > 0.f ? v[3] : 0.f;
       }
-      *reinterpret_cast<uint2*>(out + p * Cout + c0) =
-          make_uint2((uint32_t)o4[0] | ((uint32_t)o4[1] << 16), (uint32_t)o4[2] | ((uint32_t)o4[3] << 16));
+      *reinterpret_cast<uint2*>(out + o) =
+          make_uint2((uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
+                     (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
     }
   }
 }
@@ -701,24 +729,32 @@ static void conv_launch(const UNet& N, int li, bool transposed, const uint16_t* 
   const Layer& Ly = N.layers[li];
   const int cout = transposed ? Ly.cin : Ly.cout, cin = transposed ? Ly.cout : Ly.cin;
   const bf16x4* wp = (const bf16x4*)((transposed ? N.wpkT : N.wpk) + N.pk_off[li]);
-  const int tx = cdiv(W, kUTw), ty = cdiv(H, kUTh);
-  const size_t lds = (size_t)(kUTh + 2) * (kUTw + 2) * cin * sizeof(uint16_t);
-#define FVX_CONV(COB, UP)                                                                     \
-  hipLaunchKernelGGL((conv_mfma_kernel<COB, UP>), dim3(tx * ty), dim3(kUThreads), lds, s, x, cin, \
-                     wp, out, skip, maskt, relu ? 1 : 0, H, W, tx, tx * ty, N.guard)
-  const int cob = cout / 16;
-  if (ups) {
-    if (cob == 1) FVX_CONV(1, true);
-    else if (cob == 2) FVX_CONV(2, true);
-    else if (cob == 3) FVX_CONV(3, true);
-    else FVX_CONV(4, true);
-  } else {
-    if (cob == 1) FVX_CONV(1, false);
-    else if (cob == 2) FVX_CONV(2, false);
-    else if (cob == 3) FVX_CONV(3, false);
-    else FVX_CONV(4, false);
+  // Tiles 64 pixels wide (halo 1.5x) where they fill the chip with several
+  // workgroups per CU, else 16 wide (halo 1.7x) for four times the workgroups.
+  const bool wide = cdiv(W, 64) * cdiv(H, kUTh) >= 1024;
+  const int tx = cdiv(W, wide ? 64 : 16), nt = tx * cdiv(H, kUTh);
+#define FVX_CONV_NB(COB, CIB, NB)                                                              \
+  hipLaunchKernelGGL((conv_mfma_kernel<COB, CIB, NB>), dim3(nt), dim3(conv_threads(COB)), 0, s, x, \
+                     wp, out, skip, maskt, relu ? 1 : 0, ups ? 1 : 0, H, W, tx, nt, N.guard)
+#define FVX_CONV(COB, CIB)                   \
+  if (wide) FVX_CONV_NB(COB, CIB, 4);        \
+  else FVX_CONV_NB(COB, CIB, 1)
+#define FVX_CONV_CI(COB)                     \
+  switch (cin / 16) {                        \
+    case 1: FVX_CONV(COB, 1); break;         \
+    case 2: FVX_CONV(COB, 2); break;         \
+    case 3: FVX_CONV(COB, 3); break;         \
+    default: FVX_CONV(COB, 4); break;        \
   }
+  switch (cout / 16) {
+    case 1: FVX_CONV_CI(1); break;
+    case 2: FVX_CONV_CI(2); break;
+    case 3: FVX_CONV_CI(3); break;
+    default: FVX_CONV_CI(4); break;
+  }
+#undef FVX_CONV_CI
 #undef FVX_CONV
+#undef FVX_CONV_NB
 }
 
 static dim3 g2(int H, int W) { return dim3(cdiv(W, 64), cdiv(H, 4)); }

@@ -107,3 +107,20 @@ def test_weight_gradients_at_tile_edges(channels, H, W):
     for k in ref:
         err = np.linalg.norm(got[k] - ref[k]) / np.linalg.norm(ref[k])
         assert err <= tol, (k, err)
+
+
+@pytest.mark.parametrize("cin,cout,ups", [(16, 16, False), (48, 32, True), (64, 48, False),
+                                          (32, 64, False)])
+def test_conv_wide_tiles(cin, cout, ups):
+    """Enough rows for the 64-pixel tiles, whose last column holds 2 pixels
+    and whose last row of tiles 2 rows; the bound of test_single_conv_mfma."""
+    need_gpu()
+    rng = np.random.default_rng(1)
+    Hx, Wx = (685, 65) if ups else (1370, 130)
+    x = Lm.to_bf16(rng.standard_normal((Hx, Wx, cin))).astype(np.float64)
+    w = Lm.to_bf16(rng.standard_normal((3, 3, cout, cin)) * 0.2).astype(np.float64)
+    ref = U.conv3x3(U.up2(x) if ups else x, w)
+    got = Lm.conv3x3_bf16(_bf16(x), w, ups=ups).float().cpu().numpy()
+    refb = Lm.to_bf16(ref)
+    ulp = np.abs(refb).astype(np.float64) * 2.0**-7 + 1e-30
+    assert np.all(np.abs(got - refb) <= ulp + 1e-6 * np.abs(ref).max())
