@@ -29,39 +29,10 @@
 
 #include "fvx_common.hpp"
 #include "mg.hpp"
+#include "mg_level.hpp"
+#include "mg_strip.hpp"
 
 namespace fvx {
-
-enum MgKind : int { kNoflux = 0, kDirichlet = 1 };
-
-template <typename T>
-struct LevelDev {
-  int ny, nx;
-  T idx2, idy2, lam;
-  T inv_d;                 // Dirichlet scalar 1/diag
-  const uint8_t* mask;     // nullptr = all wet
-  const T* cx;             // noflux face coefficients (nullptr for Dirichlet)
-  const T* cy;
-  const T* inv;            // noflux inverse diagonal
-  T* u;                    // iterate (coarse levels: error)
-  T* b;                    // right-hand side (coarse levels: restricted residual)
-  T* t;                    // scratch (ping-pong for single-workgroup sweeps)
-  T* t2;                   // scratch for tiled sweep chains
-  T* t3;
-  // Dirichlet coarse levels with the wall correction: each dry or outside
-  // neighbour adds wall_g / h^2 to the diagonal (a ghost value wall_g u_c
-  // instead of 0); 0 = off.
-  T wall_g;
-  // The mask packed by columns (with mask): word (blk, i) = the mask of rows
-  // 32 blk .. 32 blk + 31 of column i as bits (rows beyond the level 0),
-  // blocks 0 .. ny / 32 + 1, so a 64-bit window from any row block is valid.
-  const uint32_t* mcol;
-};
-
-template <typename T>
-__device__ __forceinline__ T mval(const uint8_t* m, int64_t k) {
-  return m ? (m[k] ? T(1) : T(0)) : T(1);
-}
 
 // ---------------------------------------------------------------------------
 // Reductions: every block reduces its values in registers and LDS and writes
@@ -72,41 +43,6 @@ __device__ __forceinline__ T mval(const uint8_t* m, int64_t k) {
 // needed (on this GPU such a fence writes back the XCD's L2: with one per
 // block a 16k-block reduction cost ~0.4 ms).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int lin_tid() {
-  return threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-}
-
-// Sums of NV values over the block into partials: block ``bid`` of ``nblk``
-// stores value k at partials[k * nblk + bid].
-template <int NV, int kThreads, typename A>
-__device__ __forceinline__ void block_partials(const A (&v)[NV], double* partials, int64_t nblk,
-                                               int64_t bid) {
-  static_assert(NV <= 64, "one summing thread per value");
-  __shared__ double red[kThreads / 64][NV];
-  const int tid = lin_tid();
-  const int lane = tid & 63, wid = tid >> 6;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const A s = wave_sum_last(v[k]);
-    if (lane == 63) red[wid][k] = (double)s;
-  }
-  __syncthreads();
-  if (tid < NV) {
-    // Value-major: value k of block b at partials[k * nblocks + b], so the
-    // finishing kernel's reads are coalesced.  One thread per value sums the
-    // waves in order.
-    double s = 0.0;
-#pragma unroll
-    for (int w = 0; w < kThreads / 64; ++w) s += red[w][tid];
-    partials[tid * nblk + bid] = s;
-  }
-}
-template <int NV, int kThreads, typename A>
-__device__ __forceinline__ void block_partials(const A (&v)[NV], double* partials) {
-  block_partials<NV, kThreads>(v, partials, (int64_t)gridDim.x * gridDim.y,
-                               (int64_t)blockIdx.y * gridDim.x + blockIdx.x);
-}
-
 // Reduction sites (which scalars the finishing kernel updates).
 enum RedSite : int {
   kRedCG = 0,      // the nine PCG dots -> beta, p.Ap, alpha, predicted ||r||^2
@@ -137,8 +73,6 @@ __device__ __forceinline__ void inner_reset(PcgScalars* inner, const PcgScalars*
   inner->first = 1;
   inner->iter = 0;
 }
-// Order of the PCG dots (z = M r, a = A z, q = q_{k-1} = A p_{k-1}).
-enum CgDot : int { kZR, kZQ, kZA, kRR, kRA, kRQ, kAA, kAQ, kQQ, kNumCgDots };
 constexpr int kFinishThreads = 1024;
 
 template <int NV, int SITE>
@@ -338,56 +272,6 @@ __device__ __forceinline__ T glob_inv(const LevelDev<T>& L, int64_t k) {
   if constexpr (KIND == kDirichlet) return L.inv_d * mval<T>(L.mask, k);
   return L.inv[k];
 }
-
-// ---------------------------------------------------------------------------
-// Tiled smoother kernel.  MODE:
-//   0 SMOOTH   : NS sweeps                                  -> u_out
-//   1 DOWN     : NS sweeps, residual, restriction           -> u_out, C.b
-//   2 UP       : u += P(C.u), NS sweeps                     -> u_out
-//   3 UP_CG    : as UP with one more halo ring, then a = A z on the tile
-//                interior -> u_out (z), az_out (a), and the nine PCG dots of
-//                z, a, r (= b) and q_{k-1} (= w)
-//   4 DOWN_STEP: (wavefront tiles only) the previous PCG step on the tile,
-//                then DOWN from zero on the new residual -> upd.q_out,
-//                upd.r_out, upd.p, upd.x, u_out, C.b
-// ---------------------------------------------------------------------------
-enum TileMode : int { kSmooth = 0, kDown = 1, kUp = 2, kUpCG = 3, kDownUpd = 4 };
-
-// The PCG step that the level-0 down kernel of the next V-cycle applies
-// first (kDownUpd; wavefront tiles only): with a = A z,
-// q_out = a + beta q_in, r_out = r_in - alpha q_out, p = z + beta p,
-// x += alpha p.  r_in and q_in are read on the tile's halo as well, so they
-// cannot be the arrays written.
-template <typename T>
-struct PcgUpdArgs {
-  const T* z;
-  T* p;
-  T* x;
-  int64_t ld_x;
-  const T* q_in;
-  T* q_out;
-  const T* r_in;  // passed to the kernel as its b
-  T* r_out;
-};
-
-constexpr int kTx = 64, kTy = 16, kTileThreads = 256;
-
-template <typename T>
-struct TileArgs {
-  LevelDev<T> L, C;
-  const T* u_in;
-  const T* b;
-  T* u_out;
-  const T* w;
-  T* az_out;
-  T omega;
-  T omw[3];  // wave-tile kernels: the weight of sweep k (= omega unless the
-             // plan smooths with Chebyshev weights)
-  double* partials;
-  PcgScalars* sc;
-  int tiles_x, ntiles;
-  PcgUpdArgs<T> upd;  // kDownUpd; b is r_in
-};
 
 template <typename T, int KIND>
 __device__ __forceinline__ T prolong_at(const LevelDev<T>& C, int j, int i) {
@@ -2344,6 +2228,20 @@ static bool wave_tiled(const LevelDev<T>& L, const LevelDev<T>* C) {
   return false;
 }
 
+// Levels the strip kernels run (mg_strip.hpp): all but FP32 Dirichlet.
+template <typename T, int KIND>
+constexpr bool strip_levels() {
+  return !(std::is_same<T, float>::value && KIND == kDirichlet);
+}
+
+// The sweep weights of a launch by leg (down, up, bottom; ``uniform``: omega).
+template <typename T, int MODE>
+static void tile_weights(const Plan& P, TileArgs<T>& a, bool uniform) {
+  constexpr int role = (MODE == kDown || MODE == kDownUpd) ? 0 : (MODE == kSmooth ? 2 : 1);
+  a.omega = (T)P.omega;
+  for (int k = 0; k < 3; ++k) a.omw[k] = uniform ? a.omega : (T)P.omw[role][k];
+}
+
 template <typename T, int KIND, int NS, int MODE, bool ZERO>
 static void launch_tile(const Plan& P, const LevelDev<T>& L, const LevelDev<T>* C, const T* u_in,
                         const T* b, T* u_out, const T* w, PcgScalars* sc, hipStream_t s,
@@ -2358,12 +2256,7 @@ static void launch_tile(const Plan& P, const LevelDev<T>& L, const LevelDev<T>* 
   a.u_out = u_out;
   a.w = w;
   a.az_out = az_out;
-  a.omega = (T)P.omega;
-  {
-    // (sweep weights by leg: down, up, bottom; ``uniform``: omega throughout)
-    constexpr int role = (MODE == kDown || MODE == kDownUpd) ? 0 : (MODE == kSmooth ? 2 : 1);
-    for (int k = 0; k < 3; ++k) a.omw[k] = uniform ? a.omega : (T)P.omw[role][k];
-  }
+  tile_weights<T, MODE>(P, a, uniform);
   a.partials = P.partials;
   a.sc = sc;
   if constexpr (std::is_same<T, float>::value && KIND == kDirichlet) {
@@ -2414,7 +2307,9 @@ static void launch_tile(const Plan& P, const LevelDev<T>& L, const LevelDev<T>* 
       return;
     }
   }
-  if constexpr (MODE != kDownUpd) {
+  // (strip levels come here without sweeps only)
+  constexpr bool kLds = NS == 0 || !strip_levels<T, KIND>();
+  if constexpr (MODE != kDownUpd && kLds) {
     a.tiles_x = cdiv(L.nx, kTx);
     a.ntiles = a.tiles_x * cdiv(L.ny, kTy);
     if (L.mask)
@@ -2430,10 +2325,66 @@ static void launch_tile(const Plan& P, const LevelDev<T>& L, const LevelDev<T>* 
   }
 }
 
-// Damped-Jacobi sweeps fused into one level kernel (with the residual and
+// Damped-Jacobi sweeps fused into one wave-tile launch (with the residual and
 // restriction on the down leg, the prolongation on the up leg); more sweeps
 // per side run as separate smoothing kernels first (down) or after (up).
 constexpr int kMaxFuse = 3;
+
+// Sweeps of a leg of ``n`` that one launch takes: the strips also fuse six
+// (the reference's default), which saves a pass over the level's arrays.
+template <typename T, int KIND>
+static int fused_sweeps(int n) {
+  return strip_levels<T, KIND>() && n >= kStripMaxFuse ? kStripMaxFuse : std::min(n, kMaxFuse);
+}
+
+// One level kernel of ``ns`` sweeps (at most fused_sweeps).
+template <typename T, int KIND, int MODE>
+static void launch_level(const Plan& P, int ns, bool zero, const LevelDev<T>& L,
+                         const LevelDev<T>* C, const T* u_in, const T* b, T* u_out, const T* w,
+                         PcgScalars* sc, hipStream_t s, T* az_out = nullptr, bool finish = true,
+                         const PcgUpdArgs<T>* upd = nullptr, bool uniform = false) {
+  if constexpr (strip_levels<T, KIND>() && MODE != kDownUpd) {
+    if (ns > 0) {
+      TileArgs<T> a;
+      std::memset(&a, 0, sizeof(a));
+      a.L = L;
+      if (C) a.C = *C;
+      a.u_in = u_in;
+      a.b = b;
+      a.u_out = u_out;
+      a.w = w;
+      a.az_out = az_out;
+      tile_weights<T, MODE>(P, a, uniform);
+      a.partials = P.partials;
+      a.sc = sc;
+      const int nblk = launch_strip<T, KIND>(ns, MODE, zero, a, s);
+      if constexpr (MODE == kUpCG)
+        if (finish)
+          hipLaunchKernelGGL((reduce_finish_kernel<kNumCgDots, kRedCG>), dim3(1),
+                             dim3(kFinishThreads), 0, s, P.partials, nblk, sc, 0.0, 0.0);
+      return;
+    }
+  }
+  auto go = [&](auto n, auto z) {
+    launch_tile<T, KIND, decltype(n)::value, MODE, decltype(z)::value>(
+        P, L, C, u_in, b, u_out, w, sc, s, az_out, finish, upd, uniform);
+  };
+  auto sweeps = [&](auto z) {
+    using Z = decltype(z);
+    if constexpr (strip_levels<T, KIND>()) {
+      go(std::integral_constant<int, 0>(), Z());
+    } else {
+      if (ns == 3) go(std::integral_constant<int, 3>(), Z());
+      else if (ns == 2) go(std::integral_constant<int, 2>(), Z());
+      else if (ns == 1) go(std::integral_constant<int, 1>(), Z());
+      else go(std::integral_constant<int, 0>(), Z());
+    }
+  };
+  if constexpr (MODE == kUp || MODE == kUpCG) sweeps(std::false_type());
+  else if constexpr (MODE == kDownUpd) sweeps(std::true_type());
+  else if (zero) sweeps(std::true_type());
+  else sweeps(std::false_type());
+}
 
 // Level-0 up kernel of a preconditioning V-cycle with the PCG dots, with the
 // plan's fused post-sweeps, as the V-cycle launches it, without its
@@ -2442,11 +2393,8 @@ template <typename T, int KIND>
 static void launch_vcycle_up_cg(const Plan& P, const LevelDev<T>& L, const LevelDev<T>& C,
                                 const T* u, const T* b, T* out, const T* w, T* az,
                                 PcgScalars* sc, hipStream_t s) {
-  const int fz = P.n_post < kMaxFuse ? P.n_post : kMaxFuse;
-  if (fz == 3) launch_tile<T, KIND, 3, kUpCG, false>(P, L, &C, u, b, out, w, sc, s, az, false);
-  else if (fz == 2) launch_tile<T, KIND, 2, kUpCG, false>(P, L, &C, u, b, out, w, sc, s, az, false);
-  else if (fz == 1) launch_tile<T, KIND, 1, kUpCG, false>(P, L, &C, u, b, out, w, sc, s, az, false);
-  else launch_tile<T, KIND, 0, kUpCG, false>(P, L, &C, u, b, out, w, sc, s, az, false);
+  launch_level<T, KIND, kUpCG>(P, fused_sweeps<T, KIND>(P.n_post), false, L, &C, u, b, out, w, sc,
+                               s, az, false);
 }
 
 // Finishing kernel of a reduction over the blocks of grid2(ny, nx).
@@ -2458,43 +2406,23 @@ static void finish2(const Plan& P, int ny, int nx, PcgScalars* sc, hipStream_t s
                      P.partials, nblk, sc, rtol2, atol2);
 }
 
-// nu Jacobi sweeps on level L, up to 3 per kernel.  Ping-pongs between the
-// scratch arrays s1 / s2 (which must differ from u_in and final_out); the last
-// chunk writes final_out when given.  Returns the array holding the result.
-// The sweeps take the plan's bottom-level weights unless ``uniform`` (omega).
+// nu Jacobi sweeps on level L, fused_sweeps per kernel.  Ping-pongs between
+// the scratch arrays s1 / s2 (which must differ from u_in and final_out); the
+// last chunk writes final_out when given.  Returns the array holding the
+// result.  The sweeps take the plan's bottom-level weights unless ``uniform``
+// (omega).
 template <typename T, int KIND>
 static T* smooth_chunks(const Plan& P, const LevelDev<T>& L, const T* u_in, bool zero,
                         const T* b, int nu, T* s1, T* s2, T* final_out, PcgScalars* sc,
                         hipStream_t s, bool uniform = false) {
   const T* src = u_in;
   T* dst = nullptr;
-  const int K = (nu + 2) / 3;
-  for (int c = 0; c < K; ++c) {
-    const int ns = std::min(3, nu - 3 * c);
-    dst = (c == K - 1 && final_out) ? final_out : ((c & 1) ? s2 : s1);
-    const bool z = zero && c == 0;
-    if (ns == 3) {
-      if (z)
-        launch_tile<T, KIND, 3, kSmooth, true>(P, L, nullptr, src, b, dst, nullptr, sc, s, nullptr,
-                                                 true, nullptr, uniform);
-      else
-        launch_tile<T, KIND, 3, kSmooth, false>(P, L, nullptr, src, b, dst, nullptr, sc, s,
-                                                  nullptr, true, nullptr, uniform);
-    } else if (ns == 2) {
-      if (z)
-        launch_tile<T, KIND, 2, kSmooth, true>(P, L, nullptr, src, b, dst, nullptr, sc, s, nullptr,
-                                                 true, nullptr, uniform);
-      else
-        launch_tile<T, KIND, 2, kSmooth, false>(P, L, nullptr, src, b, dst, nullptr, sc, s,
-                                                  nullptr, true, nullptr, uniform);
-    } else {
-      if (z)
-        launch_tile<T, KIND, 1, kSmooth, true>(P, L, nullptr, src, b, dst, nullptr, sc, s, nullptr,
-                                                 true, nullptr, uniform);
-      else
-        launch_tile<T, KIND, 1, kSmooth, false>(P, L, nullptr, src, b, dst, nullptr, sc, s,
-                                                  nullptr, true, nullptr, uniform);
-    }
+  for (int c = 0; nu > 0; ++c) {
+    const int ns = fused_sweeps<T, KIND>(nu);
+    nu -= ns;
+    dst = (nu == 0 && final_out) ? final_out : ((c & 1) ? s2 : s1);
+    launch_level<T, KIND, kSmooth>(P, ns, zero && c == 0, L, nullptr, src, b, dst, nullptr, sc, s,
+                                   nullptr, true, nullptr, uniform);
     src = dst;
   }
   return dst;
@@ -2561,37 +2489,19 @@ static int v_cycle_impl(Plan& P, const T* u0, const T* rhs, T* out, T* az, const
     bool zero = (l > l0) || (u0 == nullptr);
     const T* src = (l == l0) ? u0 : nullptr;
     const int npre = P.n_pre;
-    const int fz = npre < kMaxFuse ? npre : kMaxFuse;  // fused with residual + restriction
+    const int fz = fused_sweeps<T, KIND>(npre);  // fused with residual + restriction
     if (l == 0 && upd) {
       // The previous PCG step, then this down leg from r_{k+1} = rhs
       // (pcg_iters checks that the plan allows it).
-      if (fz == 3) launch_tile<T, KIND, 3, kDownUpd, true>(P, L, &C, nullptr, upd->r_in, L.u,
-                                                           nullptr, sc, s, nullptr, true, upd);
-      else if (fz == 2) launch_tile<T, KIND, 2, kDownUpd, true>(P, L, &C, nullptr, upd->r_in, L.u,
-                                                                nullptr, sc, s, nullptr, true, upd);
-      else if (fz == 1) launch_tile<T, KIND, 1, kDownUpd, true>(P, L, &C, nullptr, upd->r_in, L.u,
-                                                                nullptr, sc, s, nullptr, true, upd);
-      else launch_tile<T, KIND, 0, kDownUpd, true>(P, L, &C, nullptr, upd->r_in, L.u, nullptr, sc,
-                                                   s, nullptr, true, upd);
+      launch_level<T, KIND, kDownUpd>(P, fz, true, L, &C, nullptr, upd->r_in, L.u, nullptr, sc, s,
+                                      nullptr, true, upd);
       continue;
     }
     if (npre - fz > 0) {
       src = smooth_chunks<T, KIND>(P, L, src, zero, b, npre - fz, L.t, L.t2, nullptr, sc, s);
       zero = false;
     }
-    if (fz == 3) {
-      if (zero) launch_tile<T, KIND, 3, kDown, true>(P, L, &C, src, b, L.u, nullptr, sc, s);
-      else launch_tile<T, KIND, 3, kDown, false>(P, L, &C, src, b, L.u, nullptr, sc, s);
-    } else if (fz == 2) {
-      if (zero) launch_tile<T, KIND, 2, kDown, true>(P, L, &C, src, b, L.u, nullptr, sc, s);
-      else launch_tile<T, KIND, 2, kDown, false>(P, L, &C, src, b, L.u, nullptr, sc, s);
-    } else if (fz == 1) {
-      if (zero) launch_tile<T, KIND, 1, kDown, true>(P, L, &C, src, b, L.u, nullptr, sc, s);
-      else launch_tile<T, KIND, 1, kDown, false>(P, L, &C, src, b, L.u, nullptr, sc, s);
-    } else {
-      if (zero) launch_tile<T, KIND, 0, kDown, true>(P, L, &C, src, b, L.u, nullptr, sc, s);
-      else launch_tile<T, KIND, 0, kDown, false>(P, L, &C, src, b, L.u, nullptr, sc, s);
-    }
+    launch_level<T, KIND, kDown>(P, fz, zero, L, &C, src, b, L.u, nullptr, sc, s);
   }
   // Coarse levels lc .. nl-1 in one workgroup (zero guess at level lc); a
   // bottom level too large for it gets n_coarse damped-Jacobi sweeps from
@@ -2623,21 +2533,15 @@ static int v_cycle_impl(Plan& P, const T* u0, const T* rhs, T* out, T* az, const
     C.u = cur;
     const T* b = (l == l0) ? rhs : L.b;
     const int npost = P.n_post;
-    const int fz = npost < kMaxFuse ? npost : kMaxFuse;
+    const int fz = fused_sweeps<T, KIND>(npost);
     const int tail = npost - fz;
     const bool dk = az && l == 0 && tail == 0;
     T* dst = (l == l0 && tail == 0) ? out : L.t;
     if (dk) {
-      if (fz == 3) launch_tile<T, KIND, 3, kUpCG, false>(P, L, &C, L.u, b, dst, w, sc, s, az);
-      else if (fz == 2) launch_tile<T, KIND, 2, kUpCG, false>(P, L, &C, L.u, b, dst, w, sc, s, az);
-      else if (fz == 1) launch_tile<T, KIND, 1, kUpCG, false>(P, L, &C, L.u, b, dst, w, sc, s, az);
-      else launch_tile<T, KIND, 0, kUpCG, false>(P, L, &C, L.u, b, dst, w, sc, s, az);
+      launch_level<T, KIND, kUpCG>(P, fz, false, L, &C, L.u, b, dst, w, sc, s, az);
       if (fused) *fused = true;
     } else {
-      if (fz == 3) launch_tile<T, KIND, 3, kUp, false>(P, L, &C, L.u, b, dst, nullptr, sc, s);
-      else if (fz == 2) launch_tile<T, KIND, 2, kUp, false>(P, L, &C, L.u, b, dst, nullptr, sc, s);
-      else if (fz == 1) launch_tile<T, KIND, 1, kUp, false>(P, L, &C, L.u, b, dst, nullptr, sc, s);
-      else launch_tile<T, KIND, 0, kUp, false>(P, L, &C, L.u, b, dst, nullptr, sc, s);
+      launch_level<T, KIND, kUp>(P, fz, false, L, &C, L.u, b, dst, nullptr, sc, s);
     }
     if (tail > 0) {
       dst = smooth_chunks<T, KIND>(P, L, dst, false, b, tail, L.t2, L.t3, l == l0 ? out : nullptr,
@@ -3453,7 +3357,8 @@ int fvx_mg_plan_create(const double* mask, const double* coeff, int ny, int nx, 
     // energy dots), kNumCgDots per level-0 tile or stencil block (PCG dots).
     const size_t n2 = (size_t)2 * cdiv(nx, 64) * cdiv(ny, 4);
     const size_t ncg = (size_t)kNumCgDots * std::max<size_t>(
-        (size_t)cdiv(nx, kTx) * cdiv(ny, kTy), (size_t)cdiv(nx, 256) * cdiv(ny, kStencilRows));
+        std::max<size_t>((size_t)cdiv(nx, kTx) * cdiv(ny, kTy), (size_t)strip_max_blocks(ny, nx)),
+        (size_t)cdiv(nx, 256) * cdiv(ny, kStencilRows));
     const size_t npart = std::max(n2, ncg) + 64;
     P->npart = npart;
     hipError_t e = hipMalloc(&P->partials, npart * sizeof(double));

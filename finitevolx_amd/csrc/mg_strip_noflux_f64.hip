@@ -1,0 +1,3 @@
+#include "mg_strip_impl.hpp"
+
+template int fvx::launch_strip<double, fvx::kNoflux>(int, int, bool, TileArgs<double>, hipStream_t);

@@ -431,3 +431,47 @@ def test_v_cycle_from_coarser_levels(ny, nx, kind, masked, varcoef):
         assert_close_scaled(to_np(got), ref0, 1e-4, f"level {li} f32")
     with pytest.raises(ValueError):
         mg.v_cycle(None, np.zeros((ny, nx)), level_idx=len(levels))
+
+
+@pytest.mark.parametrize("ny,nx,kind,masked", [
+    (72, 100, "noflux", True), (104, 116, "noflux", False), (140, 300, "dirichlet", True),
+    (228, 172, "dirichlet", False), (256, 1000, "noflux", True)])
+@pytest.mark.parametrize("npre,npost", [(1, 2), (2, 1), (3, 6), (6, 3), (4, 7)])
+def test_strip_kernels_at_strip_edges(ny, nx, kind, masked, npre, npost):
+    """Levels that end inside a strip's columns (50, 56, 58, 60 or 62 written)
+    and rows (4 to 32), with every number of fused sweeps, from zero and from
+    a guess; FP64 rounding over the ~20 sweeps of a cycle stays under 1e-12 of
+    the maximum, FP32 under 1e-5 (2e-16 and 6e-8 a sweep, with room for the
+    operator's cancellation)."""
+    need_gpu()
+    m, coeff, dx, dy, lam = _setup(ny, nx, kind, masked, kind == "noflux", seed=ny)
+    rng = np.random.default_rng(nx)
+    b, u0 = rng.standard_normal((ny, nx)) * m, rng.standard_normal((ny, nx))
+    kw = dict(n_pre=npre, n_post=npost, n_coarse=8, omega=0.9)
+    levels = fvx.build_multigrid(m, dx, dy, lam, coeff, kind=kind, n_levels=2)
+    for prec, tol in (("float64", 1e-12), ("float32", 1e-5)):
+        mg = S.build_multigrid_solver(m, dx, dy, lam, coeff, kind=kind, precision=prec, n_levels=2,
+                                      **kw)
+        dt = torch.float64 if prec == "float64" else torch.float32
+        bt, ut = (torch.tensor(x, dtype=dt) for x in (b, u0))
+        ref = fvx.v_cycle(levels, np.zeros_like(b), b, **kw)
+        assert_close_scaled(to_np(mg.v_cycle(None, bt)), ref, tol, f"V(0, b) {prec}")
+        ref = fvx.v_cycle(levels, u0, b, **kw)
+        assert_close_scaled(to_np(mg.v_cycle(ut, bt)), ref, tol, f"V(u0, b) {prec}")
+        for n in (1, 6, 8):
+            got = S.weighted_jacobi(ut, bt, mg.levels[0], 0.9, n)
+            assert_close_scaled(to_np(got), fvx.weighted_jacobi(u0, b, levels[0], 0.9, n), tol,
+                                f"jacobi{n} {prec}")
+
+
+def test_strip_kernels_long_strips():
+    """A level large enough for 32-row strips, both axes ending inside one."""
+    need_gpu()
+    ny, nx = 2092, 1980
+    m, coeff, dx, dy, lam = _setup(ny, nx, "noflux", True, True, seed=7)
+    b = np.random.default_rng(8).standard_normal((ny, nx)) * m
+    kw = dict(n_pre=2, n_post=1, n_coarse=2, omega=0.9)
+    levels = fvx.build_multigrid(m, dx, dy, lam, coeff, kind="noflux", n_levels=2)
+    mg = S.build_multigrid_solver(m, dx, dy, lam, coeff, n_levels=2, **kw)
+    ref = fvx.v_cycle(levels, np.zeros_like(b), b, **kw)
+    assert_close_scaled(to_np(mg.v_cycle(None, b)), ref, 1e-12, "V(0, b)")
