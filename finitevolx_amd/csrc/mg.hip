@@ -12,13 +12,15 @@
 //  * preconditioner:  make_multigrid_preconditioner (preconditioners.py:207-244)
 //
 // GPU design (gfx950): per fine level one fused DOWN kernel (nu1 Jacobi sweeps
-// temporally blocked in an LDS tile + residual + 2x2 restriction) and one fused
-// UP kernel (prolongation + correction + nu2 sweeps); the coarse levels
-// (<= kCoarseCells cells) run inside a single workgroup; PCG vector updates
-// and dot products are fused kernels whose last workgroup finishes each
-// reduction on the device (no host round trip); every kernel of an iteration
-// exits immediately once the device-side convergence flag is set, so the host
-// can enqueue a predicted number of iterations and synchronise once.
+// + residual + 2x2 restriction) and one fused UP kernel (prolongation +
+// correction + nu2 sweeps): FP32 Dirichlet levels as wavefront tiles in
+// registers (below), all others as strips a wavefront marches over
+// (mg_strip.hpp); the coarse levels (<= kCoarseCells cells) run inside a
+// single workgroup (mg_coarse.hpp); PCG vector updates and dot products are
+// fused kernels whose reductions a finishing kernel ends on the device (no
+// host round trip); every kernel of an iteration exits immediately once the
+// device-side convergence flag is set, so the host can enqueue a predicted
+// number of iterations and synchronise once.
 
 #include <algorithm>
 #include <cmath>
@@ -29,6 +31,7 @@
 
 #include "fvx_common.hpp"
 #include "mg.hpp"
+#include "mg_coarse.hpp"
 #include "mg_level.hpp"
 #include "mg_strip.hpp"
 
@@ -1053,378 +1056,6 @@ __global__ __launch_bounds__(256) void mg_wave_tile_kernel(TileArgs<float> a) {
 }
 
 // ---------------------------------------------------------------------------
-// Single-workgroup coarse V-cycle (levels lc .. nL-1) on global arrays that
-// stay resident in L2.  Starts from a zero guess at level lc (preconditioner
-// use) and writes the result to levels[lc].u.
-// ---------------------------------------------------------------------------
-constexpr int kCoarseThreads = 1024;
-// Per-sweep weights the coarse kernel carries for each leg (sweeps past the
-// last take the last weight).
-constexpr int kMaxW = 8;
-
-template <typename T>
-struct CoarseArgs {
-  LevelDev<T> lv[16];
-  int lc, nl, n_pre, n_post, n_coarse;
-  int nonzero_init;  // level lc starts from lv[lc].u instead of zero
-  T omega;
-  T w[3][kMaxW];  // sweep weights: pre-smoothing, post-smoothing, bottom
-  const int* done;
-};
-
-template <typename T, int KIND>
-__device__ void cw_sweeps(const LevelDev<T>& L, int n, bool zero, const T* w) {
-  const int N = L.ny * L.nx;
-  T* src = L.u;
-  T* dst = L.t;
-  for (int s = 0; s < n; ++s) {
-    const T om = w[s < kMaxW ? s : kMaxW - 1];
-    for (int k = threadIdx.x; k < N; k += kCoarseThreads) {
-      const int j = k / L.nx, i = k % L.nx;
-      const T m = mval<T>(L.mask, k);
-      const T inv = glob_inv<T, KIND>(L, k);
-      T un;
-      if (zero && s == 0) un = (om * inv * L.b[k]) * m;
-      else un = (src[k] + om * inv * (L.b[k] - glob_Au<T, KIND>(L, src, j, i))) * m;
-      dst[k] = un;
-    }
-    __syncthreads();
-    T* tmp = src;
-    src = dst;
-    dst = tmp;
-  }
-  if (src != L.u) {  // odd number of sweeps: copy back
-    for (int k = threadIdx.x; k < N; k += kCoarseThreads) L.u[k] = src[k];
-    __syncthreads();
-  }
-}
-
-// Level l of the coarse kernel with its iterate, scratch and right-hand side
-// in LDS (u, t, b at cell offset off), coefficients and masks in global memory.
-template <typename T, bool LDS>
-__device__ __forceinline__ LevelDev<T> lds_level(const CoarseArgs<T>& a, int l, T* sm, int off) {
-  LevelDev<T> L = a.lv[l];
-  if constexpr (!LDS) return L;
-  const int n = L.ny * L.nx;
-  L.u = sm + off;
-  L.t = sm + off + n;
-  L.b = sm + off + 2 * n;
-  return L;
-}
-
-// LDS = false keeps every level in global memory (bottom levels too large
-// for LDS: grids that stop halving early).
-template <typename T, int KIND, bool LDS>
-__global__ __launch_bounds__(kCoarseThreads) void mg_coarse_kernel(CoarseArgs<T> a) {
-  const bool skip = a.done && *a.done;
-  if (!LDS && skip) return;
-  extern __shared__ __align__(16) unsigned char coarse_smem[];
-  T* sm = reinterpret_cast<T*>(coarse_smem);
-  int off[16];
-  {
-    int o = 0;
-    for (int l = a.lc; l < a.nl; ++l) {
-      off[l] = o;
-      o += 3 * a.lv[l].ny * a.lv[l].nx;
-    }
-  }
-  // Level lc's right-hand side (and guess) from global memory.
-  if constexpr (LDS) {
-    const LevelDev<T>& G = a.lv[a.lc];
-    const LevelDev<T> L = lds_level<T, LDS>(a, a.lc, sm, off[a.lc]);
-    for (int k = threadIdx.x; k < G.ny * G.nx; k += kCoarseThreads) {
-      L.b[k] = G.b[k];
-      if (a.nonzero_init) L.u[k] = G.u[k];
-    }
-    if (skip) return;
-    __syncthreads();
-  }
-  // Down leg.
-  for (int l = a.lc; l < a.nl - 1; ++l) {
-    const LevelDev<T> L = lds_level<T, LDS>(a, l, sm, off[l]);
-    const LevelDev<T> C = lds_level<T, LDS>(a, l + 1, sm, off[l + 1]);
-    const bool zero = !(a.nonzero_init && l == a.lc);
-    if (a.n_pre > 0) {
-      cw_sweeps<T, KIND>(L, a.n_pre, zero, a.w[0]);
-    } else if (zero) {
-      for (int k = threadIdx.x; k < L.ny * L.nx; k += kCoarseThreads) L.u[k] = T(0);
-      __syncthreads();
-    }
-    for (int k = threadIdx.x; k < C.ny * C.nx; k += kCoarseThreads) {
-      const int J = k / C.nx, I = k % C.nx;
-      T s4 = T(0), cnt = T(0);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int dj = (q == 1 || q == 3), di = (q >= 2);
-        const int j = 2 * J + dj, i = 2 * I + di;
-        const int64_t f = (int64_t)j * L.nx + i;
-        const T m = mval<T>(L.mask, f);
-        const T r = (L.b[f] - glob_Au<T, KIND>(L, L.u, j, i)) * m;
-        s4 += r * m;
-        cnt += m;
-      }
-      const T rs = KIND == kDirichlet ? s4 * T(0.25) : s4 / (cnt > T(1) ? cnt : T(1));
-      C.b[k] = rs * mval<T>(C.mask, k);
-    }
-    __syncthreads();
-  }
-  // Bottom solve: n_coarse sweeps from zero (from the guess when the whole
-  // hierarchy is one level and a guess was given).
-  {
-    const LevelDev<T> B = lds_level<T, LDS>(a, a.nl - 1, sm, off[a.nl - 1]);
-    const bool zero = !(a.nonzero_init && a.lc == a.nl - 1);
-    if (a.n_coarse > 0) {
-      cw_sweeps<T, KIND>(B, a.n_coarse, zero, a.w[2]);
-    } else if (zero) {
-      for (int k = threadIdx.x; k < B.ny * B.nx; k += kCoarseThreads) B.u[k] = T(0);
-      __syncthreads();
-    }
-  }
-  // Up leg.
-  for (int l = a.nl - 2; l >= a.lc; --l) {
-    const LevelDev<T> L = lds_level<T, LDS>(a, l, sm, off[l]);
-    const LevelDev<T> C = lds_level<T, LDS>(a, l + 1, sm, off[l + 1]);
-    for (int k = threadIdx.x; k < L.ny * L.nx; k += kCoarseThreads) {
-      const int j = k / L.nx, i = k % L.nx;
-      const T m = mval<T>(L.mask, k);
-      L.u[k] = (L.u[k] + prolong_at<T, KIND>(C, j, i) * m) * m;
-    }
-    __syncthreads();
-    cw_sweeps<T, KIND>(L, a.n_post, false, a.w[1]);
-  }
-  // Level lc's corrected iterate back to global memory.
-  if constexpr (LDS) {
-    const LevelDev<T>& G = a.lv[a.lc];
-    const LevelDev<T> L = lds_level<T, LDS>(a, a.lc, sm, off[a.lc]);
-    for (int k = threadIdx.x; k < G.ny * G.nx; k += kCoarseThreads) G.u[k] = L.u[k];
-  }
-}
-
-// LDS-resident coarse V-cycle.  Levels lc .. nl-1 keep their iterate u,
-// scratch t and right-hand side b in dynamic LDS, addressed by cell offsets
-// (ds_read/ds_write); the 1024 threads tile each level as 32 x 32 blocks of
-// cells, so no integer division is needed.  Every stored iterate is already
-// multiplied by its mask, which is the reference's u * mask before the
-// stencil (multigrid.py:383).
-template <typename T, int KIND>
-struct CoarseLds {
-  T* sm;
-  __device__ __forceinline__ T m_at(const LevelDev<T>& L, int k) const {
-    return mval<T>(L.mask, k);
-  }
-  __device__ __forceinline__ T inv_at(const LevelDev<T>& L, int k, T m) const {
-    if constexpr (KIND == kDirichlet) return L.inv_d * m;
-    return L.inv[k];
-  }
-  // (A u)(j, i) for u at LDS offset ou (zero outside the level).
-  __device__ __forceinline__ T Au(const LevelDev<T>& L, int ou, int j, int i, int k, T m) const {
-    const T c = sm[ou + k];
-    const T e = (i + 1 < L.nx) ? sm[ou + k + 1] : T(0);
-    const T w = (i > 0) ? sm[ou + k - 1] : T(0);
-    const T n = (j + 1 < L.ny) ? sm[ou + k + L.nx] : T(0);
-    const T s = (j > 0) ? sm[ou + k - L.nx] : T(0);
-    T lap;
-    if constexpr (KIND == kDirichlet) {
-      lap = (e + w - T(2) * c) * L.idx2 + (n + s - T(2) * c) * L.idy2;
-    } else {
-      const T cxe = L.cx[k], cxw = (i > 0) ? L.cx[k - 1] : T(0);
-      const T cyn = L.cy[k], cys = (j > 0) ? L.cy[k - L.nx] : T(0);
-      lap = (cxe * (e - c) - cxw * (c - w)) * L.idx2 + (cyn * (n - c) - cys * (c - s)) * L.idy2;
-    }
-    return (lap - L.lam * c) * m;
-  }
-  // n damped-Jacobi sweeps of level L (u at ou, scratch at ot, b at ob); the
-  // result ends in ou.
-  __device__ void sweeps(const LevelDev<T>& L, int ou, int ot, int ob, int n, bool zero,
-                         const T* w, int tx, int ty) const {
-    int src = ou, dst = ot;
-    for (int sw = 0; sw < n; ++sw) {
-      const T om = w[sw < kMaxW ? sw : kMaxW - 1];
-      for (int j = ty; j < L.ny; j += 32)
-        for (int i = tx; i < L.nx; i += 32) {
-          const int k = j * L.nx + i;
-          const T m = m_at(L, k);
-          const T inv = inv_at(L, k, m);
-          T un;
-          if (zero && sw == 0) un = (om * inv * sm[ob + k]) * m;
-          else un = (sm[src + k] + om * inv * (sm[ob + k] - Au(L, src, j, i, k, m))) * m;
-          sm[dst + k] = un;
-        }
-      __syncthreads();
-      const int tmp = src;
-      src = dst;
-      dst = tmp;
-    }
-    if (src != ou) {  // odd number of sweeps: copy back
-      for (int j = ty; j < L.ny; j += 32)
-        for (int i = tx; i < L.nx; i += 32) sm[ou + j * L.nx + i] = sm[src + j * L.nx + i];
-      __syncthreads();
-    }
-  }
-};
-
-template <typename T, int KIND>
-__device__ __forceinline__ void mg_coarse_lds_body(const CoarseArgs<T>& a,
-                                                   unsigned char* coarse_smem) {
-  const bool skip = a.done && *a.done;
-  CoarseLds<T, KIND> S{reinterpret_cast<T*>(coarse_smem)};
-  T* sm = S.sm;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  // LDS offsets of each level's u, t, b (a table in LDS: indexed by the
-  // runtime level, a private array would live in scratch memory).
-  __shared__ int ou[16], ot[16], ob[16];
-  if (threadIdx.x == 0) {
-    int o = 0;
-    for (int l = a.lc; l < a.nl; ++l) {
-      const int n = a.lv[l].ny * a.lv[l].nx;
-      ou[l] = o;
-      ot[l] = o + n;
-      ob[l] = o + 2 * n;
-      o += 3 * n;
-    }
-  }
-  __syncthreads();
-  // Level lc's right-hand side (and masked guess) from global memory.
-  {
-    const LevelDev<T>& G = a.lv[a.lc];
-    for (int j = ty; j < G.ny; j += 32)
-      for (int i = tx; i < G.nx; i += 32) {
-        const int k = j * G.nx + i;
-        sm[ob[a.lc] + k] = G.b[k];
-        if (a.nonzero_init) sm[ou[a.lc] + k] = G.u[k] * S.m_at(G, k);
-      }
-    if (skip) return;
-    __syncthreads();
-  }
-  // Down leg: pre-smoothing, residual, mask-weighted 2x2 restriction.
-  for (int l = a.lc; l < a.nl - 1; ++l) {
-    const LevelDev<T>& L = a.lv[l];
-    const LevelDev<T>& C = a.lv[l + 1];
-    const bool zero = !(a.nonzero_init && l == a.lc);
-    if (a.n_pre > 0) {
-      S.sweeps(L, ou[l], ot[l], ob[l], a.n_pre, zero, a.w[0], tx, ty);
-    } else if (zero) {
-      for (int j = ty; j < L.ny; j += 32)
-        for (int i = tx; i < L.nx; i += 32) sm[ou[l] + j * L.nx + i] = T(0);
-      __syncthreads();
-    }
-    // residual r = (b - A u) m into the scratch array
-    for (int j = ty; j < L.ny; j += 32)
-      for (int i = tx; i < L.nx; i += 32) {
-        const int k = j * L.nx + i;
-        const T m = S.m_at(L, k);
-        sm[ot[l] + k] = (sm[ob[l] + k] - S.Au(L, ou[l], j, i, k, m)) * m;
-      }
-    __syncthreads();
-    for (int J = ty; J < C.ny; J += 32)
-      for (int I = tx; I < C.nx; I += 32) {
-        const int f = (2 * J) * L.nx + 2 * I;
-        const T m00 = S.m_at(L, f), m01 = S.m_at(L, f + 1), m10 = S.m_at(L, f + L.nx),
-                m11 = S.m_at(L, f + L.nx + 1);
-        const T s4 = sm[ot[l] + f] * m00 + sm[ot[l] + f + 1] * m01 + sm[ot[l] + f + L.nx] * m10 +
-                     sm[ot[l] + f + L.nx + 1] * m11;
-        const T cnt = m00 + m01 + m10 + m11;
-        const int kc = J * C.nx + I;
-        const T rs = KIND == kDirichlet ? s4 * T(0.25) : s4 / (cnt > T(1) ? cnt : T(1));
-        sm[ob[l + 1] + kc] = rs * S.m_at(C, kc);
-      }
-    __syncthreads();
-  }
-  // Bottom solve.
-  {
-    const int lb = a.nl - 1;
-    const LevelDev<T>& B = a.lv[lb];
-    const bool zero = !(a.nonzero_init && a.lc == lb);
-    if (a.n_coarse > 0) {
-      S.sweeps(B, ou[lb], ot[lb], ob[lb], a.n_coarse, zero, a.w[2], tx, ty);
-    } else if (zero) {
-      for (int j = ty; j < B.ny; j += 32)
-        for (int i = tx; i < B.nx; i += 32) sm[ou[lb] + j * B.nx + i] = T(0);
-      __syncthreads();
-    }
-  }
-  // Up leg: u += P(u_c) (9/3/3/1 weights, mask renormalised), post-smoothing.
-  for (int l = a.nl - 2; l >= a.lc; --l) {
-    const LevelDev<T>& L = a.lv[l];
-    const LevelDev<T>& C = a.lv[l + 1];
-    for (int j = ty; j < L.ny; j += 32)
-      for (int i = tx; i < L.nx; i += 32) {
-        const int k = j * L.nx + i;
-        const T m = S.m_at(L, k);
-        const int J = j >> 1, I = i >> 1;
-        const int sj = (j & 1) ? 1 : -1, si = (i & 1) ? 1 : -1;
-        auto vm = [&](int jj, int ii, T& mm) -> T {
-          if (jj < 0 || jj >= C.ny || ii < 0 || ii >= C.nx) {
-            mm = T(0);
-            return T(0);
-          }
-          const int kc = jj * C.nx + ii;
-          mm = S.m_at(C, kc);
-          return sm[ou[l + 1] + kc];  // stored iterates are already masked
-        };
-        T mc, mx, my, md;
-        const T vc = vm(J, I, mc), vx = vm(J, I + si, mx), vy = vm(J + sj, I, my),
-                vd = vm(J + sj, I + si, md);
-        const T w = T(9) * vc + T(3) * vx + T(3) * vy + vd;
-        const T d = T(9) * mc + T(3) * mx + T(3) * my + md;
-        const T e = KIND == kDirichlet ? w * T(0.0625) : w / (d > T(1) ? d : T(1));
-        sm[ou[l] + k] = (sm[ou[l] + k] + e * m) * m;
-      }
-    __syncthreads();
-    S.sweeps(L, ou[l], ot[l], ob[l], a.n_post, false, a.w[1], tx, ty);
-  }
-  // Level lc's corrected iterate back to global memory.
-  {
-    const LevelDev<T>& G = a.lv[a.lc];
-    for (int j = ty; j < G.ny; j += 32)
-      for (int i = tx; i < G.nx; i += 32) G.u[j * G.nx + i] = sm[ou[a.lc] + j * G.nx + i];
-  }
-}
-template <typename T, int KIND>
-__global__ __launch_bounds__(kCoarseThreads) void mg_coarse_lds_kernel(CoarseArgs<T> a) {
-  extern __shared__ __align__(16) unsigned char coarse_smem[];
-  mg_coarse_lds_body<T, KIND>(a, coarse_smem);
-}
-
-// Dynamic LDS of the coarse kernel for levels lc .. nl-1 (u, t, b each).
-template <typename T>
-size_t coarse_lds_bytes(const CoarseArgs<T>& a) {
-  size_t n = 0;
-  for (int l = a.lc; l < a.nl; ++l) n += 3 * (size_t)a.lv[l].ny * a.lv[l].nx;
-  return n * sizeof(T);
-}
-// Dynamic LDS available to the coarse kernel: 160 KB less its static offset
-// table (3 x 16 ints).
-constexpr size_t kCoarseLdsMax = 160 * 1024 - 3 * 16 * sizeof(int);
-
-template <typename T, int KIND>
-static void launch_coarse(const CoarseArgs<T>& ca, hipStream_t s) {
-  const size_t lds = coarse_lds_bytes(ca);
-  if (lds <= kCoarseLdsMax)
-    hipLaunchKernelGGL((mg_coarse_lds_kernel<T, KIND>), dim3(1), dim3(kCoarseThreads), lds, s,
-                       ca);
-  else
-    hipLaunchKernelGGL((mg_coarse_kernel<T, KIND, false>), dim3(1), dim3(kCoarseThreads), 0, s,
-                       ca);
-}
-
-// Allow the LDS-resident coarse kernels the full 160 KB (once per process).
-static void coarse_lds_attributes() {
-  static bool done = false;
-  if (done) return;
-  done = true;
-  const int big = (int)kCoarseLdsMax;
-  (void)hipFuncSetAttribute((const void*)mg_coarse_lds_kernel<float, kDirichlet>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  (void)hipFuncSetAttribute((const void*)mg_coarse_lds_kernel<float, kNoflux>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  (void)hipFuncSetAttribute((const void*)mg_coarse_lds_kernel<double, kDirichlet>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, big);
-  (void)hipFuncSetAttribute((const void*)mg_coarse_lds_kernel<double, kNoflux>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, big);
-}
-
-// ---------------------------------------------------------------------------
 // Pointwise / matvec kernels on one level (global memory, 64 x 4 blocks).
 // ---------------------------------------------------------------------------
 template <typename T, int KIND>
@@ -2203,8 +1834,6 @@ static void free_hier(Hier<T>& H) {
   H.lv.clear();
 }
 
-// Cells at or below which a level is handled by the coarse single-workgroup kernel.
-constexpr int kCoarseCells = 64 * 64;
 // Independent solve slots (device scalar blocks) per plan.
 constexpr int kSlots = 8;
 
@@ -3692,12 +3321,6 @@ __global__ __launch_bounds__(256) void mg_wave_tile_batch_kernel(
   mg_wave_tile_body<NS, MODE, ZERO, kTileRows, true>(a, b - first[e], first[e + 1] - first[e]);
 }
 
-template <typename T, int KIND>
-__global__ __launch_bounds__(kCoarseThreads) void mg_coarse_batch_kernel(
-    const CoarseArgs<T>* __restrict__ args) {
-  extern __shared__ __align__(16) unsigned char coarse_smem[];
-  mg_coarse_lds_body<T, KIND>(args[blockIdx.x], coarse_smem);
-}
 
 template <int NV, int SITE>
 __global__ __launch_bounds__(kFinishThreads) void finish_batch_kernel(
@@ -3802,6 +3425,7 @@ struct BatchSlot {
   DevList<TileArgs<float>> wdown_upd[2], wup_cg[2];
   DevList<CoarseArgs<float>> coarse;
   size_t coarse_lds = 0;
+  int64_t coarse_cells = 0;  // the largest level lc
   DevList<FinishArgs> fin_cg, fin_res;
   DevList<UpdArgs> upd;
   DevList<RefUpdArgs> refupd;
@@ -3985,7 +3609,7 @@ static int batch_build_slot(MgBatch& B, int s) {
       c.omega = (float)Pm.omega;
       coarse_weights(Pm, c);
       c.done = &sc->done;
-      S.coarse_lds = std::max(S.coarse_lds, coarse_lds_bytes(c));
+      S.coarse_cells = std::max(S.coarse_cells, (int64_t)c.lv[c.lc].ny * c.lv[c.lc].nx);
       ca.push_back(c);
       cb.push_back(1);
     }
@@ -4007,6 +3631,8 @@ static int batch_build_slot(MgBatch& B, int s) {
     ua.push_back(UpdArgs{L0.ny, L0.nx, (int)gd.x, H.x, H.z, H.az, H.p, H.q, H.r, L0.nx, sc});
     ub.push_back((int)(gd.x * gd.y));
   }
+  for (const CoarseArgs<float>& c : ca)
+    S.coarse_lds = std::max(S.coarse_lds, coarse_lds_bytes(c, S.coarse_cells > kCoarseCells));
   FVX_CHECK_ARG(S.coarse_lds <= kCoarseLdsMax, "a member's coarse levels exceed the LDS");
   if (int rc = upload_list(ca, cb, S.coarse, B.allocs)) return rc;
   if (int rc = upload_list(fc, ones, S.fin_cg, B.allocs)) return rc;
@@ -4110,8 +3736,7 @@ static void batch_vcycle(MgBatch& B, BatchSlot& S, hipStream_t s, int step = -1)
     }
   }
   if (S.coarse.n)
-    hipLaunchKernelGGL((mg_coarse_batch_kernel<float, KIND>), dim3(S.coarse.n),
-                       dim3(kCoarseThreads), S.coarse_lds, s, S.coarse.args);
+    launch_coarse_batch<KIND>(S.coarse.args, S.coarse.n, S.coarse_cells, S.coarse_lds, s);
   for (int l = B.lc_max - 1; l >= 0; --l) {
     const DevList<TileArgs<float>>& u0 = S.up[0][l];
     const DevList<TileArgs<float>>& u1 = S.up[1][l];
@@ -4240,10 +3865,6 @@ int fvx_mg_batch_create(void* const* plans, int n, void** batch_out) {
     B->P.push_back(Pm);
   }
   coarse_lds_attributes();
-  (void)hipFuncSetAttribute((const void*)mg_coarse_batch_kernel<float, kDirichlet>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCoarseLdsMax);
-  (void)hipFuncSetAttribute((const void*)mg_coarse_batch_kernel<float, kNoflux>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCoarseLdsMax);
   *batch_out = B;
   return kOk;
 }

@@ -79,3 +79,25 @@ def test_batched_solve_matches_per_member_solver():
         assert io.converged
         err = np.abs(to_np(x) - to_np(xo)).max() / np.abs(to_np(xo)).max()
         assert err <= 1e-8, (m.shape, err)
+
+
+def test_batch_with_a_large_bottom_level():
+    """A member whose grid stops halving at 125 x 65 cells puts the whole
+    batch on the kernel for large bottom levels; every member still certifies
+    its FP64 residual, checked again with the oracle's operator."""
+    need_gpu()
+    rng = np.random.default_rng(5)
+    mgs, bs, xs, levs = [], [], [], []
+    for ny, nx in ((250, 130), (64, 96)):
+        m = np.ones((ny, nx))
+        mgs.append(S.build_multigrid_solver(m, 1.0, 1.0, 0.5, kind="dirichlet", precision="mixed",
+                                            n_pre=2, n_post=2, n_coarse=8, omega=0.85))
+        levs.append(fvx.build_multigrid(m, 1.0, 1.0, 0.5, n_levels=1, kind="dirichlet")[0])
+        bs.append(torch.tensor(rng.standard_normal((ny, nx)), device="cuda"))
+        xs.append(torch.zeros_like(bs[-1]))
+    batch = S.MultigridBatch(mgs)
+    batch.enqueue(bs, xs, n_outer=4, n_inner=(20, 20, 20, 20))
+    for (info, _, _), b, x, lev in zip(batch.status(n_outer=4), bs, xs, levs):
+        assert info.converged
+        r = to_np(b) - fvx.apply_operator(to_np(x), lev)
+        assert np.linalg.norm(r) <= 1.0001e-8 * np.linalg.norm(to_np(b))
