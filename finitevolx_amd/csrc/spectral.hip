@@ -10,13 +10,17 @@
 //         -4/dx^2 sin^2(pi k / (2 n)); the k = l = 0 mode is set to zero
 //         when the operator is singular)
 //   fft : periodic (eigenvalues -4/dx^2 sin^2(pi k / n))
-// Transforms along x run as batched real FFTs (hipFFT) of the odd / even
-// extension of each row, written transposed so the y transform is again a
-// batch of contiguous rows.
+// DST / DCT plans up to the sizes of use_gemm transform by matrix products on
+// the FP64 matrix cores (spec_gemm_kernel: four launches for a whole batch of
+// right-hand sides); larger ones by batched real FFTs (hipFFT) of the odd /
+// even extension of each row, written transposed so the y transform is again a
+// batch of contiguous rows; periodic solves by hipFFT's 2-D real FFT.
 
 #include <hipfft/hipfft.h>
 
+#include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "fvx_common.hpp"
@@ -164,6 +168,257 @@ struct FftTypes<float> {
   }
 };
 
+// ---------------------------------------------------------------------------
+// Transforms as matrix products.
+//
+// The kernels sin(pi (j + 1) (k + 1) / (n + 1)) and cos(pi (2 j + 1) k / 2 n)
+// are even (k even) or odd (k odd) under j -> n - 1 - j, so a forward
+// transform contracts x_j + x_{n-1-j} with the h x n0 matrix of the even k
+// (class 0) and x_j - x_{n-1-j} with the h x n1 matrix of the odd ones (class
+// 1; h = n0 = ceil(n / 2), n1 = floor(n / 2)), and the inverse one gives
+// x_j = E_j + O_j, x_{n-1-j} = E_j - O_j: half the products of the full
+// matrix.  Spectral indices stay ordered by class.
+//
+// Why: for the extended lengths 2 (n + 1) hipFFT falls to Bluestein's method
+// at most n (n = 512: 1026 = 2 3^3 19), and each transform took an extension,
+// 3-4 FFT kernels and an extraction per right-hand side.  Arithmetic is FP64
+// for both precisions, each sum in chunks of 16 products.  Bound: FP64 matrix
+// cores (45 TFLOP/s with v_mfma_f64_16x16x4 alone; 64 TFLOP/s of plain FMAs
+// would need four times the LDS reads).  Measured: 3 x 512 x 768 DST 151 us a
+// solve (20 TFLOP/s) against 535 through hipFFT; error against long double
+// 3.2e-16 to 4.4e-16 (FP32 data 3.6e-8 to 6.1e-8) from 64 to 512 points, hipFFT
+// 3.1e-16 to 7.6e-16 (1.4e-7 to 3.1e-7).
+// ---------------------------------------------------------------------------
+constexpr int kSpecBatch = 16;  // right-hand sides a launch
+
+// Whether an extended length has a direct FFT (hipFFT's radices).
+static bool fft_smooth(int m) {
+  for (int p : {2, 3, 5, 7, 11, 13})
+    while (m % p == 0) m /= p;
+  return m == 1;
+}
+// Matrix products up to the size where the FFTs take less time (us a solve,
+// n^2, matrix / FFT).  FP64: direct lengths 768 110 / 132, 1000 168 / 155;
+// others 1024 160 / 397, 1536 508 / 636.  FP32 (products in FP64): direct 512
+// 52 / 67, 768 115 / 107; others 1024 175 / 230, 1200 300 / 278.
+static bool use_gemm(int ny, int nx, int bc, int bits) {
+  if (bc == kFft) return false;
+  const int ext = bc == kDst ? 2 : 0;
+  const bool direct = fft_smooth(2 * nx + ext) && fft_smooth(2 * ny + ext);
+  const int most = bits == 64 ? (direct ? 1800 : 3072) : (direct ? 1400 : 2200);
+  return ny + nx <= most;
+}
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+template <typename T>
+struct SpecGemm {
+  const T* in;   // forward: physical along the transformed axis, else spectral
+  T* out;
+  int64_t ld_in, bs_in, ld_out, bs_out;  // row pitch and batch stride
+  const double *s0, *s1;  // class matrices [h][n0], [h][n1]
+  int n, h, n0, n1;       // the transformed axis
+  int other;              // points along the other axis
+  // Division by the eigenvalues (forward, second axis): squared sines of this
+  // axis and the other in spectral order.
+  const double *et, *eo;
+  double ct, co, scale;
+  int divide, halve0;  // halve0: the DCT's k = 0 weight along each axis
+  double lam[kSpecBatch];
+};
+
+// LEFT: the transformed axis is the arrays' row index (out = S in), else the
+// column index (out = in S).  A workgroup owns 32 outputs x 32 points of the
+// other axis; its 8 waves are two groups that split each K slab (64 points)
+// between them, four waves of 16 x 16 outputs in a group, and sum their parts
+// through LDS at the end.  Small tiles and two groups keep several short
+// chains on every CU: 3 x 512 x 768 takes 143 us a solve (151 with the chunked
+// sums), 156 with tiles of 64, 167 with four groups.
+constexpr int kSpecThreads = 512;
+template <typename T, bool LEFT, bool INV>
+__global__ __launch_bounds__(kSpecThreads) void spec_gemm_kernel(SpecGemm<T> g) {
+  constexpr int BT = 32, BK = 64, P = BT + 2, PER = BT * BK / kSpecThreads;
+  constexpr int NC = INV ? 2 : 1;  // accumulated classes
+  __shared__ __align__(16) double smem[2 * BK * P];
+  double(*sm)[P] = reinterpret_cast<double(*)[P]>(smem);           // matrix operand [k][t]
+  double(*sd)[P] = reinterpret_cast<double(*)[P]>(smem + BK * P);  // data operand [k][o]
+  static_assert(NC * 4 * 256 <= 2 * BK * P, "a group's sums fit in the slabs");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave >> 2, w4 = wave & 3;
+  const int o0 = blockIdx.x * BT;
+  int cls = 0, t0 = blockIdx.y * BT;
+  if constexpr (!INV) {
+    const int tiles0 = (g.n0 + BT - 1) / BT;
+    if ((int)blockIdx.y >= tiles0) {
+      cls = 1;
+      t0 = (blockIdx.y - tiles0) * BT;
+    }
+  }
+  const T* in = g.in + (int64_t)blockIdx.z * g.bs_in;
+  const int nt = INV ? g.h : (cls ? g.n1 : g.n0);  // outputs of the class
+  f64x4 acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] = f64x4{0., 0., 0., 0.};
+
+  // Element e of a slab: its place (contiguous in memory along the fast index).
+  auto mat_at = [&](int e, int& k, int& t) {
+    if constexpr (INV) {
+      k = e % BK;
+      t = e / BK;
+    } else {
+      t = e % BT;
+      k = e / BT;
+    }
+  };
+  auto dat_at = [&](int e, int& k, int& o) {
+    if constexpr (LEFT) {
+      o = e % BT;
+      k = e / BT;
+    } else {
+      k = e % BK;
+      o = e / BK;
+    }
+  };
+  double rm[PER], rd[PER];
+  auto load = [&](int c, int k0) {
+    const double* S = c ? g.s1 : g.s0;
+    const int nc = c ? g.n1 : g.n0, K = INV ? nc : g.h;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      int k, t;
+      mat_at(tid + i * kSpecThreads, k, t);
+      k += k0;
+      t += t0;
+      rm[i] = (k < K && t < nt) ? S[INV ? (int64_t)t * nc + k : (int64_t)k * nc + t] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      int k, o;
+      dat_at(tid + i * kSpecThreads, k, o);
+      k += k0;
+      o += o0;
+      double v = 0.0;
+      if (k < K && o < g.other) {
+        auto at = [&](int q) -> double {
+          return (double)in[LEFT ? (int64_t)q * g.ld_in + o : (int64_t)o * g.ld_in + q];
+        };
+        if constexpr (INV) {
+          v = at((c ? g.n0 : 0) + k);
+        } else {
+          const int km = g.n - 1 - k;
+          const double u = at(k), w = at(km);
+          v = c ? u - w : u + w;
+          if (km == k) v = c ? 0.0 : u;  // (the middle point has no partner)
+        }
+      }
+      rd[i] = v;
+    }
+  };
+  const int lr = lane & 15, lk = lane >> 4;
+  const int wm = (w4 >> 1) * 16, wn = (w4 & 1) * 16;  // rows / columns of D
+#pragma unroll
+  for (int ci = 0; ci < NC; ++ci) {
+    const int c = INV ? ci : cls;
+    const int K = INV ? (c ? g.n1 : g.n0) : g.h;
+    load(c, 0);
+    for (int k0 = 0; k0 < K; k0 += BK) {
+      __syncthreads();  // (the previous slab has been read)
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        int k, t;
+        mat_at(tid + i * kSpecThreads, k, t);
+        sm[k][t] = rm[i];
+        dat_at(tid + i * kSpecThreads, k, t);
+        sd[k][t] = rd[i];
+      }
+      __syncthreads();
+      if (k0 + BK < K) load(c, k0 + BK);
+      // chunks of 16 products, summed on their own: a serial sum of the whole
+      // axis rounds sqrt(n / 16) times as much
+      f64x4 chunk[2] = {f64x4{0., 0., 0., 0.}, f64x4{0., 0., 0., 0.}};
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = grp * 32 + h * 16 + 4 * kk + lk;
+          const double fa = (LEFT ? sm : sd)[k][wm + lr], fb = (LEFT ? sd : sm)[k][wn + lr];
+          chunk[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, fb, chunk[h], 0, 0, 0);
+        }
+      acc[ci] += chunk[0] + chunk[1];
+    }
+  }
+  // The second group's sums into the first's.
+  f64x4* part = reinterpret_cast<f64x4*>(smem) + w4 * 64 + lane;
+  __syncthreads();
+  if (grp == 1) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) part[c * 256] = acc[c];
+  }
+  __syncthreads();
+  if (grp == 1) return;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) acc[c] += part[c * 256];
+
+  // D of a 16 x 16 block: row 4 i + lane / 16, column lane % 16.
+  T* out = g.out + (int64_t)blockIdx.z * g.bs_out;
+  const double lam = g.lam[blockIdx.z];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int m = wm + 4 * i + lk, n = wn + lr;
+    const int t = t0 + (LEFT ? m : n), o = o0 + (LEFT ? n : m);
+    if (t >= nt || o >= g.other) continue;
+    auto put_at = [&](int q, double v) {
+      out[LEFT ? (int64_t)q * g.ld_out + o : (int64_t)o * g.ld_out + q] = (T)v;
+    };
+    if constexpr (INV) {
+      const double e = acc[0][i], d = acc[NC - 1][i];
+      put_at(t, e + d);
+      if (g.n - 1 - t != t) put_at(g.n - 1 - t, e - d);
+    } else {
+      const int q = (cls ? g.n0 : 0) + t;
+      double v = acc[0][i];
+      if (g.divide) {
+        const double den = g.ct * g.et[q] + g.co * g.eo[o] - lam;
+        double f = g.scale;
+        if (g.halve0) f *= (q == 0 ? 0.5 : 1.0) * (o == 0 ? 0.5 : 1.0);
+        v = den != 0.0 ? v * f / den : 0.0;
+      }
+      put_at(q, v);
+    }
+  }
+}
+
+// Class matrices and squared sines of one axis of n points.
+__global__ void spec_matrix_kernel(double* __restrict__ s0, double* __restrict__ s1,
+                                   double* __restrict__ e, int n, int bc) {
+  const int h = (n + 1) / 2, n0 = h, n1 = n / 2;
+  const int64_t total = (int64_t)h * n;
+  for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < total;
+       x += (int64_t)gridDim.x * blockDim.x) {
+    const int j = (int)(x / n), q = (int)(x % n);
+    const int c = q >= n0, r = c ? q - n0 : q, k = 2 * r + c;
+    // the angle as an integer multiple of pi / n', reduced exactly
+    double v;
+    if (bc == kDst) {
+      const int64_t m = ((int64_t)(j + 1) * (k + 1)) % (2 * (n + 1));
+      v = sinpi((double)m / (n + 1));
+    } else {
+      const int64_t m = ((int64_t)(2 * j + 1) * k) % (4 * n);
+      v = cospi((double)m / (2.0 * n));
+    }
+    (c ? s1 : s0)[(int64_t)j * (c ? n1 : n0) + r] = v;
+    if (j == 0) {
+      const double sn = bc == kDst ? sinpi((k + 1) / (2.0 * (n + 1))) : sinpi(k / (2.0 * n));
+      e[q] = sn * sn;
+    }
+  }
+}
+
+struct SpecAxis {
+  int n = 0;
+  double *s0 = nullptr, *s1 = nullptr, *e = nullptr;  // one allocation, s0
+};
+
 struct SpecPlan {
   int ny, nx, bc, prec;
   // per-direction batched 1-D plans (x: ny rows of length Mx; y: nx rows of length My)
@@ -172,6 +427,8 @@ struct SpecPlan {
   void* spec = nullptr;  // complex buffer
   void* a = nullptr;     // transposed real (nx, ny)
   void* b = nullptr;     // real (ny, nx) / second transposed buffer
+  bool gemm = false;     // transforms by matrix products
+  SpecAxis ax, ay;
 };
 
 #define FVX_FFT(call)                                                  \
@@ -183,9 +440,27 @@ struct SpecPlan {
     }                                                                  \
   } while (0)
 
+static int spec_axis(SpecAxis& A, int n, int bc) {
+  A.n = n;
+  const size_t h = (n + 1) / 2, n1 = n / 2;
+  FVX_HIP(hipMalloc(&A.s0, (h * h + h * n1 + n) * sizeof(double)));
+  A.s1 = A.s0 + h * h;
+  A.e = A.s1 + h * n1;
+  hipLaunchKernelGGL(spec_matrix_kernel, dim3(1024), dim3(256), 0, nullptr, A.s0, A.s1, A.e, n, bc);
+  FVX_LAUNCH_CHECK();
+  FVX_HIP(hipStreamSynchronize(nullptr));  // solves run on any stream
+  return kOk;
+}
+
 template <typename T>
 static int spec_create(SpecPlan* P) {
   const int ny = P->ny, nx = P->nx;
+  if (use_gemm(ny, nx, P->bc, P->prec)) {
+    P->gemm = true;
+    FVX_HIP(hipMalloc(&P->a, 2 * (size_t)ny * nx * sizeof(T)));
+    if (int rc = spec_axis(P->ax, nx, P->bc)) return rc;
+    return spec_axis(P->ay, ny, P->bc);
+  }
   using FT = FftTypes<T>;
   using C = typename Cplx<T>::type;
   size_t ext_elems = 0, spec_elems = 0;
@@ -257,11 +532,74 @@ __global__ void copy_pitched_kernel(const T* __restrict__ src, int64_t lds, T* _
   if (i < nx && j < ny) dst[(int64_t)j * ldd + i] = src[(int64_t)j * lds + i];
 }
 
+template <typename T, bool LEFT, bool INV>
+static int launch_spec(const SpecGemm<T>& g, int nb, hipStream_t s) {
+  const dim3 grid(cdiv(g.other, 32), INV ? cdiv(g.h, 32) : cdiv(g.n0, 32) + cdiv(g.n1, 32), nb);
+  hipLaunchKernelGGL((spec_gemm_kernel<T, LEFT, INV>), grid, dim3(kSpecThreads), 0, s, g);
+  FVX_LAUNCH_CHECK();
+  return kOk;
+}
+
+// nb solves (right-hand side b at rhs + b bs_rhs, solution at out + b bs_out,
+// its lambda in lam[b]) by matrix products; work: 2 nb ny nx elements.
+template <typename T>
+static int gemm_solve(SpecPlan* P, const T* rhs, int64_t ld_rhs, int64_t bs_rhs, T* out,
+                      int64_t ld_out, int64_t bs_out, int nb, const double* lam, double dx,
+                      double dy, T* work, hipStream_t s) {
+  const int ny = P->ny, nx = P->nx;
+  const int64_t N = (int64_t)ny * nx;
+  for (int b0 = 0; b0 < nb; b0 += kSpecBatch) {
+    const int m = std::min(kSpecBatch, nb - b0);
+    T *A = work + 2 * b0 * N, *B = A + m * N;
+    SpecGemm<T> g;
+    std::memset(&g, 0, sizeof(g));
+    for (int b = 0; b < m; ++b) g.lam[b] = lam[b0 + b];
+    auto axis = [&](const SpecAxis& X, int other) {
+      g.n = X.n;
+      g.h = g.n0 = (X.n + 1) / 2;
+      g.n1 = X.n / 2;
+      g.s0 = X.s0;
+      g.s1 = X.s1;
+      g.other = other;
+    };
+    auto arrays = [&](const T* in, int64_t ldi, int64_t bsi, T* o, int64_t ldo, int64_t bso) {
+      g.in = in;
+      g.ld_in = ldi;
+      g.bs_in = bsi;
+      g.out = o;
+      g.ld_out = ldo;
+      g.bs_out = bso;
+    };
+    axis(P->ax, ny);
+    arrays(rhs + b0 * bs_rhs, ld_rhs, bs_rhs, A, nx, N);
+    if (int rc = launch_spec<T, false, false>(g, m, s)) return rc;
+    axis(P->ay, nx);
+    arrays(A, nx, N, B, nx, N);
+    g.divide = 1;
+    g.halve0 = P->bc == kDct;
+    g.et = P->ay.e;
+    g.eo = P->ax.e;
+    g.ct = -4.0 / (dy * dy);
+    g.co = -4.0 / (dx * dx);
+    g.scale = P->bc == kDst ? (2.0 / (nx + 1)) * (2.0 / (ny + 1)) : (2.0 / nx) * (2.0 / ny);
+    if (int rc = launch_spec<T, true, false>(g, m, s)) return rc;
+    g.divide = 0;
+    arrays(B, nx, N, A, nx, N);
+    if (int rc = launch_spec<T, true, true>(g, m, s)) return rc;
+    axis(P->ax, ny);
+    arrays(A, nx, N, out + b0 * bs_out, ld_out, bs_out);
+    if (int rc = launch_spec<T, false, true>(g, m, s)) return rc;
+  }
+  return kOk;
+}
+
 template <typename T>
 static int spec_solve(SpecPlan* P, const T* rhs, int64_t ld_rhs, T* out, int64_t ld_out,
                       double dx, double dy, double lam, hipStream_t s) {
   using C = typename Cplx<T>::type;
   const int ny = P->ny, nx = P->nx;
+  if (P->gemm)
+    return gemm_solve<T>(P, rhs, ld_rhs, 0, out, ld_out, 0, 1, &lam, dx, dy, (T*)P->a, s);
   T* A = (T*)P->a;
   T* B = (T*)P->b;
   if (P->bc == kFft) {
@@ -302,6 +640,8 @@ static int spec_solve(SpecPlan* P, const T* rhs, int64_t ld_rhs, T* out, int64_t
 
 extern "C" {
 
+int fvx_spectral_plan_destroy(void* plan);
+
 // bc: 0 = DST-I (Dirichlet), 1 = DCT-II (Neumann), 2 = FFT (periodic);
 // precision 32 or 64.  ny, nx: the array the solve runs on (interior only).
 int fvx_spectral_plan_create(int ny, int nx, int bc, int precision, void** plan_out) {
@@ -317,7 +657,7 @@ int fvx_spectral_plan_create(int ny, int nx, int bc, int precision, void** plan_
   P->prec = precision;
   int rc = precision == 64 ? spec_create<double>(P) : spec_create<float>(P);
   if (rc) {
-    delete P;
+    fvx_spectral_plan_destroy(P);
     return rc;
   }
   *plan_out = P;
@@ -331,6 +671,8 @@ int fvx_spectral_plan_destroy(void* plan) {
   (void)hipDeviceSynchronize();
   for (hipfftHandle h : {P->fx, P->fy, P->ix, P->iy, P->f2, P->i2})
     if (h) hipfftDestroy(h);
+  (void)hipFree(P->ax.s0);
+  (void)hipFree(P->ay.s0);
   (void)hipFree(P->ext);
   (void)hipFree(P->spec);
   (void)hipFree(P->a);
@@ -360,4 +702,34 @@ int fvx_spectral_helmholtz_f32(void* plan, const float* rhs, int64_t ld_rhs, flo
   FVX_CHECK_ARG(dx > 0 && dy > 0, "grid spacing must be positive");
   return spec_solve<float>(P, rhs, ld_rhs, out, ld_out, dx, dy, lambda_, (hipStream_t)stream);
 }
+
+// nb solves of contiguous (ny, nx) fields back to back, (lap - lambda_[b])
+// out_b = rhs_b (lambda_: host array); out may be rhs.  work: device scratch of 2 nb ny nx elements for the call (the caller's, so that calls on
+// several streams or threads do not share any); may be null for the periodic
+// boundary condition.
+#define FVX_SPEC_BATCH(SUF, T, PREC)                                                             \
+  int fvx_spectral_helmholtz_batch_##SUF(void* plan, const T* rhs, T* out, int nb,               \
+                                         const double* lambda_, double dx, double dy, T* work,   \
+                                         void* stream) {                                         \
+    using namespace fvx;                                                                         \
+    FVX_CHECK_ARG(plan && rhs && out && lambda_, "null argument");                               \
+    SpecPlan* P = (SpecPlan*)plan;                                                               \
+    FVX_CHECK_ARG(P->prec == PREC, "plan was built for the other precision");                    \
+    FVX_CHECK_ARG(dx > 0 && dy > 0, "grid spacing must be positive");                            \
+    FVX_CHECK_ARG(nb >= 0, "negative batch");                                                    \
+    const int64_t N = (int64_t)P->ny * P->nx;                                                    \
+    if (P->gemm) {                                                                               \
+      FVX_CHECK_ARG(work || nb == 0, "null work array");                                         \
+      return gemm_solve<T>(P, rhs, P->nx, N, out, P->nx, N, nb, lambda_, dx, dy, work,           \
+                           (hipStream_t)stream);                                                 \
+    }                                                                                            \
+    for (int b = 0; b < nb; ++b)                                                                 \
+      if (int rc = spec_solve<T>(P, rhs + b * N, P->nx, out + b * N, P->nx, dx, dy, lambda_[b],  \
+                                 (hipStream_t)stream))                                           \
+        return rc;                                                                               \
+    return kOk;                                                                                  \
+  }
+FVX_SPEC_BATCH(f64, double, 64)
+FVX_SPEC_BATCH(f32, float, 32)
+#undef FVX_SPEC_BATCH
 }

@@ -483,6 +483,8 @@ _lib.extra_signatures({
     "fvx_spectral_plan_destroy": [_vp],
     "fvx_spectral_helmholtz_f64": [_vp, _vp, _i64, _vp, _i64, _d, _d, _d, _vp],
     "fvx_spectral_helmholtz_f32": [_vp, _vp, _i64, _vp, _i64, _d, _d, _d, _vp],
+    "fvx_spectral_helmholtz_batch_f64": [_vp, _vp, _vp, _i, C.POINTER(_d), _d, _d, _vp, _vp],
+    "fvx_spectral_helmholtz_batch_f32": [_vp, _vp, _vp, _i, C.POINTER(_d), _d, _d, _vp, _vp],
 })
 
 _BC = {"dst": 0, "dct": 1, "fft": 2}
@@ -507,6 +509,8 @@ _SPEC_PLANS: dict = {}
 
 
 def _spectral(rhs, dx, dy, lambda_, bc):
+    """Solve every trailing 2-D slice in one call; ``lambda_`` is a number or
+    one per entry of the last leading axis."""
     b = _lib.as_field(rhs)
     if b.dim() < 2:
         raise ValueError("spectral solves need at least 2-D input")
@@ -518,28 +522,31 @@ def _spectral(rhs, dx, dy, lambda_, bc):
         if len(_SPEC_PLANS) > 8:
             _SPEC_PLANS.clear()
         plan = _SPEC_PLANS[key] = _SpecPlan(ny, nx, bc, bits)
-    flat = b.reshape(-1, ny, nx)
-    out = torch.empty_like(flat)
-    for k in range(flat.shape[0]):
-        _lib.call(f"fvx_spectral_helmholtz_{_lib.suffix(b)}", plan.h, flat[k].data_ptr(), nx,
-                  out[k].data_ptr(), nx, float(dx), float(dy), float(lambda_), _lib.stream())
-    return out.reshape(b.shape)
+    nb = b.numel() // (ny * nx) if b.numel() else 0
+    out = torch.empty_like(b)
+    # (scratch of this call's stream: solves on several streams share a plan)
+    work = None if bc == "fft" else torch.empty((2, *b.shape), dtype=b.dtype, device=b.device)
+    lam = np.broadcast_to(np.asarray(lambda_, dtype=np.float64), b.shape[:-2]).ravel()
+    _lib.call(f"fvx_spectral_helmholtz_batch_{_lib.suffix(b)}", plan.h, b.data_ptr(),
+              out.data_ptr(), nb, (_d * nb)(*lam), float(dx), float(dy), _lib.ptr(work),
+              _lib.stream())
+    return out
 
 
 def solve_helmholtz_dst(rhs, dx, dy, lambda_=0.0):
     """Dirichlet ``(lap - lambda) psi = rhs`` on an interior-only array (DST-I)."""
-    return _spectral(rhs, dx, dy, lambda_, "dst")
+    return _spectral(rhs, dx, dy, float(lambda_), "dst")
 
 
 def solve_helmholtz_dct(rhs, dx, dy, lambda_=0.0):
     """Neumann (no-flux, cell-centred) Helmholtz solve (DCT-II); the mean
     mode is set to zero when ``lambda_ == 0``."""
-    return _spectral(rhs, dx, dy, lambda_, "dct")
+    return _spectral(rhs, dx, dy, float(lambda_), "dct")
 
 
 def solve_helmholtz_fft(rhs, dx, dy, lambda_=0.0):
     """Periodic Helmholtz solve (2-D real FFT); zero mean mode when singular."""
-    return _spectral(rhs, dx, dy, lambda_, "fft")
+    return _spectral(rhs, dx, dy, float(lambda_), "fft")
 
 
 def solve_poisson_dst(rhs, dx, dy):
@@ -657,24 +664,24 @@ def pv_inversion(pv, dx, dy, lambda_, bc="dst", method="spectral", mask=None,
     pv = _lib.as_field(pv)
     lam = np.asarray(lambda_, dtype=np.float64)
 
-    def one(f, lk):
-        if method == "spectral":
-            return _spectral_dispatch(f, dx, dy, lk, bc)
-        return _solve_cg_method(f, dx, dy, lk, mask, preconditioner)
-
-    if lam.ndim == 0:
-        flat = pv.reshape(-1, *pv.shape[-2:])
-        out = torch.stack([one(f, float(lam)) for f in flat])
-        return out.reshape(pv.shape)
-    if pv.dim() < 3:
-        raise ValueError(f"pv must have at least 3 dims when lambda_ is an array, got shape "
-                         f"{tuple(pv.shape)}")
-    nl = lam.shape[0]
-    if pv.shape[-3] != nl:
-        raise ValueError(f"pv.shape[-3]={pv.shape[-3]} does not match lambda_ length {nl}")
-    flat = pv.reshape(-1, nl, *pv.shape[-2:])
-    out = torch.stack([torch.stack([one(f[k], float(lam[k])) for k in range(nl)])
-                       for f in flat])
+    if lam.ndim > 0:
+        if pv.dim() < 3:
+            raise ValueError(f"pv must have at least 3 dims when lambda_ is an array, got shape "
+                             f"{tuple(pv.shape)}")
+        nl = lam.shape[0]
+        if pv.shape[-3] != nl:
+            raise ValueError(f"pv.shape[-3]={pv.shape[-3]} does not match lambda_ length {nl}")
+        lam = np.array([float(lk) for lk in lam])
+    if pv.numel() == 0:
+        raise RuntimeError(f"pv has no cells: shape {tuple(pv.shape)}")
+    if method == "spectral":
+        if bc in _HELMHOLTZ_DISPATCH and lam.ndim > 0:
+            return _spectral(pv, dx, dy, lam, bc)
+        return _spectral_dispatch(pv, dx, dy, lam, bc)
+    flat = pv.reshape(-1, *pv.shape[-2:])
+    per = np.broadcast_to(lam, pv.shape[:-2]).ravel()
+    out = torch.stack([_solve_cg_method(f, dx, dy, float(lk), mask, preconditioner)
+                       for f, lk in zip(flat, per)])
     return out.reshape(pv.shape)
 
 

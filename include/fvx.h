@@ -343,7 +343,8 @@ int fvx_mg_batch_status(void* batch, int slot, int n_outer_budget, fvx_cg_info* 
  * used by scripts/qg_1p5_layer.py:443).  bc 0 = DST-I (Dirichlet just
  * outside the array), 1 = DCT-II (no-flux cell-centred Neumann), 2 = FFT
  * (periodic); each is the exact inverse of the matching 5-point operator.
- * The plan owns hipFFT plans and work buffers for one (ny, nx, bc, dtype). */
+ * The plan owns the transform matrices or hipFFT plans and work buffers of
+ * one (ny, nx, bc, dtype). */
 int fvx_spectral_plan_create(int ny, int nx, int bc, int precision, void** plan_out);
 int fvx_spectral_plan_destroy(void* plan);
 int fvx_spectral_helmholtz_f32(void* plan, const float* rhs, int64_t ld_rhs, float* out,
@@ -352,6 +353,16 @@ int fvx_spectral_helmholtz_f32(void* plan, const float* rhs, int64_t ld_rhs, flo
 int fvx_spectral_helmholtz_f64(void* plan, const double* rhs, int64_t ld_rhs, double* out,
                                int64_t ld_out, double dx, double dy, double lambda_,
                                void* stream);
+/* nb solves of contiguous (ny, nx) fields back to back, (lap - lambda_[b])
+ * out_b = rhs_b (lambda_: host array of nb; pv_inversion's per-layer lambda,
+ * solvers/elliptic.py:390-542); out may be rhs.  work: device scratch of
+ * 2 nb ny nx elements that the call uses alone (null for bc 2). */
+int fvx_spectral_helmholtz_batch_f32(void* plan, const float* rhs, float* out, int nb,
+                                     const double* lambda_, double dx, double dy, float* work,
+                                     void* stream);
+int fvx_spectral_helmholtz_batch_f64(void* plan, const double* rhs, double* out, int nb,
+                                     const double* lambda_, double dx, double dy, double* work,
+                                     void* stream);
 
 /* ---- QG 1.5-layer step (composition; nearest reference
  * scripts/qg_1p5_layer.py:420-497; operators as cited above) -------------- */
