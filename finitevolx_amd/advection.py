@@ -31,6 +31,10 @@ _lib.extra_signatures({
                                       _vp]
     for s in ("f32", "f64") for v in ("", "_noalloc")
 })
+_lib.extra_signatures({
+    f"fvx_advection_rk3_step_into_{s}": [_i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _d,
+                                         _d, _d, _vp, _vp] for s in ("f32", "f64")
+})
 
 
 def method_codes(method: str) -> tuple[int, int]:
@@ -78,9 +82,9 @@ class Advection2D:
         (``enforce_periodic``), and the result leaves with its ghosts filled;
         the same as ``enforce_periodic(rk3_ssp_step(h, lambda q:
         self(enforce_periodic(q, ng), u, v, method), dt), ng)`` as one native
-        call (``fvx_advection_rk3_step_*``).  Returns a new array."""
+        call (``fvx_advection_rk3_step_into_*``).  Returns a new array."""
         m, lim = method_codes(method)
-        h = _lib.as_field(h).clone()
+        h = _lib.as_field(h)
         u = _lib.as_field(u, h.dtype)
         v = _lib.as_field(v, h.dtype)
         if h.dim() != 2 or h.shape != u.shape or h.shape != v.shape:
@@ -91,10 +95,13 @@ class Advection2D:
             mh = self.mask.device("h")
             if method in _MASK_DISPATCHABLE:
                 tx, ty = self.mask.device("tier_x"), self.mask.device("tier_y")
-        _lib.call(f"fvx_advection_rk3_step_{_lib.suffix(h)}", m, lim, h.data_ptr(), u.data_ptr(),
-                  v.data_ptr(), _lib.ptr(tx), _lib.ptr(ty), _lib.ptr(mh), ny, nx, int(ng),
-                  float(self.grid.dx), float(self.grid.dy), float(dt), _lib.stream())
-        return h
+        out = torch.empty_like(h)
+        work = torch.empty((2, ny, nx), dtype=h.dtype, device=h.device)
+        _lib.call(f"fvx_advection_rk3_step_into_{_lib.suffix(h)}", m, lim, h.data_ptr(),
+                  out.data_ptr(), u.data_ptr(), v.data_ptr(), _lib.ptr(tx), _lib.ptr(ty),
+                  _lib.ptr(mh), ny, nx, int(ng), float(self.grid.dx), float(self.grid.dy),
+                  float(dt), work.data_ptr(), _lib.stream())
+        return out
 
 
 _lib.extra_signatures({

@@ -133,34 +133,67 @@ __device__ __forceinline__ T wenoz3_right(T q0, T qp, T qpp) {  // weno.py:438-4
 // for positive flow and (qppp, qpp, qp, q0, qm) for negative flow: the
 // right-biased reference formula (weno.py:462-491) is the left-biased one
 // (weno.py:350-376) on the mirrored stencil, so one evaluation serves both.
+//
+// The face value is c + S with S a function of the four differences d1 = b - a,
+// d2 = c - b, d3 = d - c, d4 = e - d alone:
+//   candidates  - c : 5/6 d2 - 1/3 d1,  1/6 d2 + 1/3 d3,  2/3 d3 - 1/6 d4
+//   indicators / k1 : s^2 + 3/13 r^2 (k1 = 13/12, k2 = 1/4) with
+//                     s = d2 - d1, r = 2 d2 + s;  s = d3 - d2, r = d2 + d3;
+//                     s = d4 - d3, r = s - 2 d3
+// (the weights are ratios, so k1 divides out with eps / k1).  A difference is
+// shared by the four faces around it and the mirrored stencil only reverses
+// them, so a face costs ~55 issue slots instead of ~69 from five values.
+// S is odd: the mirrored (negative) flow has S(-d) = -S(d).
 template <typename T, bool Z>
-__device__ __forceinline__ T weno5_upwind(T a, T b, T c, T d, T e) {
-  const T qi1 = T(1.0 / 3.0) * a - T(7.0 / 6.0) * b + T(11.0 / 6.0) * c;
-  const T qi2 = T(-1.0 / 6.0) * b + T(5.0 / 6.0) * c + T(1.0 / 3.0) * d;
-  const T qi3 = T(1.0 / 3.0) * c + T(5.0 / 6.0) * d - T(1.0 / 6.0) * e;
-  const T k1 = T(13.0 / 12.0), k2 = T(0.25);
-  const T s1 = a - T(2) * b + c, r1 = a - T(4) * b + T(3) * c;
-  const T s2 = b - T(2) * c + d, r2 = b - d;
-  const T s3 = c - T(2) * d + e, r3 = T(3) * c - T(4) * d + e;
-  const T b1 = k1 * (s1 * s1) + k2 * (r1 * r1);
-  const T b2 = k1 * (s2 * s2) + k2 * (r2 * r2);
-  const T b3 = k1 * (s3 * s3) + k2 * (r3 * r3);
+__device__ __forceinline__ T weno5_delta(T d1, T d2, T d3, T d4) {
+  const T p1 = T(5.0 / 6.0) * d2 - T(1.0 / 3.0) * d1;
+  const T p2 = T(1.0 / 6.0) * d2 + T(1.0 / 3.0) * d3;
+  const T p3 = T(2.0 / 3.0) * d3 - T(1.0 / 6.0) * d4;
+  const T s1 = d2 - d1, r1 = T(2) * d2 + s1;  // a - 4 b + 3 c
+  const T s2 = d3 - d2, r2 = d2 + d3;         // d - b
+  const T s3 = d4 - d3, r3 = s3 - T(2) * d3;  // 3 c - 4 d + e
+  const T k = T(3.0 / 13.0);
   if constexpr (!Z) {  // Jiang-Shu weights d_k / (b_k + eps)^2, eps 1e-8
-    const T eps = T(1e-8);
-    const T t1 = b1 + eps, t2 = b2 + eps, t3 = b3 + eps;
-    return blend3(T(0.1), t1 * t1, qi1, T(0.6), t2 * t2, qi2, T(0.3), t3 * t3, qi3);
+    const T eps = T(1e-8 * 12.0 / 13.0);
+    const T t1 = s1 * s1 + ((k * r1) * r1 + eps), t2 = s2 * s2 + ((k * r2) * r2 + eps),
+            t3 = s3 * s3 + ((k * r3) * r3 + eps);
+    return blend3(T(0.1), t1 * t1, p1, T(0.6), t2 * t2, p2, T(0.3), t3 * t3, p3);
   } else {  // WENO-Z (Borges et al. 2008), weno.py:379-410, eps 1e-16
-    const T eps = T(1e-16);
+    const T eps = T(1e-16 * 12.0 / 13.0);
+    const T b1 = s1 * s1 + (k * r1) * r1, b2 = s2 * s2 + (k * r2) * r2,
+            b3 = s3 * s3 + (k * r3) * r3;
     const T tau5 = fabs(b1 - b3);
     if constexpr (sizeof(T) == 4) {
       const T w1 = T(0.1) * (T(1) + tau5 * rcp(b1 + eps));
       const T w2 = T(0.6) * (T(1) + tau5 * rcp(b2 + eps));
       const T w3 = T(0.3) * (T(1) + tau5 * rcp(b3 + eps));
-      return (w1 * qi1 + w2 * qi2 + w3 * qi3) * rcp(w1 + w2 + w3);
+      return (w1 * p1 + w2 * p2 + w3 * p3) * rcp(w1 + w2 + w3);
     } else {
       const T t1 = b1 + eps, t2 = b2 + eps, t3 = b3 + eps;
-      return blend3(T(0.1) * (t1 + tau5), t1, qi1, T(0.6) * (t2 + tau5), t2, qi2,
-                    T(0.3) * (t3 + tau5), t3, qi3);
+      return blend3(T(0.1) * (t1 + tau5), t1, p1, T(0.6) * (t2 + tau5), t2, p2,
+                    T(0.3) * (t3 + tau5), t3, p3);
+    }
+  }
+}
+template <typename T, bool Z>
+__device__ __forceinline__ T weno5_upwind(T a, T b, T c, T d, T e) {
+  return c + weno5_delta<T, Z>(b - a, c - b, d - c, e - d);
+}
+// The 3-point schemes' face value less c, from d2 = c - b and d3 = d - c (also
+// odd).
+template <typename T, bool Z>
+__device__ __forceinline__ T weno3_delta(T d2, T d3) {
+  const T b1 = d2 * d2, b2 = d3 * d3;
+  if constexpr (!Z) {  // weno.py:297-320
+    const T t1 = b1 + T(1e-8), t2 = b2 + T(1e-8);
+    return T(0.5) * blend2(T(1.0 / 3.0), t1 * t1, d2, T(2.0 / 3.0), t2 * t2, d3);
+  } else {  // weno.py:323-347
+    const T t1 = b1 + T(1e-14), t2 = b2 + T(1e-14), tau = fabs(b2 - b1);
+    if constexpr (sizeof(T) == 4) {
+      const T w1 = T(1.0 / 3.0) * (T(1) + tau * rcp(t1)), w2 = T(2.0 / 3.0) * (T(1) + tau * rcp(t2));
+      return T(0.5) * ((w1 * d2 + w2 * d3) * rcp(w1 + w2));
+    } else {
+      return T(0.5) * blend2(T(1.0 / 3.0) * (t1 + tau), t1, d2, T(2.0 / 3.0) * (t2 + tau), t2, d3);
     }
   }
 }
@@ -243,6 +276,9 @@ template <typename T>
 struct StageCoef {
   const T* hn = nullptr;
   double a = 0.0, b = 0.0, cdt = 0.0;
+  // Periodic stages: the ghost width, and whether the output's ghosts are
+  // written too (advection_kernel).
+  int ng = 0, images = 0;
 };
 
 // Face value from the stencil mirrored to the upwind side of the face:
@@ -292,15 +328,53 @@ __device__ __forceinline__ T upwind_face(const T (&m)[5], bool near, int tier) {
   }
 }
 
+// WENO5 / WENO-Z5 flux through the face between values h0 and h1, from the
+// differences around it (dk between cells k and k + 1 of the face's cell 0):
+// the upwind cell's value plus or minus the oriented weno5_delta; the masked
+// tier dispatch as upwind_face.
+template <typename T, bool Z, bool MASKED>
+__device__ __forceinline__ T weno5_flux(T h0, T h1, T dm2, T dm1, T d0, T d1, T d2, T vel,
+                                        bool near, int tier) {
+  const bool pos = vel >= T(0);
+  const T a1 = pos ? dm2 : d2, a2 = pos ? dm1 : d1, a4 = pos ? d1 : dm1;
+  T sd = T(0);
+  if (!MASKED || tier == 6) {
+    if (near) sd = weno3_delta<T, Z>(a2, d0);
+    else sd = weno5_delta<T, Z>(a1, a2, d0, a4);
+  } else if (tier == 4) {
+    sd = weno3_delta<T, Z>(a2, d0);
+  }
+  const T f = ((pos ? h0 : h1) + (pos ? sd : -sd)) * vel;
+  return (!MASKED || tier >= 2) ? f : T(0);
+}
+
 // One wavefront per tile of 58 output columns (lanes 3..60; three halo lanes
-// each side) x kAdvRows rows.  Each lane keeps its column of h on rows
-// j0-3 .. j0+kAdvRows+2 in registers; the x stencils come from DPP lane
+// each side) x R rows.  Each lane keeps its column of h on rows
+// j0-3 .. j0+R+2 in registers; the x stencils come from DPP lane
 // shifts, the y stencils from neighbouring registers.  Each lane evaluates
 // the east face of its cell (the west face is the east face of the lane
 // beside it) and the north faces of its column, so every face flux is
 // reconstructed once; no LDS, no barriers, no integer division per cell.
 // Grids up to 512^2 take tiles of 2 rows: more wavefronts for the chip, a
 // shorter chain of loads and arithmetic per wavefront.
+//
+// Bound by issue slots (FP64 also by the FP64 pipe) and by the loads' latency,
+// so: differences instead of values (weno5_delta); every array of the tile
+// requested before the first flux (a stage's output may alias its h_n, so the
+// compiler does not move those loads up itself); and a tile away from every
+// edge (INNER: all but the outermost ring) runs without the clamps, zero
+// fills, fallbacks and ring tests of the others.  One Advection2D call, us,
+// before and now, FP64 / FP32 (the prefetch costs FP64 one wavefront in four a
+// SIMD, 3 instead of 4, and is still worth it):
+//   weno5 2048^2          48.5 -> 37.2 / 30.4 -> 23.5
+//   weno5 3000^2         114.5 -> 76.7 / 48.4 -> 40.6
+//   weno5 masked 3000^2  144.5 -> 106.9 / 66.4 -> 48.3
+//   van_leer 3000^2       65.3 -> 58.4 / 34.6 -> 32.7
+//
+// Periodic stages (ng > 0: the ghost width): h is read through the index map
+// of enforce_periodic (a ghost cell is its doubly wrapped interior cell), so
+// the caller fills no ghosts between stages; only interior cells are written,
+// with ``images`` also the ghost cells that copy them.
 constexpr int kAdvRows = 8, kAdvShortRows = 2, kAdvCols = 58;
 constexpr int64_t kAdvShortMaxCells = 514 * 514;
 
@@ -312,82 +386,172 @@ template <typename T>
 __device__ __forceinline__ T adv_w(T v) {
   return dpp_move<0x138>(v);  // wave_shr 1: value of lane - 1, 0 in lane 0
 }
+// Index of the cell that cell k of n holds after the periodic fill.
+__device__ __forceinline__ int adv_wrap(int k, int n, int ng) {
+  return k < ng ? k + (n - 2 * ng) : (k >= n - ng ? k - (n - 2 * ng) : k);
+}
 
-template <typename T, int M, int L, bool MASKED, int R>
-__global__ __launch_bounds__(256) void advection_kernel(
-    const T* __restrict__ h, const T* __restrict__ u, const T* __restrict__ v,
-    T* out, const uint8_t* __restrict__ tier_x, const uint8_t* __restrict__ tier_y,
-    const uint8_t* __restrict__ mh, int ny, int nx, T idx, T idy, int tiles_x, int ntiles,
-    const T* hn, T ca, T cb, T ccdt) {
+template <typename T>
+struct AdvArgs {
+  const T *h, *u, *v;
+  T* out;
+  const uint8_t *tier_x, *tier_y, *mh;
+  int ny, nx;
+  T idx, idy;
+  int tiles_x, ntiles;
+  const T* hn;
+  T ca, cb, ccdt;
+  int ng, images;
+};
+
+// INNER: every cell, face and stencil of the tile lies inside the array, away
+// from the edge fallbacks, the output ring and the periodic ghosts and images.
+template <typename T, int M, int L, bool MASKED, int R, bool INNER>
+__device__ __forceinline__ void advection_tile(const AdvArgs<T>& a, int i0, int j0, int lane) {
   constexpr int HR = R + 6;
-  const int lane = threadIdx.x & 63;
-  const int tile =
-      __builtin_amdgcn_readfirstlane(xcd_swizzle(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6));
-  if (tile >= ntiles) return;  // whole wavefront (no block-level barrier below)
-  const int tyi = tile / tiles_x;
-  const int i0 = (tile - tyi * tiles_x) * kAdvCols, j0 = tyi * R;
+  constexpr bool W5 = M == kWeno5 || M == kWenoZ5, Z = M == kWenoZ5;
+  const int ny = a.ny, nx = a.nx, ng = INNER ? 0 : a.ng;
   const int gi = i0 - 3 + lane;
-  const bool colin = gi >= 0 && gi < nx;
-  const int64_t gic = min(max(gi, 0), nx - 1);
-  // h on rows j0-3+r (zero outside the array)
-  T hr[HR];
+  const bool colin = INNER || (gi >= 0 && gi < nx);
+  const unsigned gic = INNER ? (unsigned)gi : (unsigned)min(max(gi, 0), nx - 1);
+  const unsigned gih = (unsigned)(ng > 0 ? adv_wrap((int)gic, nx, ng) : (int)gic);
+  auto row = [&](int gj) -> int64_t {
+    return (int64_t)(INNER ? gj : min(max(gj, 0), ny - 1)) * nx;
+  };
+  // h on rows j0-3+r (zero outside the array), v on rows j0-1 .. j0+R-1 (the
+  // faces between rows j0-1+t and j0+t), u on the output rows
+  T hr[HR], vr[R + 1], ur[R], hs[R];
+  int tyr[MASKED ? R + 2 : 1], txr[MASKED ? R : 1], mr[R];
 #pragma unroll
   for (int r = 0; r < HR; ++r) {
-    const int gj = j0 - 3 + r;
-    const int64_t gjc = min(max(gj, 0), ny - 1);
-    const T x = h[gjc * nx + gic];
-    hr[r] = (colin && gj >= 0 && gj < ny) ? x : T(0);
+    if constexpr (INNER) {
+      hr[r] = (a.h + row(j0 - 3 + r))[gih];
+    } else {
+      const int gj = min(max(j0 - 3 + r, 0), ny - 1);
+      hr[r] = (a.h + (int64_t)(ng > 0 ? adv_wrap(gj, ny, ng) : gj) * nx)[gih];
+    }
+  }
+#pragma unroll
+  for (int t = 0; t <= R; ++t) vr[t] = (a.v + row(j0 - 1 + t))[gic];
+#pragma unroll
+  for (int t = 0; t < R; ++t) ur[t] = (a.u + row(j0 + t))[gic];
+  if constexpr (MASKED) {
+#pragma unroll
+    for (int t = 0; t < R + 2; ++t) tyr[t] = (a.tier_y + row(j0 - 1 + t))[gic];
+#pragma unroll
+    for (int t = 0; t < R; ++t) txr[t] = (a.tier_x + row(j0 + t))[gic];
+  }
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    mr[t] = a.mh ? (a.mh + row(j0 + t))[gic] : 1;
+    hs[t] = a.hn ? (a.hn + row(j0 + t))[gic] : T(0);
+  }
+  if constexpr (!INNER) {
+#pragma unroll
+    for (int r = 0; r < HR; ++r) {
+      const int gj = j0 - 3 + r;
+      if (!colin || gj < 0 || gj >= ny) hr[r] = T(0);
+    }
+  }
+  // (W5) differences of neighbouring rows, shared by the faces around them
+  T dy_[W5 ? HR - 1 : 1];
+  if constexpr (W5) {
+#pragma unroll
+    for (int r = 0; r < HR - 1; ++r) dy_[r] = hr[r + 1] - hr[r];
   }
   // North faces fj = j0-1+t (between rows j0-1+t and j0+t), t = 0 .. R.
   T fn[R + 1];
 #pragma unroll
   for (int t = 0; t <= R; ++t) {
     const int r = t + 2, fj = j0 - 1 + t;
-    const int64_t fjc = min(max(fj, 0), ny - 1);
-    const int64_t c = fjc * nx + gic;
-    const T vel = v[c];
+    const T vel = vr[t];
     const bool pos = vel >= T(0);
-    const T m[5] = {pos ? hr[r - 2] : hr[r + 3], pos ? hr[r - 1] : hr[r + 2],
-                    pos ? hr[r] : hr[r + 1], pos ? hr[r + 1] : hr[r],
-                    pos ? hr[r + 2] : hr[r - 1]};
     int tier = 0;
-    if constexpr (MASKED) tier = pos ? tier_y[c] : tier_y[min(fjc + 1, (int64_t)ny - 1) * nx + gic];
-    const bool valid = colin && gi >= 2 && gi <= nx - 3 && fj >= 1 && fj <= ny - 3;
-    const T f = upwind_face<T, M, L, MASKED>(m, pos ? fj == 1 : fj == ny - 3, tier) * vel;
-    fn[t] = valid ? f : T(0);
+    if constexpr (MASKED) {
+      tier = pos ? tyr[t] : tyr[t + 1];
+    }
+    const bool near = !INNER && (pos ? fj == 1 : fj == ny - 3);
+    T f;
+    if constexpr (W5) {
+      f = weno5_flux<T, Z, MASKED>(hr[r], hr[r + 1], dy_[r - 2], dy_[r - 1], dy_[r], dy_[r + 1],
+                                   dy_[r + 2], vel, near, tier);
+    } else {
+      const T m[5] = {pos ? hr[r - 2] : hr[r + 3], pos ? hr[r - 1] : hr[r + 2],
+                      pos ? hr[r] : hr[r + 1], pos ? hr[r + 1] : hr[r],
+                      pos ? hr[r + 2] : hr[r - 1]};
+      f = upwind_face<T, M, L, MASKED>(m, near, tier) * vel;
+    }
+    fn[t] = INNER || (colin && gi >= 2 && gi <= nx - 3 && fj >= 1 && fj <= ny - 3) ? f : T(0);
   }
-  const bool lout = colin && lane >= 3 && lane <= 60;
+  const bool lout = colin && lane >= 3 && lane <= 60 && (ng == 0 || (gi >= ng && gi < nx - ng));
 #pragma unroll
   for (int t = 0; t < R; ++t) {
     const int r = t + 3, gj = j0 + t;
-    const int64_t gjc = min(gj, ny - 1);
-    const int64_t c = gjc * nx + gic;
     // East face fi = gi of this row (between columns gi and gi+1).
     const T hc = hr[r];
-    const T e1 = adv_e(hc), e2 = adv_e(e1), e3 = adv_e(e2);
-    const T w1 = adv_w(hc), w2 = adv_w(w1);
-    const T vel = u[c];
+    const T e1 = adv_e(hc);
+    const T vel = ur[t];
     const bool pos = vel >= T(0);
-    const T m[5] = {pos ? w2 : e3, pos ? w1 : e2, pos ? hc : e1, pos ? e1 : hc, pos ? e2 : w1};
     int tier = 0;
     if constexpr (MASKED) {
-      const int tx = tier_x[c];
-      const int txe = __builtin_amdgcn_mov_dpp(tx, 0x130, 0xf, 0xf, true);  // lane + 1
-      tier = pos ? tx : txe;
+      const int txe = __builtin_amdgcn_mov_dpp(txr[t], 0x130, 0xf, 0xf, true);  // lane + 1
+      tier = pos ? txr[t] : txe;
     }
-    const bool valid = colin && gj >= 2 && gj <= ny - 3 && gi >= 1 && gi <= nx - 3;
-    const T fe0 = upwind_face<T, M, L, MASKED>(m, pos ? gi == 1 : gi == nx - 3, tier) * vel;
-    const T fe = valid ? fe0 : T(0);
+    const bool near = !INNER && (pos ? gi == 1 : gi == nx - 3);
+    T fe;
+    if constexpr (W5) {
+      const T d0 = e1 - hc, dm1 = adv_w(d0), dm2 = adv_w(dm1), d1 = adv_e(d0), d2 = adv_e(d1);
+      fe = weno5_flux<T, Z, MASKED>(hc, e1, dm2, dm1, d0, d1, d2, vel, near, tier);
+    } else {
+      const T e2 = adv_e(e1), e3 = adv_e(e2), w1 = adv_w(hc), w2 = adv_w(w1);
+      const T m[5] = {pos ? w2 : e3, pos ? w1 : e2, pos ? hc : e1, pos ? e1 : hc, pos ? e2 : w1};
+      fe = upwind_face<T, M, L, MASKED>(m, near, tier) * vel;
+    }
+    if constexpr (!INNER)
+      fe = colin && gj >= 2 && gj <= ny - 3 && gi >= 1 && gi <= nx - 3 ? fe : T(0);
     const T fw = adv_w(fe);
-    if (lout && gj < ny) {
+    if (lout && (INNER || (gj < ny && (ng == 0 || (gj >= ng && gj < ny - ng))))) {
       T res = T(0);
-      if (gj >= 2 && gj <= ny - 3 && gi >= 2 && gi <= nx - 3)
-        res = -((fe - fw) * idx + (fn[t + 1] - fn[t]) * idy);
-      if (mh) res = res * (T)(mh[c] ? 1 : 0);
-      if (hn) res = ca * hn[c] + cb * hc + ccdt * res;
-      out[c] = res;
+      if (INNER || (gj >= 2 && gj <= ny - 3 && gi >= 2 && gi <= nx - 3))
+        res = -((fe - fw) * a.idx + (fn[t + 1] - fn[t]) * a.idy);
+      if (a.mh) res = res * (T)(mr[t] ? 1 : 0);
+      if (a.hn) res = a.ca * hs[t] + a.cb * hc + a.ccdt * res;
+      T* o = a.out + (int64_t)gj * nx;
+      o[gi] = res;
+      if (!INNER && a.images) {  // the ghost cells this cell fills
+        const int pi = nx - 2 * ng, pj = ny - 2 * ng;
+        const bool xe = gi < 2 * ng, xw = gi >= nx - 2 * ng;  // image east / west
+        if (xe) o[gi + pi] = res;
+        if (xw) o[gi - pi] = res;
+        if (gj < 2 * ng) {
+          T* q = o + (int64_t)pj * nx;
+          q[gi] = res;
+          if (xe) q[gi + pi] = res;
+          if (xw) q[gi - pi] = res;
+        }
+        if (gj >= ny - 2 * ng) {
+          T* q = o - (int64_t)pj * nx;
+          q[gi] = res;
+          if (xe) q[gi + pi] = res;
+          if (xw) q[gi - pi] = res;
+        }
+      }
     }
   }
+}
+
+template <typename T, int M, int L, bool MASKED, int R>
+__global__ __launch_bounds__(256) void advection_kernel(AdvArgs<T> a) {
+  const int lane = threadIdx.x & 63;
+  const int tile =
+      __builtin_amdgcn_readfirstlane(xcd_swizzle(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6));
+  if (tile >= a.ntiles) return;  // whole wavefront (no block-level barrier below)
+  const int tyi = tile / a.tiles_x;
+  const int i0 = (tile - tyi * a.tiles_x) * kAdvCols, j0 = tyi * R;
+  const int mg = 2 * a.ng;
+  const bool inner = i0 - 3 >= mg && i0 + 61 <= a.nx - mg && j0 - 3 >= mg && j0 + R + 3 <= a.ny - mg;
+  if (inner) advection_tile<T, M, L, MASKED, R, true>(a, i0, j0, lane);
+  else advection_tile<T, M, L, MASKED, R, false>(a, i0, j0, lane);
 }
 
 template <typename T, int M, int L, bool MASKED>
@@ -398,14 +562,13 @@ static void launch_adv(const T* h, const T* u, const T* v, T* out, const uint8_t
   const int rows = short_tiles ? kAdvShortRows : kAdvRows;
   const int tiles_x = cdiv(nx, kAdvCols), tiles_y = cdiv(ny, rows);
   const int ntiles = tiles_x * tiles_y;
+  const AdvArgs<T> a{h,  u,  v,  out, tx_, ty_, mh, ny, nx, (T)(1.0 / dx), (T)(1.0 / dy), tiles_x,
+                     ntiles, sc.hn, (T)sc.a, (T)sc.b, (T)sc.cdt, sc.ng, sc.images};
+  const dim3 grid(cdiv(ntiles, 4)), block(256);
   if (short_tiles)
-    hipLaunchKernelGGL((advection_kernel<T, M, L, MASKED, kAdvShortRows>), dim3(cdiv(ntiles, 4)),
-                       dim3(256), 0, s, h, u, v, out, tx_, ty_, mh, ny, nx, (T)(1.0 / dx),
-                       (T)(1.0 / dy), tiles_x, ntiles, sc.hn, (T)sc.a, (T)sc.b, (T)sc.cdt);
+    hipLaunchKernelGGL((advection_kernel<T, M, L, MASKED, kAdvShortRows>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((advection_kernel<T, M, L, MASKED, kAdvRows>), dim3(cdiv(ntiles, 4)),
-                       dim3(256), 0, s, h, u, v, out, tx_, ty_, mh, ny, nx, (T)(1.0 / dx),
-                       (T)(1.0 / dy), tiles_x, ntiles, sc.hn, (T)sc.a, (T)sc.b, (T)sc.cdt);
+    hipLaunchKernelGGL((advection_kernel<T, M, L, MASKED, kAdvRows>), grid, block, 0, s, a);
 }
 
 template <typename T, bool MASKED>
@@ -586,24 +749,13 @@ int face_flux_call(int method, int lim, int dir, const T* h, const T* vel, T* ou
 // One rk3_ssp_step (timestepping/explicit_rk.py:74-121) of a doubly periodic
 // tracer: per stage the periodic ghost fill of width ng (boundary.py:52-78,
 // as the periodic advection tests do before each tendency) and the
-// Advection2D tendency with the Shu-Osher combination fused into its launch;
-// h advances in place and leaves with its ghosts filled.  Scratch: the two
-// stage states y1, y2.
+// Advection2D tendency with the Shu-Osher combination, in one launch each:
+// the stages read their input through the fill's index map, and the last one
+// writes the result's ghosts.  Scratch: the two stage states y1, y2 (interior
+// only).  Per step, FP64 WENO5: 38.7 us with the fills as launches of their own,
+// now 24.3 at 256^2 (the host's time per call; the three kernels take 16 us);
+// 83 -> 47 at 1000^2, 104 -> 72 at 1500^2.
 // ---------------------------------------------------------------------------
-
-}  // namespace fvx
-
-extern "C" int fvx_enforce_periodic_f32(float*, int, int, int, void*);
-extern "C" int fvx_enforce_periodic_f64(double*, int, int, int, void*);
-
-namespace fvx {
-
-static int periodic(float* f, int ny, int nx, int ng, hipStream_t s) {
-  return fvx_enforce_periodic_f32(f, ny, nx, ng, s);
-}
-static int periodic(double* f, int ny, int nx, int ng, hipStream_t s) {
-  return fvx_enforce_periodic_f64(f, ny, nx, ng, s);
-}
 
 // Argument checks shared by both entry points (no device work).
 template <typename T>
@@ -617,31 +769,30 @@ static int adv_rk3_check(const T* h, const T* u, const T* v, int ny, int nx, int
   return kOk;
 }
 
+// h -> res (which may be h).
 template <typename T>
-static int adv_rk3_enqueue(int method, int lim, T* h, const T* u, const T* v,
+static int adv_rk3_enqueue(int method, int lim, const T* h, T* res, const T* u, const T* v,
                            const uint8_t* tier_x, const uint8_t* tier_y, const uint8_t* mh,
                            int ny, int nx, int ng, double dx, double dy, double dt, T* y1, T* y2,
                            hipStream_t s) {
   // Each stage is one advection launch with the Shu-Osher combination fused
-  // (out = a h + b q + cdt L(q) on every cell, q the stage's input).
-  auto stage = [&](const T* q, T* out, double a, double b, double cdt) {
+  // (out = a h + b q + cdt L(q) on every interior cell, q the stage's input).
+  auto stage = [&](const T* q, T* out, double a, double b, double cdt, int images) {
     StageCoef<T> sc;
     sc.hn = h;
     sc.a = a;
     sc.b = b;
     sc.cdt = cdt;
+    sc.ng = ng;
+    sc.images = images;
     return advection<T>(method, lim, q, u, v, out, tier_x, tier_y, mh, ny, nx, dx, dy, s, sc);
   };
-  int rc;
-  // y1 = h + dt L(h)
-  if ((rc = periodic(h, ny, nx, ng, s)) || (rc = stage(h, y1, 0.0, 1.0, dt))) return rc;
-  // y2 = 3/4 h + 1/4 y1 + 1/4 dt L(y1)
-  if ((rc = periodic(y1, ny, nx, ng, s)) || (rc = stage(y1, y2, 0.75, 0.25, 0.25 * dt))) return rc;
-  // h = 1/3 h + 2/3 y2 + 2/3 dt L(y2) (the output may alias h: read per cell)
-  if ((rc = periodic(y2, ny, nx, ng, s)) ||
-      (rc = stage(y2, h, 1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0 * dt)))
-    return rc;
-  return periodic(h, ny, nx, ng, s);
+  // y1 = h + dt L(h), y2 = 3/4 h + 1/4 y1 + 1/4 dt L(y1),
+  // 1/3 h + 2/3 y2 + 2/3 dt L(y2) (the output may alias h: an interior cell is
+  // read by the lane that writes it, a ghost cell is not read)
+  if (int rc = stage(h, y1, 0.0, 1.0, dt, 0)) return rc;
+  if (int rc = stage(y1, y2, 0.75, 0.25, 0.25 * dt, 0)) return rc;
+  return stage(y2, res, 1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0 * dt, 1);
 }
 
 // Stage arrays of the allocating entry point: one buffer per device, grown
@@ -673,7 +824,7 @@ static int adv_rk3_step(int method, int lim, T* h, const T* u, const T* v,
     }
     buf = (T*)g_stage_buf[dev];
   }
-  return adv_rk3_enqueue<T>(method, lim, h, u, v, tier_x, tier_y, mh, ny, nx, ng, dx, dy, dt,
+  return adv_rk3_enqueue<T>(method, lim, h, h, u, v, tier_x, tier_y, mh, ny, nx, ng, dx, dy, dt,
                             buf, buf + (size_t)ny * nx, s);
 }
 
@@ -720,7 +871,7 @@ static int adv_rk3_step_noalloc(int method, int lim, T* h, const T* u, const T* 
   void* p = nullptr;
   if (int rc = scratch_ptr(&p)) return rc;
   T* y1 = (T*)p;
-  return adv_rk3_enqueue<T>(method, lim, h, u, v, tier_x, tier_y, mh, ny, nx, ng, dx, dy, dt, y1,
+  return adv_rk3_enqueue<T>(method, lim, h, h, u, v, tier_x, tier_y, mh, ny, nx, ng, dx, dy, dt, y1,
                             y1 + (size_t)ny * nx, s);
 }
 
@@ -746,6 +897,25 @@ extern "C" {
 FVX_ADV_RK3(f32, float)
 FVX_ADV_RK3(f64, double)
 #undef FVX_ADV_RK3
+
+// The step from h into out (another array), with the caller's scratch of
+// 2 ny nx elements: no allocation, no array shared with other calls.
+#define FVX_ADV_RK3_INTO(SUF, T)                                                                 \
+  int fvx_advection_rk3_step_into_##SUF(int method, int limiter, const T* h, T* out, const T* u, \
+                                        const T* v, const uint8_t* tier_x,                       \
+                                        const uint8_t* tier_y, const uint8_t* mask_h, int ny,    \
+                                        int nx, int ng, double dx, double dy, double dt,         \
+                                        T* work, void* stream) {                                 \
+    if (int rc = fvx::adv_rk3_check<T>(h, u, v, ny, nx, ng, dx, dy, dt)) return rc;              \
+    FVX_CHECK_ARG(out && work, "null field pointer");                                            \
+    FVX_CHECK_ARG(out != h, "out must not alias h");                                             \
+    return fvx::adv_rk3_enqueue<T>(method, limiter, h, out, u, v, tier_x, tier_y, mask_h, ny,    \
+                                   nx, ng, dx, dy, dt, work, work + (size_t)ny * nx,             \
+                                   (hipStream_t)stream);                                         \
+  }
+FVX_ADV_RK3_INTO(f32, float)
+FVX_ADV_RK3_INTO(f64, double)
+#undef FVX_ADV_RK3_INTO
 
 int fvx_face_flux_f64(int method, int limiter, int dir, const double* h, const double* vel,
                       double* out, const uint8_t* tier, int ny, int nx, void* stream) {

@@ -105,6 +105,19 @@ int fvx_advection_rk3_step_noalloc_f64(int method, int limiter, double* h, const
                                        const uint8_t* tier_y, const uint8_t* mask_h, int ny,
                                        int nx, int ng, double dx, double dy, double dt,
                                        void* stream);
+/* The same step from h into out (another array, every cell written), with
+ * the caller's device scratch of 2 ny nx elements: it allocates nothing and
+ * shares no array with other calls. */
+int fvx_advection_rk3_step_into_f32(int method, int limiter, const float* h, float* out,
+                                    const float* u, const float* v, const uint8_t* tier_x,
+                                    const uint8_t* tier_y, const uint8_t* mask_h, int ny, int nx,
+                                    int ng, double dx, double dy, double dt, float* work,
+                                    void* stream);
+int fvx_advection_rk3_step_into_f64(int method, int limiter, const double* h, double* out,
+                                    const double* u, const double* v, const uint8_t* tier_x,
+                                    const uint8_t* tier_y, const uint8_t* mask_h, int ny, int nx,
+                                    int ng, double dx, double dy, double dt, double* work,
+                                    void* stream);
 
 /* ---- One Runge-Kutta stage of a tracer with an Advection2D tendency ---------
  * out = a hn + b hs + cdt L(hs), L the Advection2D.__call__ tendency

@@ -71,6 +71,31 @@ def test_periodic_step_methods(method):
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
+@pytest.mark.parametrize("ny,nx,ng,method,masked", [
+    (5, 6, 1, "weno5", False), (6, 9, 2, "wenoz5", False),   # ghosts reach their own images
+    (9, 9, 3, "van_leer", False), (23, 61, 1, "weno5", True),
+    (75, 133, 4, "wenoz5", False),      # 2-row tiles, three tile columns, odd rows
+    (521, 523, 3, "weno5", False),      # 8-row tiles, inner and edge tiles
+    (523, 641, 2, "van_leer", True)])
+def test_periodic_step_at_tile_and_ghost_edges(ny, nx, ng, method, masked, dtype, tol):
+    need_gpu()
+    rng = np.random.default_rng(ny * nx + ng)
+    h = 1.0 + 0.5 * rng.standard_normal((ny, nx))  # the ghosts of h hold anything
+    u, v = 0.7 * rng.standard_normal((2, ny, nx))
+    wet = random_mask(ny, nx, 5) if masked else None
+    ref = _oracle_step(h, u, v, 0.3, 0.4, 0.02, method, ng,
+                       fvx.Mask2D(wet) if masked else None)
+    g = fx.CartesianGrid2D(Nx=nx, Ny=ny, Lx=0.3 * (nx - 2), Ly=0.4 * (ny - 2), dx=0.3, dy=0.4)
+    adv = fx.Advection2D(g, fx.Mask2D(wet) if masked else None)
+    ht = torch.tensor(h, dtype=dtype, device="cuda")
+    h0 = ht.clone()
+    got = adv.rk3_step(ht, torch.tensor(u, dtype=dtype), torch.tensor(v, dtype=dtype), 0.02,
+                       method, ng=ng)
+    assert torch.equal(ht, h0)
+    assert_close_scaled(to_np(got), ref, tol, f"{method} {ny}x{nx} ng {ng}")
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
 def test_masked_weno5_fp32_and_fp64(dtype, tol):
     """Masked tier dispatch (the 3-layer configuration's tracer is a masked
     FP32 WENO5 field) against the oracle, both precisions."""
