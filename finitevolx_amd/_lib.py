@@ -107,18 +107,31 @@ def require_gpu() -> torch.device:
 
 
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current device's current stream.  (Without a Stream object
+    in between: 0.4 us instead of 2.8, of the 15 us of host work that an
+    operator call took; 8.5 with as_field's short way.)"""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+_FIELD_DTYPES = (torch.float32, torch.float64)
 
 
 def as_field(x, dtype=None) -> torch.Tensor:
     """Return ``x`` as a contiguous float32/float64 CUDA tensor."""
+    # What the conversions below would hand back as it is: a plain tensor of the
+    # wanted type, contiguous, on the current device (0.5 us instead of 1.9; a
+    # call takes up to four).
+    if type(x) is torch.Tensor and x.is_cuda and x.dtype in _FIELD_DTYPES \
+            and (dtype is None or dtype == x.dtype) and x.is_contiguous() \
+            and x.get_device() == torch.cuda.current_device():
+        return x
     dev = require_gpu()
     if isinstance(x, torch.Tensor):
         t = x
     else:
         t = torch.from_numpy(np.ascontiguousarray(np.asarray(x)))
     if dtype is None:
-        dtype = t.dtype if t.dtype in (torch.float32, torch.float64) else torch.float64
+        dtype = t.dtype if t.dtype in _FIELD_DTYPES else torch.float64
     return t.to(device=dev, dtype=dtype).contiguous()
 
 

@@ -753,7 +753,7 @@ int face_flux_call(int method, int lim, int dir, const T* h, const T* vel, T* ou
 // the stages read their input through the fill's index map, and the last one
 // writes the result's ghosts.  Scratch: the two stage states y1, y2 (interior
 // only).  Per step, FP64 WENO5: 38.7 us with the fills as launches of their own,
-// now 24.3 at 256^2 (the host's time per call; the three kernels take 16 us);
+// now 17.1 at 256^2 (the three kernels take 16);
 // 83 -> 47 at 1000^2, 104 -> 72 at 1500^2.
 // ---------------------------------------------------------------------------
 

@@ -236,3 +236,25 @@ def test_momentum_advection_schemes(scheme, masked):
         assert_close_scaled(to_np(dv), ref[1], tol, f"dv {scheme} {dtype}")
     with pytest.raises(ValueError):
         madv(torch.tensor(u), torch.tensor(v), "bogus")
+
+
+@pytest.mark.parametrize("make", [
+    lambda x: x, lambda x: x.float(), lambda x: x.t(), lambda x: x[::2, 1:], lambda x: x[1:],
+    lambda x: x.cpu(), lambda x: x.half(), lambda x: (x * 8).long(), lambda x: x.cpu().numpy(),
+    lambda x: torch.nn.Parameter(x)])
+@pytest.mark.parametrize("dtype", [None, torch.float32, torch.float64])
+def test_field_arguments_of_every_kind(make, dtype):
+    """A field argument arrives as the contiguous array of its values on the
+    GPU, whatever it was; the stream handle follows torch's current stream."""
+    need_gpu()
+    from finitevolx_amd import _lib
+    x = make(torch.randn(12, 10, dtype=torch.float64, device="cuda"))
+    t = torch.as_tensor(x)
+    got = _lib.as_field(x, dtype)
+    want = dtype or (t.dtype if t.dtype in (torch.float32, torch.float64) else torch.float64)
+    assert got.dtype == want and got.is_contiguous() and got.device == torch.device("cuda", 0)
+    assert torch.equal(got.cpu(), t.detach().cpu().to(want))
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        assert _lib.stream() == s.cuda_stream
+    assert _lib.stream() == torch.cuda.current_stream().cuda_stream
