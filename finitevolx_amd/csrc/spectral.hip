@@ -223,6 +223,7 @@ struct SpecGemm {
   const double *et, *eo;
   double ct, co, scale;
   int divide, halve0;  // halve0: the DCT's k = 0 weight along each axis
+  int ring;            // (last product) zero the one-cell ring around the output
   double lam[kSpecBatch];
 };
 
@@ -234,6 +235,25 @@ struct SpecGemm {
 // chains on every CU: 3 x 512 x 768 takes 143 us a solve (151 with the chunked
 // sums), 156 with tiles of 64, 167 with four groups.
 constexpr int kSpecThreads = 512;
+// The cells of the one-cell zero ring that lie next to cell (j, i) of the
+// ny x nx array at out.
+template <typename T>
+__device__ __forceinline__ void ring_around(T* out, int64_t ld, int j, int i, int ny, int nx) {
+  T* p = out + (int64_t)j * ld + i;
+  const bool w = i == 0, e = i == nx - 1;
+  if (w) p[-1] = T(0);
+  if (e) p[1] = T(0);
+  if (j == 0) {
+    p[-ld] = T(0);
+    if (w) p[-ld - 1] = T(0);
+    if (e) p[-ld + 1] = T(0);
+  }
+  if (j == ny - 1) {
+    p[ld] = T(0);
+    if (w) p[ld - 1] = T(0);
+    if (e) p[ld + 1] = T(0);
+  }
+}
 template <typename T, bool LEFT, bool INV>
 __global__ __launch_bounds__(kSpecThreads) void spec_gemm_kernel(SpecGemm<T> g) {
   constexpr int BT = 32, BK = 64, P = BT + 2, PER = BT * BK / kSpecThreads;
@@ -369,6 +389,9 @@ __global__ __launch_bounds__(kSpecThreads) void spec_gemm_kernel(SpecGemm<T> g) 
     if (t >= nt || o >= g.other) continue;
     auto put_at = [&](int q, double v) {
       out[LEFT ? (int64_t)q * g.ld_out + o : (int64_t)o * g.ld_out + q] = (T)v;
+      if constexpr (INV && !LEFT) {
+        if (g.ring) ring_around(out, g.ld_out, o, q, g.other, g.n);
+      }
     };
     if constexpr (INV) {
       const double e = acc[0][i], d = acc[NC - 1][i];
@@ -532,6 +555,19 @@ __global__ void copy_pitched_kernel(const T* __restrict__ src, int64_t lds, T* _
   if (i < nx && j < ny) dst[(int64_t)j * ldd + i] = src[(int64_t)j * lds + i];
 }
 
+template <typename T>
+__global__ void ring_kernel(T* out, int64_t ld, int ny, int nx) {
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k < nx) {
+    ring_around(out, ld, 0, k, ny, nx);
+    ring_around(out, ld, ny - 1, k, ny, nx);
+  }
+  if (k < ny) {
+    ring_around(out, ld, k, 0, ny, nx);
+    ring_around(out, ld, k, nx - 1, ny, nx);
+  }
+}
+
 template <typename T, bool LEFT, bool INV>
 static int launch_spec(const SpecGemm<T>& g, int nb, hipStream_t s) {
   const dim3 grid(cdiv(g.other, 32), INV ? cdiv(g.h, 32) : cdiv(g.n0, 32) + cdiv(g.n1, 32), nb);
@@ -545,7 +581,7 @@ static int launch_spec(const SpecGemm<T>& g, int nb, hipStream_t s) {
 template <typename T>
 static int gemm_solve(SpecPlan* P, const T* rhs, int64_t ld_rhs, int64_t bs_rhs, T* out,
                       int64_t ld_out, int64_t bs_out, int nb, const double* lam, double dx,
-                      double dy, T* work, hipStream_t s) {
+                      double dy, T* work, hipStream_t s, bool ring = false) {
   const int ny = P->ny, nx = P->nx;
   const int64_t N = (int64_t)ny * nx;
   for (int b0 = 0; b0 < nb; b0 += kSpecBatch) {
@@ -588,6 +624,7 @@ static int gemm_solve(SpecPlan* P, const T* rhs, int64_t ld_rhs, int64_t bs_rhs,
     if (int rc = launch_spec<T, true, true>(g, m, s)) return rc;
     axis(P->ax, ny);
     arrays(A, nx, N, out + b0 * bs_out, ld_out, bs_out);
+    g.ring = ring;
     if (int rc = launch_spec<T, false, true>(g, m, s)) return rc;
   }
   return kOk;
@@ -732,4 +769,33 @@ int fvx_spectral_helmholtz_f32(void* plan, const float* rhs, int64_t ld_rhs, flo
 FVX_SPEC_BATCH(f64, double, 64)
 FVX_SPEC_BATCH(f32, float, 32)
 #undef FVX_SPEC_BATCH
+
+// One solve on the interior of full (ny + 2, nx + 2) fields: out's one-cell
+// ring is written zero, rhs' ring is not read.  work as in the batched solve.
+#define FVX_SPEC_FIELD(SUF, T, PREC)                                                             \
+  int fvx_spectral_helmholtz_field_##SUF(void* plan, const T* rhs, T* out, double dx, double dy, \
+                                         double lambda_, T* work, void* stream) {                \
+    using namespace fvx;                                                                         \
+    FVX_CHECK_ARG(plan && rhs && out, "null argument");                                          \
+    FVX_CHECK_ARG(rhs != out, "out must be another array");                                      \
+    SpecPlan* P = (SpecPlan*)plan;                                                               \
+    FVX_CHECK_ARG(P->prec == PREC, "plan was built for the other precision");                    \
+    FVX_CHECK_ARG(dx > 0 && dy > 0, "grid spacing must be positive");                            \
+    const int64_t ld = P->nx + 2;                                                                \
+    hipStream_t s = (hipStream_t)stream;                                                         \
+    if (P->gemm) {                                                                               \
+      FVX_CHECK_ARG(work, "null work array");                                                    \
+      return gemm_solve<T>(P, rhs + ld + 1, ld, 0, out + ld + 1, ld, 0, 1, &lambda_, dx, dy,     \
+                           work, s, true);                                                       \
+    }                                                                                            \
+    if (int rc = spec_solve<T>(P, rhs + ld + 1, ld, out + ld + 1, ld, dx, dy, lambda_, s))       \
+      return rc;                                                                                 \
+    hipLaunchKernelGGL(ring_kernel<T>, dim3(cdiv(std::max(P->ny, P->nx), 256)), dim3(256), 0, s, \
+                       out + ld + 1, ld, P->ny, P->nx);                                          \
+    FVX_LAUNCH_CHECK();                                                                          \
+    return kOk;                                                                                  \
+  }
+FVX_SPEC_FIELD(f64, double, 64)
+FVX_SPEC_FIELD(f32, float, 32)
+#undef FVX_SPEC_FIELD
 }

@@ -393,6 +393,88 @@ int enforce_periodic(T* f, int ny, int nx, int ng, hipStream_t s) {
   return kOk;
 }
 
+// ---------------------------------------------------------------------------
+// The double-gyre example's tendency (scripts/qg_1p5_layer.py:454-478) and
+// velocities (:115-145) in one pass, with the fields' composition of the
+// operators above: X = T_to_X(psi), u = -diff_y_X_to_U(X), v = diff_x_X_to_V(X),
+//   rhs = advection(q; upwind1) - beta V_to_T(v) + wind
+//         - drag laplacian(psi) + viscosity laplacian(q)
+// (every operator's ghost ring zero, the advection's two cells wide; wind on
+// every cell).  One thread a cell: the velocities around the cell take the nine
+// psi values around it, so nothing is exchanged.  Why: as the eight operator
+// calls it was one short launch each, all bound by the host's time per call
+// (64^2 step: 382 us so, 158 with this kernel and the inversion from field to
+// field).  q null: velocities only.
+// ---------------------------------------------------------------------------
+template <typename T>
+struct GyreArgs {
+  const T *q, *psi, *wind;
+  T *rhs, *u, *v;
+  int ny, nx;
+  T idx, idy, beta, drag, visc;
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void gyre_kernel(GyreArgs<T> g) {
+  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+  const int ny = g.ny, nx = g.nx;
+  if (i >= nx || j >= ny) return;
+  const int64_t c = (int64_t)j * nx + i;
+  const bool in = j >= 1 && j <= ny - 2 && i >= 1 && i <= nx - 2;
+  T u0 = T(0), v0 = T(0), rhs = T(0);
+  if (in) {
+    T p[3][3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) p[b][a] = g.psi[c + (int64_t)(b - 1) * nx + (a - 1)];
+    // X[b][a] at (j - 1 + b, i - 1 + a), zero on the ring
+    T X[2][2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+        X[b][a] = j - 1 + b >= 1 && i - 1 + a >= 1
+                      ? T(0.25) * (p[b][a] + p[b][a + 1] + p[b + 1][a] + p[b + 1][a + 1])
+                      : T(0);
+    u0 = -((X[1][1] - X[0][1]) * g.idy);
+    v0 = (X[1][1] - X[1][0]) * g.idx;
+    if (g.q) {
+      const T uw = -((X[1][0] - X[0][0]) * g.idy), vs = (X[0][1] - X[0][0]) * g.idx;
+      const T q0 = g.q[c], qe = g.q[c + 1], qw = g.q[c - 1], qn = g.q[c + nx], qs = g.q[c - nx];
+      T adv = T(0);
+      if (j >= 2 && j <= ny - 3 && i >= 2 && i <= nx - 3) {
+        const T fe = (u0 >= T(0) ? q0 : qe) * u0, fw = (uw >= T(0) ? qw : q0) * uw;
+        const T fn = (v0 >= T(0) ? q0 : qn) * v0, fs = (vs >= T(0) ? qs : q0) * vs;
+        adv = -((fe - fw) * g.idx + (fn - fs) * g.idy);
+      }
+      const T zeta = ((p[1][2] - p[1][1]) - (p[1][1] - p[1][0])) * (g.idx * g.idx) +
+                     ((p[2][1] - p[1][1]) - (p[1][1] - p[0][1])) * (g.idy * g.idy);
+      const T lq = ((qe - q0) - (q0 - qw)) * (g.idx * g.idx) +
+                   ((qn - q0) - (q0 - qs)) * (g.idy * g.idy);
+      rhs = (adv - g.beta * (T(0.5) * (v0 + vs))) - g.drag * zeta + g.visc * lq;
+    }
+  }
+  g.u[c] = u0;
+  g.v[c] = v0;
+  if (g.q) g.rhs[c] = rhs + g.wind[c];
+}
+
+template <typename T>
+static int gyre(const T* q, const T* psi, const T* wind, T* rhs, T* u, T* v, int ny, int nx,
+                double dx, double dy, double beta, double drag, double visc, hipStream_t s) {
+  FVX_CHECK_ARG(psi && u && v, "null field pointer");
+  FVX_CHECK_ARG(!q || (wind && rhs), "the tendency needs the wind field and an output");
+  FVX_CHECK_ARG(ny >= 3 && nx >= 3, "array too small (%d x %d); need >= 3 x 3", ny, nx);
+  FVX_CHECK_ARG(!q || (ny >= 5 && nx >= 5), "advection needs at least 5 x 5 (%d x %d)", ny, nx);
+  FVX_CHECK_ARG(dx > 0 && dy > 0, "grid spacing must be positive");
+  const GyreArgs<T> g{q,  psi, wind, rhs, u, v, ny, nx, (T)(1.0 / dx), (T)(1.0 / dy), (T)beta,
+                      (T)drag, (T)visc};
+  hipLaunchKernelGGL(gyre_kernel<T>, dim3(cdiv(nx, 64), cdiv(ny, 4)), dim3(64, 4), 0, s, g);
+  FVX_LAUNCH_CHECK();
+  return kOk;
+}
+
 }  // namespace fvx
 
 // ---------------------------------------------------------------------------
@@ -432,6 +514,12 @@ extern "C" {
   }                                                                                         \
   int fvx_enforce_periodic_##SUF(T* field, int ny, int nx, int ng, void* stream) {          \
     return fvx::enforce_periodic<T>(field, ny, nx, ng, (hipStream_t)stream);                \
+  }                                                                                         \
+  int fvx_gyre_tendency_##SUF(const T* q, const T* psi, const T* wind, T* rhs, T* u, T* v,  \
+                              int ny, int nx, double dx, double dy, double beta,            \
+                              double drag, double viscosity, void* stream) {                \
+    return fvx::gyre<T>(q, psi, wind, rhs, u, v, ny, nx, dx, dy, beta, drag, viscosity,     \
+                        (hipStream_t)stream);                                               \
   }
 
 FVX_DT(f32, float)

@@ -8,9 +8,10 @@ Each step is ``heun_step`` of
 
 with upwind1 advection, u = -d_y(T_to_X psi), v = d_x(T_to_X psi) at the
 U / V faces, zeta = lap(psi) and the wall (zero ghost ring) condition
-re-applied before each tendency and after the step (``:420-497``).  Every
-operator is one HIP kernel of ``libfvx_hip.so``; the Helmholtz inversion is the
-hipFFT DST-I solve.  Snapshots are returned as arrays (the reference writes
+re-applied before each tendency and after the step (``:420-497``).  The
+tendency's operators are one HIP kernel of ``libfvx_hip.so`` (one kernel each
+where the model's operators were replaced); the Helmholtz inversion is the
+DST-I solve.  Snapshots are returned as arrays (the reference writes
 them with xarray / Zarr, absent here).
 """
 
@@ -26,7 +27,7 @@ from finitevolx_amd.advection import Advection2D
 from finitevolx_amd.boundary import pad_interior
 from finitevolx_amd.grid import CartesianGrid2D
 from finitevolx_amd.operators import Difference2D, Interpolation2D
-from finitevolx_amd.solvers import solve_helmholtz_dst
+from finitevolx_amd.solvers import dirichlet_field_solve, solve_helmholtz_dst
 from finitevolx_amd.timestepping import heun_step, lincomb
 
 
@@ -58,9 +59,34 @@ def to_wall_field(interior) -> torch.Tensor:
     return torch.nn.functional.pad(t[None, None], (1, 1, 1, 1))[0, 0].contiguous()
 
 
+_lib.extra_signatures({
+    f"fvx_gyre_tendency_{s}": [_lib._vp] * 6 + [_lib._i] * 2 + [_lib._d] * 5 + [_lib._vp]
+    for s in ("f32", "f64")
+})
+
+
+def _unmasked(op, cls) -> bool:
+    return type(op) is cls and op.mask is None
+
+
+def _gyre(q, psi, wind, grid, beta=0.0, drag=0.0, viscosity=0.0):
+    """``(rhs, u, v)`` of the unmasked operators in one kernel; ``q`` None: no rhs."""
+    u, v = torch.empty_like(psi), torch.empty_like(psi)
+    rhs = None if q is None else torch.empty_like(q)
+    ny, nx = psi.shape
+    _lib.call(f"fvx_gyre_tendency_{_lib.suffix(psi)}", _lib.ptr(q), psi.data_ptr(),
+              _lib.ptr(wind), _lib.ptr(rhs), u.data_ptr(), v.data_ptr(), ny, nx,
+              float(grid.dx), float(grid.dy), float(beta), float(drag), float(viscosity),
+              _lib.stream())
+    return rhs, u, v
+
+
 def geostrophic_velocity_from_streamfunction(psi_field, diff: Difference2D,
                                              interp: Interpolation2D):
     """T-point psi -> (u, v) at U / V faces through X points (``:115-145``)."""
+    psi = _lib.as_field(psi_field)
+    if psi.dim() == 2 and _unmasked(diff, Difference2D) and _unmasked(interp, Interpolation2D):
+        return _gyre(None, psi, None, diff.grid)[1:]
     psi_on_x = interp.T_to_X(psi_field)
     return -diff.diff_y_X_to_U(psi_on_x), diff.diff_x_X_to_V(psi_on_x)
 
@@ -96,6 +122,8 @@ class QG1p5LayerModel:
 
     def invert_streamfunction(self, q_field):
         """(lap - 1/Ld^2) psi = q on the interior, psi = 0 walls (``:432-452``)."""
+        if q_field.dim() == 2 and min(q_field.shape) >= 4:
+            return dirichlet_field_solve(q_field, self.grid.dx, self.grid.dy, self.lam)
         psi_i = solve_helmholtz_dst(q_field[1:-1, 1:-1].contiguous(), self.grid.dx,
                                     self.grid.dy, self.lam)
         return to_wall_field(psi_i)
@@ -104,6 +132,12 @@ class QG1p5LayerModel:
         """``(q_rhs, psi, u, v)`` of ``tendency`` (``:454-478``)."""
         c = self.config
         psi = self.invert_streamfunction(q_field)
+        if self._plain_operators():
+            q, p = _lib.as_field(q_field), _lib.as_field(psi)
+            wind = _lib.as_field(self.wind_curl, q.dtype)
+            if q.dim() == 2 and p.dtype == q.dtype and p.shape == q.shape == wind.shape:
+                q_rhs, u, v = _gyre(q, p, wind, self.grid, c.beta, c.drag, c.viscosity)
+                return q_rhs, psi, u, v
         u, v = geostrophic_velocity_from_streamfunction(psi, self.diff, self.interp)
         q_rhs = self.adv(q_field, u, v, method="upwind1")
         # V_to_T's ghost ring is zero, so the full-array combination adds
@@ -113,6 +147,12 @@ class QG1p5LayerModel:
         zeta = self.diff.laplacian(psi)
         q_rhs = lincomb(1.0, q_rhs, -c.drag, zeta, c.viscosity, self.diff.laplacian(q_field))
         return q_rhs, psi, u, v
+
+    def _plain_operators(self) -> bool:
+        """Whether the tendency is that of the unmasked operators on one grid."""
+        return (_unmasked(self.diff, Difference2D) and _unmasked(self.interp, Interpolation2D)
+                and _unmasked(self.adv, Advection2D)
+                and self.diff.grid is self.grid and self.adv.grid is self.grid)
 
     @staticmethod
     def apply_bc(q_field):

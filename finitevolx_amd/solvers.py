@@ -483,6 +483,8 @@ _lib.extra_signatures({
     "fvx_spectral_plan_destroy": [_vp],
     "fvx_spectral_helmholtz_f64": [_vp, _vp, _i64, _vp, _i64, _d, _d, _d, _vp],
     "fvx_spectral_helmholtz_f32": [_vp, _vp, _i64, _vp, _i64, _d, _d, _d, _vp],
+    "fvx_spectral_helmholtz_field_f64": [_vp, _vp, _vp, _d, _d, _d, _vp, _vp],
+    "fvx_spectral_helmholtz_field_f32": [_vp, _vp, _vp, _d, _d, _d, _vp, _vp],
     "fvx_spectral_helmholtz_batch_f64": [_vp, _vp, _vp, _i, C.POINTER(_d), _d, _d, _vp, _vp],
     "fvx_spectral_helmholtz_batch_f32": [_vp, _vp, _vp, _i, C.POINTER(_d), _d, _d, _vp, _vp],
 })
@@ -508,6 +510,16 @@ class _SpecPlan:
 _SPEC_PLANS: dict = {}
 
 
+def _spec_plan(ny, nx, bc, bits):
+    key = (ny, nx, bc, bits)
+    plan = _SPEC_PLANS.get(key)
+    if plan is None:
+        if len(_SPEC_PLANS) > 8:
+            _SPEC_PLANS.clear()
+        plan = _SPEC_PLANS[key] = _SpecPlan(ny, nx, bc, bits)
+    return plan
+
+
 def _spectral(rhs, dx, dy, lambda_, bc):
     """Solve every trailing 2-D slice in one call; ``lambda_`` is a number or
     one per entry of the last leading axis."""
@@ -515,13 +527,7 @@ def _spectral(rhs, dx, dy, lambda_, bc):
     if b.dim() < 2:
         raise ValueError("spectral solves need at least 2-D input")
     ny, nx = b.shape[-2:]
-    bits = 64 if b.dtype == torch.float64 else 32
-    key = (ny, nx, bc, bits)
-    plan = _SPEC_PLANS.get(key)
-    if plan is None:
-        if len(_SPEC_PLANS) > 8:
-            _SPEC_PLANS.clear()
-        plan = _SPEC_PLANS[key] = _SpecPlan(ny, nx, bc, bits)
+    plan = _spec_plan(ny, nx, bc, 64 if b.dtype == torch.float64 else 32)
     nb = b.numel() // (ny * nx) if b.numel() else 0
     out = torch.empty_like(b)
     # (scratch of this call's stream: solves on several streams share a plan)
@@ -529,6 +535,20 @@ def _spectral(rhs, dx, dy, lambda_, bc):
     lam = np.broadcast_to(np.asarray(lambda_, dtype=np.float64), b.shape[:-2]).ravel()
     _lib.call(f"fvx_spectral_helmholtz_batch_{_lib.suffix(b)}", plan.h, b.data_ptr(),
               out.data_ptr(), nb, (_d * nb)(*lam), float(dx), float(dy), _lib.ptr(work),
+              _lib.stream())
+    return out
+
+
+def dirichlet_field_solve(field, dx, dy, lambda_):
+    """``solve_helmholtz_dst`` on the interior of a full 2-D field, the solution
+    in a full field with a zero ring: one call, no strip and no pad."""
+    b = _lib.as_field(field)
+    ny, nx = b.shape[0] - 2, b.shape[1] - 2
+    plan = _spec_plan(ny, nx, "dst", 64 if b.dtype == torch.float64 else 32)
+    out = torch.empty_like(b)
+    work = torch.empty((2, ny, nx), dtype=b.dtype, device=b.device)
+    _lib.call(f"fvx_spectral_helmholtz_field_{_lib.suffix(b)}", plan.h, b.data_ptr(),
+              out.data_ptr(), float(dx), float(dy), float(lambda_), work.data_ptr(),
               _lib.stream())
     return out
 

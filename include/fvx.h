@@ -198,6 +198,18 @@ int fvx_masked_laplacian_f64(const double* psi, const double* mask, double* out,
 int fvx_enforce_periodic_f32(float* field, int ny, int nx, int ng, void* stream);
 int fvx_enforce_periodic_f64(double* field, int ny, int nx, int ng, void* stream);
 
+/* ---- the double-gyre example's tendency and face velocities
+ * (scripts/qg_1p5_layer.py:115-145, :454-478) in one pass: u = -d_y(T_to_X
+ * psi), v = d_x(T_to_X psi), rhs = advection(q; upwind1) - beta V_to_T(v) +
+ * wind - drag lap(psi) + viscosity lap(q), unmasked; q NULL (then wind and rhs
+ * too): velocities only. */
+int fvx_gyre_tendency_f32(const float* q, const float* psi, const float* wind, float* rhs,
+                          float* u, float* v, int ny, int nx, double dx, double dy, double beta,
+                          double drag, double viscosity, void* stream);
+int fvx_gyre_tendency_f64(const double* q, const double* psi, const double* wind, double* rhs,
+                          double* u, double* v, int ny, int nx, double dx, double dy, double beta,
+                          double drag, double viscosity, void* stream);
+
 /* ---- rk3_ssp_step stage combination (timestepping/explicit_rk.py:104-121) --
  * out = a*x + b*y + c*z (+ d*w) over n elements (y, z, w nullable); out may
  * be one of the inputs (each element is read before it is written).         */
@@ -376,6 +388,13 @@ int fvx_spectral_helmholtz_batch_f32(void* plan, const float* rhs, float* out, i
 int fvx_spectral_helmholtz_batch_f64(void* plan, const double* rhs, double* out, int nb,
                                      const double* lambda_, double dx, double dy, double* work,
                                      void* stream);
+/* One solve on the interior of full (ny + 2, nx + 2) fields (ny, nx: the
+ * plan's): out's one-cell ring is written zero, rhs' ring is not read; out is
+ * another array.  work: 2 ny nx elements, as above. */
+int fvx_spectral_helmholtz_field_f32(void* plan, const float* rhs, float* out, double dx,
+                                     double dy, double lambda_, float* work, void* stream);
+int fvx_spectral_helmholtz_field_f64(void* plan, const double* rhs, double* out, double dx,
+                                     double dy, double lambda_, double* work, void* stream);
 
 /* ---- QG 1.5-layer step (composition; nearest reference
  * scripts/qg_1p5_layer.py:420-497; operators as cited above) -------------- */
