@@ -29,6 +29,7 @@ _RESTYPES = {"fvx_last_error": C.c_char_p}
 for _suf in ("f32", "f64"):
     _SIGS.update({
         f"fvx_stencil2d_{_suf}": [_i, _vp, _vp, _vp, _i, _i, _d, _d, _vp, _vp],
+        f"fvx_grad_perp_{_suf}": [_vp, _vp, _vp, _i, _i, _d, _d, _vp, _vp, _vp],
         f"fvx_diffusion2d_{_suf}": [_vp, _vp, _d, _vp, _i, _i, _d, _d, _vp, _vp, _vp, _vp],
         f"fvx_diffusion2d_fluxes_{_suf}": [_vp, _vp, _d, _vp, _vp, _i, _i, _d, _d, _vp, _vp, _vp],
         f"fvx_biharmonic2d_{_suf}": [_vp, _vp, _i, _i, _d, _d, _d, _vp, _vp],

@@ -95,7 +95,20 @@ class Difference2D:
 
     def grad_perp(self, psi):
         """T-point psi -> (u, v) at U/V points (``difference.py:456-519``)."""
-        return self._op("grad_perp_u", psi), self._op("grad_perp_v", psi)
+        a = _lib.as_field(psi)
+        if a.dim() != 2:
+            raise ValueError(f"expected a 2-D field, got shape {tuple(a.shape)}")
+        mu, mv = (None, None) if self.mask is None else (self.mask.device("u"),
+                                                         self.mask.device("v"))
+        for m in (mu, mv):
+            if m is not None and tuple(m.shape) != tuple(a.shape):
+                raise ValueError(f"mask shape {tuple(m.shape)} != field shape {tuple(a.shape)}")
+        u, v = torch.empty_like(a), torch.empty_like(a)
+        ny, nx = a.shape
+        _lib.call(f"fvx_grad_perp_{_lib.suffix(a)}", a.data_ptr(), u.data_ptr(), v.data_ptr(), ny,
+                  nx, float(self.grid.dx), float(self.grid.dy), _lib.ptr(mu), _lib.ptr(mv),
+                  _lib.stream())
+        return u, v
 
 
 def divergence_2d(u, v, dx: float, dy: float):

@@ -51,6 +51,12 @@ int fvx_stencil2d_f32(int op, const float* a, const float* b, float* out, int ny
                       double dx, double dy, const uint8_t* mask, void* stream);
 int fvx_stencil2d_f64(int op, const double* a, const double* b, double* out, int ny, int nx,
                       double dx, double dy, const uint8_t* mask, void* stream);
+/* Both components of Difference2D.grad_perp (operators/difference.py:456-519)
+ * in one pass; mask_u / mask_v: their stagger masks or NULL. */
+int fvx_grad_perp_f32(const float* psi, float* u, float* v, int ny, int nx, double dx, double dy,
+                      const uint8_t* mask_u, const uint8_t* mask_v, void* stream);
+int fvx_grad_perp_f64(const double* psi, double* u, double* v, int ny, int nx, double dx,
+                      double dy, const uint8_t* mask_u, const uint8_t* mask_v, void* stream);
 
 /* ---- Advection2D.__call__ (advection/advection.py:329-420) -----------------
  * method: FVX_ADV_*; limiter used when method == FVX_ADV_TVD.

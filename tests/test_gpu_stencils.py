@@ -83,6 +83,46 @@ def test_diffusion_goldens(variant):
                                rtol=1e-12, atol=1e-14)
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("ny,nx", [(3, 3), (4, 5), (5, 4), (6, 62), (9, 125), (5, 64),
+                                   (725, 731), (4099, 129), (130, 4097)])
+def test_operators_at_tile_edges(ny, nx, masked, dtype, tol):
+    """Every operator at the edges of its strips (60, 62 and 64 columns, 1 to 8
+    rows), on both sides of the size where the wavefronts take more rows."""
+    need_gpu()
+    rng = np.random.default_rng(ny + nx)
+    u, v, h, psi = rng.standard_normal((4, ny, nx))
+    kap = rng.random((ny, nx))
+    wet = random_mask(ny, nx, 4) if masked else None
+    om, m = (fvx.Mask2D(wet), fx.Mask2D(wet)) if masked else (None, None)
+    dx, dy = 0.3, 0.4
+    g = fx.CartesianGrid2D(nx, ny, 1.0, 1.0, dx, dy)
+    d = fx.Difference2D(g, m)
+    t = {k: torch.tensor(a, dtype=dtype, device="cuda")
+         for k, a in dict(u=u, v=v, h=h, psi=psi, kap=kap).items()}
+    src = dict(u=u, v=v, h=h)
+    pairs = [(getattr(d, name)(t[arg]), ref(src[arg], dx if sp == "dx" else dy, om), name)
+             for name, arg, ref, sp in DIFF_OPS]
+    pairs += [(d.laplacian(t["h"]), fvx.laplacian(h, dx, dy, om), "laplacian"),
+              (d.curl(t["u"], t["v"]), fvx.curl(u, v, dx, dy, om), "curl"),
+              (d.divergence(t["u"], t["v"]), fvx.divergence(u, v, dx, dy, om), "divergence"),
+              (fx.Divergence2D(g, m).noflux(t["u"], t["v"]),
+               fvx.divergence_noflux(u, v, dx, dy, om), "noflux"),
+              (fx.Interpolation2D(g, m).T_to_X(t["h"]), fvx.T_to_X(h, om), "T_to_X"),
+              (fx.Diffusion2D(g, m)(t["h"], t["kap"]), fvx.diffusion_2d(h, kap, dx, dy, om), "diff"),
+              (fx.BiharmonicDiffusion2D(g, m)(t["h"], 0.7), fvx.biharmonic_2d(h, 0.7, dx, dy, om),
+               "biharmonic"),
+              (fx.arakawa_jacobian(t["psi"], t["h"], dx, dy), fvx.arakawa_jacobian(psi, h, dx, dy),
+               "arakawa")]
+    pairs += list(zip(d.grad_perp(t["psi"]), fvx.grad_perp(psi, dx, dy, om), ("gu", "gv")))
+    for s in ("energy", "enstrophy", "al"):
+        pairs += list(zip(fx.MomentumAdvection2D(g, m)(t["u"], t["v"], s),
+                          fvx.momentum_advection_2d(u, v, dx, dy, s, om), (s + " du", s + " dv")))
+    for got, ref, name in pairs:
+        assert_close_scaled(to_np(got), ref, tol, f"{name} {ny}x{nx}")
+
+
 ALL_METHODS = ["naive", "upwind1", "upwind2", "upwind3", "weno3", "weno5", "wenoz5",
                "minmod", "van_leer", "superbee", "mc"]
 
