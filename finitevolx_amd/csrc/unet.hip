@@ -193,8 +193,9 @@ __global__ __launch_bounds__(conv_threads(COB)) void conv_mfma_kernel(
 // writes its own fp32 slot of ``part`` once; reduce_slots_kernel sums them.
 // Bound: reading x and gy (16 channels: 16.8 MB at 512^2, ~3 us) and the
 // transposing LDS writes.  Measured: 16 -> 16 channels at 512^2 11 us, 48 -> 48
-// at 128^2 16 us (112 us each with 64 blocks gathering the fragments two bytes
-// at a time and adding every tile to the slot in memory).
+// at 128^2 9.5 us (112 us each with 64 blocks gathering the fragments two bytes
+// at a time and adding every tile to the slot in memory; 17 with one item of a
+// tile at a time and a block per tile), 64 -> 64 at 64^2 9.5 us (21).
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -211,15 +212,34 @@ __device__ __forceinline__ void transpose4(const uint2 (&p)[4], uint2 (&c)[4]) {
                     (p[2].y >> 16) | (p[3].y & 0xffff0000u));
 }
 
+// items items of 4 pixels x 4 channels: load(item, pixels), transposed,
+// store(item, channels), the loads of two items a thread in flight together
+// (one after the other, each item was a memory latency).
+template <typename Load, typename Store>
+__device__ __forceinline__ void stage_items(int items, Load load, Store store) {
+  for (int k = threadIdx.x; k < items; k += 2 * kUThreads) {
+    uint2 p[2][4], c[4];
+    const int k1 = k + kUThreads;
+    load(k, p[0]);
+    load(min(k1, items - 1), p[1]);
+    transpose4(p[0], c);
+    store(k, c);
+    if (k1 < items) {
+      transpose4(p[1], c);
+      store(k1, c);
+    }
+  }
+}
+
 template <int PW, int RS, bool UPS>
 __global__ __launch_bounds__(kUThreads) void conv_bwdw_mfma_kernel(
-    const uint16_t* __restrict__ x, int Cin, const uint16_t* __restrict__ gy, int Cout,
+    const uint16_t* __restrict__ x, int Cin, const uint16_t* __restrict__ gy, int Cout, int cobn,
     float* __restrict__ part, int H, int W, int tiles_x, int ntiles) {
   extern __shared__ __align__(16) uint16_t smem[];
   uint16_t* sx = smem;                           // [Cin][TH + 2][kWXRow]
-  uint16_t* sg = smem + (int64_t)Cin * kWXPitch;  // [Cout][TH][TW]
+  uint16_t* sg = smem + (int64_t)Cin * kWXPitch;  // [16 cobn][TH][TW]
   constexpr int NWP = 4 / RS, ROWS = kUTh / RS;
-  const int COB = Cout / 16, CIB = Cin / 16, NP = COB * CIB;
+  const int CIB = Cin / 16, NP = cobn * CIB, cob0 = blockIdx.y * cobn;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wp = wave % NWP, rs = wave / NWP;
@@ -234,42 +254,45 @@ __global__ __launch_bounds__(kUThreads) void conv_bwdw_mfma_kernel(
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const int i0 = (t % tiles_x) * kUTw, j0 = (t / tiles_x) * kUTh;
     __syncthreads();
-    const int c4x = Cin / 4;
-    for (int k = tid; k < (kUTh + 2) * 17 * c4x; k += kUThreads) {
-      const int c4 = k % c4x, u = k / c4x, g = u % 17, ry = u / 17;
-      const int gyy = j0 - 1 + ry;
-      uint2 px[4], ch[4];
+    const int c4x = Cin / 4, c4g = 4 * cobn;
+    stage_items(
+        (kUTh + 2) * 17 * c4x,
+        [&](int k, uint2(&px)[4]) {
+          const int c4 = k % c4x, u = k / c4x, g = u % 17, gyy = j0 - 1 + u / 17;
+          const int cy = min(max(gyy, 0), H - 1);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int gxx = i0 - 1 + 4 * g + e;
-        px[e] = make_uint2(0u, 0u);
-        if (gyy >= 0 && gyy < H && gxx >= 0 && gxx < W) {
-          const int sy = UPS ? (gyy >> 1) : gyy, sxx = UPS ? (gxx >> 1) : gxx;
-          px[e] = *reinterpret_cast<const uint2*>(x + ((int64_t)sy * Wx + sxx) * Cin + 4 * c4);
-        }
-      }
-      transpose4(px, ch);
+          for (int e = 0; e < 4; ++e) {
+            const int gxx = i0 - 1 + 4 * g + e, cx = min(max(gxx, 0), W - 1);
+            const int sy = UPS ? (cy >> 1) : cy, sxx = UPS ? (cx >> 1) : cx;
+            px[e] = *reinterpret_cast<const uint2*>(x + ((int64_t)sy * Wx + sxx) * Cin + 4 * c4);
+            if (cy != gyy || cx != gxx) px[e] = make_uint2(0u, 0u);
+          }
+        },
+        [&](int k, const uint2(&ch)[4]) {
+          const int c4 = k % c4x, u = k / c4x, g = u % 17, ry = u / 17;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        *reinterpret_cast<uint2*>(sx + (4 * c4 + e) * kWXPitch + ry * kWXRow + 4 * g) = ch[e];
-    }
-    const int c4g = Cout / 4;
-    for (int k = tid; k < kUTh * (kUTw / 4) * c4g; k += kUThreads) {
-      const int c4 = k % c4g, u = k / c4g, g = u % (kUTw / 4), ry = u / (kUTw / 4);
-      const int gyy = j0 + ry;
-      uint2 px[4], ch[4];
+          for (int e = 0; e < 4; ++e)
+            *reinterpret_cast<uint2*>(sx + (4 * c4 + e) * kWXPitch + ry * kWXRow + 4 * g) = ch[e];
+        });
+    stage_items(
+        kUTh * (kUTw / 4) * c4g,
+        [&](int k, uint2(&px)[4]) {
+          const int c4 = k % c4g, u = k / c4g, g = u % (kUTw / 4), gyy = j0 + u / (kUTw / 4);
+          const int cy = min(gyy, H - 1);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int gxx = i0 + 4 * g + e;
-        px[e] = (gyy < H && gxx < W) ? *reinterpret_cast<const uint2*>(
-                                           gy + ((int64_t)gyy * W + gxx) * Cout + 4 * c4)
-                                     : make_uint2(0u, 0u);
-      }
-      transpose4(px, ch);
+          for (int e = 0; e < 4; ++e) {
+            const int gxx = i0 + 4 * g + e, cx = min(gxx, W - 1);
+            px[e] = *reinterpret_cast<const uint2*>(gy + ((int64_t)cy * W + cx) * Cout +
+                                                    16 * cob0 + 4 * c4);
+            if (cy != gyy || cx != gxx) px[e] = make_uint2(0u, 0u);
+          }
+        },
+        [&](int k, const uint2(&ch)[4]) {
+          const int c4 = k % c4g, u = k / c4g, g = u % (kUTw / 4), ry = u / (kUTw / 4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        *reinterpret_cast<uint2*>(sg + (4 * c4 + e) * kWGPitch + ry * kUTw + 4 * g) = ch[e];
-    }
+          for (int e = 0; e < 4; ++e)
+            *reinterpret_cast<uint2*>(sg + (4 * c4 + e) * kWGPitch + ry * kUTw + 4 * g) = ch[e];
+        });
     __syncthreads();
     for (int rk = 0; rk < 2 * ROWS; ++rk) {
       const int r = rs * ROWS + (rk >> 1), col = 32 * (rk & 1) + 8 * lgrp;
@@ -331,19 +354,33 @@ __global__ __launch_bounds__(kUThreads) void conv_bwdw_mfma_kernel(
     for (int q = 0; q < 9; ++q)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        mine[((int64_t)q * Cout + cob * 16 + 4 * lgrp + i) * Cin + cib * 16 + lrow] = acc[k][q][i];
+        mine[((int64_t)q * Cout + (cob0 + cob) * 16 + 4 * lgrp + i) * Cin + cib * 16 + lrow] = acc[k][q][i];
   }
 }
 
-// out[e] (+)= sum over slots of part[g][e], 64 elements a block: 16 wavefronts
-// take every 16th slot (independent loads in flight; with one thread per
-// element the 64 slots were a 15 us chain), then sum in LDS in wave order.
-constexpr int kRedWaves = 16;
-__global__ __launch_bounds__(64 * kRedWaves) void reduce_slots_kernel(
-    const float* __restrict__ part, int nslot, int n, float* __restrict__ out, int accumulate) {
+// out[e] += sum over slots of part[g][e] for every layer of a backward pass in
+// one launch (14 of them took 5 us each at the default network), 64 elements a
+// block: 16 wavefronts take every 16th slot (independent loads in flight; with
+// one thread per element the 64 slots were a 15 us chain), then sum in LDS in
+// wave order.
+constexpr int kRedWaves = 16, kMaxLayers = 31;  // 8 levels: 16 + 14 + 1
+struct RedTable {
+  int layers = 0, blocks = 0;
+  struct {
+    const float* part;
+    float* out;
+    int nslot, n, block0;
+  } l[kMaxLayers];
+};
+__global__ __launch_bounds__(64 * kRedWaves) void reduce_slots_kernel(RedTable t) {
   __shared__ float red[kRedWaves][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int e = blockIdx.x * 64 + lane;
+  int k = 0;
+  while (k + 1 < t.layers && (int)blockIdx.x >= t.l[k + 1].block0) ++k;
+  const float* part = t.l[k].part;
+  float* out = t.l[k].out;
+  const int nslot = t.l[k].nslot, n = t.l[k].n;
+  const int e = ((int)blockIdx.x - t.l[k].block0) * 64 + lane;
   float s = 0.f;
   if (e < n) {
 #pragma unroll 8
@@ -354,8 +391,8 @@ __global__ __launch_bounds__(64 * kRedWaves) void reduce_slots_kernel(
   if (wave == 0 && e < n) {
     float v = 0.f;
 #pragma unroll
-    for (int k = 0; k < kRedWaves; ++k) v += red[k][lane];
-    out[e] = accumulate ? out[e] + v : v;
+    for (int q = 0; q < kRedWaves; ++q) v += red[q][lane];
+    out[e] += v;
   }
 }
 
@@ -464,7 +501,8 @@ __global__ void conv_last_bwd_data_kernel(const float* __restrict__ gy, const fl
 // the gradient of the first layer).  A thread owns 8 channels of every
 // (256 * 8 / C)-th pixel of its block: one 16-byte load of sc and nine of s1
 // feed its 72 register sums, where one pass over both fields per (tap, c)
-// took 846 us at 512^2 with 16 channels (now 34 us).  part: [nblk][9 * C].
+// took 846 us at 512^2 with 16 channels (now 15 us; 34 with 216 lane moves in
+// the sums over lanes).  part: [nblk][9 * C].
 __global__ __launch_bounds__(256) void edge_bwdw_kernel(const float* __restrict__ s1,
                                                         const uint16_t* __restrict__ sc, int C,
                                                         int sgn, float* __restrict__ part, int H,
@@ -496,29 +534,49 @@ __global__ __launch_bounds__(256) void edge_bwdw_kernel(const float* __restrict_
 #pragma unroll
       for (int t = 0; t < 9; ++t) {
         const int y = j - sgn * (t / 3 - 1), x = i - sgn * (t % 3 - 1);
-        const bool in = y >= 0 && y < H && x >= 0 && x < W;
-        const float g = in ? s1[(int64_t)y * W + x] : 0.f;
+        const int cy = min(max(y, 0), H - 1), cx = min(max(x, 0), W - 1);
+        float g = s1[(int64_t)cy * W + cx];
+        g = cy == y && cx == x ? g : 0.f;
 #pragma unroll
         for (int h = 0; h < 8; ++h) acc[t][h] += g * f[h];
       }
     }
   }
-  // Sum over the lanes of one channel group (stride cg; power-of-two groups
-  // by butterflies, six groups through their first lanes).
+  // Sum over the lanes of one channel group (stride cg).  Power-of-two groups:
+  // three butterfly steps that hand half of the sums to the other lane each
+  // (channels 4, 2, 1: 63 lane moves instead of 216), then plain ones; lane l
+  // ends with the nine taps of channel 4 l5 + 2 l4 + l3 of its group.  Six
+  // groups through their first lanes.
+  if (cg != 6) {
+    float r4[9][4], r2[9][2], r1[9];
+    const bool h5 = lane & 32, h4 = lane & 16, h3 = lane & 8;
 #pragma unroll
-  for (int t = 0; t < 9; ++t)
+    for (int t = 0; t < 9; ++t) {
 #pragma unroll
-    for (int h = 0; h < 8; ++h) {
-      float s = acc[t][h];
-      if (cg != 6) {
-        for (int o = 32; o >= cg; o >>= 1) s += __shfl_xor(s, o);
-      } else {
-        float r = s;
-        for (int k = 1; k < 10; ++k) r += __shfl(s, min(lane + 6 * k, 63));
-        s = r;
-      }
-      if (lane < cg) red[wave][t * C + 8 * c8 + h] = s;
+      for (int h = 0; h < 4; ++h)
+        r4[t][h] = (h5 ? acc[t][h + 4] : acc[t][h]) +
+                   __shfl_xor(h5 ? acc[t][h] : acc[t][h + 4], 32);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        r2[t][h] = (h4 ? r4[t][h + 2] : r4[t][h]) + __shfl_xor(h4 ? r4[t][h] : r4[t][h + 2], 16);
+      r1[t] = (h3 ? r2[t][1] : r2[t][0]) + __shfl_xor(h3 ? r2[t][0] : r2[t][1], 8);
+      for (int o = 4; o >= cg; o >>= 1) r1[t] += __shfl_xor(r1[t], o);
     }
+    const int h = (h5 ? 4 : 0) + (h4 ? 2 : 0) + (h3 ? 1 : 0);
+    if ((lane & 7) < cg) {
+#pragma unroll
+      for (int t = 0; t < 9; ++t) red[wave][t * C + 8 * c8 + h] = r1[t];
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int h = 0; h < 8; ++h) {
+        float r = acc[t][h];
+        for (int k = 1; k < 10; ++k) r += __shfl(acc[t][h], min(lane + 6 * k, 63));
+        if (lane < cg) red[wave][t * C + 8 * c8 + h] = r;
+      }
+  }
   __syncthreads();
   for (int e = tid; e < 9 * C; e += 256)
     part[(int64_t)blockIdx.x * 9 * C + e] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
@@ -695,8 +753,8 @@ struct UNet {
   // activations per level: x (pooled input, l > 0), h1e, e (=h2e), h1d, d
   std::vector<uint16_t*> xin, h1e, ee, h1d, dd, gA, gB, gC;
   float *rin = nullptr, *yout = nullptr, *gy = nullptr, *eref = nullptr;
-  float* part = nullptr;
-  size_t part_elems = 0;
+  float* part = nullptr;     // weight-gradient slots, each layer's from part_off
+  std::vector<size_t> part_off;
   double* rms_part = nullptr;
   float* scal = nullptr;
   double* loss = nullptr;
@@ -799,30 +857,52 @@ static int unet_forward(UNet& N, int H, int W, hipStream_t s, bool last = true) 
   return kOk;
 }
 
-// Blocks of a weight-gradient launch: two per CU (each writes a slot that the
-// reduction reads back, so more only add traffic).
-constexpr int kBwdwBlocks = 512;
-
-template <int PW, int RS, bool UPS>
-static void launch_bwdw(UNet& N, const Layer& Ly, const uint16_t* x, const uint16_t* gyt, int G,
-                        int H, int W, int tx, int nt, hipStream_t s) {
-  const size_t stage = ((size_t)Ly.cin * kWXPitch + (size_t)Ly.cout * kWGPitch) * sizeof(uint16_t);
-  const size_t sums = (size_t)(RS - 1) * (4 / RS) * PW * 9 * 64 * sizeof(f32x4);
-  hipLaunchKernelGGL((conv_bwdw_mfma_kernel<PW, RS, UPS>), dim3(G), dim3(kUThreads),
-                     std::max(stage, sums), s, x, Ly.cin, gyt, Ly.cout, N.part, H, W, tx, nt);
+// Slots of layer li's weight gradient at H x W pixels: a block per tile, at most
+// two per CU (each writes a slot that the reduction reads back, so more only add
+// traffic) and 9.4 MB; the one-channel layers a block per 256 pixels.
+constexpr int kBwdwBlocks = 512, kBwdwSplit = 256;
+static int bwdw_slots(const Layer& Ly, int H, int W) {
+  if (Ly.cout == 1 || Ly.cin == 1)
+    return (int)std::min<int64_t>(((int64_t)H * W + 255) / 256, kBwdwBlocks);
+  const size_t n = (size_t)9 * Ly.cout * Ly.cin;
+  const int nt = cdiv(W, kUTw) * cdiv(H, kUTh);
+  return (int)std::min<size_t>(std::min(nt, kBwdwBlocks), (size_t)64 * 9 * 64 * 64 / n);
+}
+static void red_add(const UNet& N, int li, int nslot, RedTable& t) {
+  const Layer& Ly = N.layers[li];
+  auto& e = t.l[t.layers++];
+  e.part = N.part + N.part_off[li];
+  e.out = N.g + Ly.off;
+  e.nslot = nslot;
+  e.n = 9 * Ly.cout * Ly.cin;
+  e.block0 = t.blocks;
+  t.blocks += cdiv(e.n, 64);
 }
 
-static int bwdw_launch(UNet& N, int li, const uint16_t* x, const uint16_t* gyt, bool ups, int H,
-                       int W, hipStream_t s) {
+template <int PW, int RS, bool UPS>
+static void launch_bwdw(float* part, const Layer& Ly, const uint16_t* x, const uint16_t* gyt, int G,
+                        int cobn, int H, int W, int tx, int nt, hipStream_t s) {
+  const size_t stage = ((size_t)Ly.cin * kWXPitch + (size_t)16 * cobn * kWGPitch) * sizeof(uint16_t);
+  const size_t sums = (size_t)(RS - 1) * (4 / RS) * PW * 9 * 64 * sizeof(f32x4);
+  hipLaunchKernelGGL((conv_bwdw_mfma_kernel<PW, RS, UPS>), dim3(G, Ly.cout / 16 / cobn),
+                     dim3(kUThreads), std::max(stage, sums), s, x, Ly.cin, gyt, Ly.cout, cobn,
+                     part, H, W, tx, nt);
+}
+
+static void bwdw_launch(UNet& N, int li, const uint16_t* x, const uint16_t* gyt, bool ups, int H,
+                        int W, RedTable& red, hipStream_t s) {
   const Layer& Ly = N.layers[li];
+  float* part = N.part + N.part_off[li];
   const int tx = cdiv(W, kUTw), ty = cdiv(H, kUTh), nt = tx * ty;
-  const size_t n = (size_t)9 * Ly.cout * Ly.cin;
-  const int G = (int)std::min<size_t>(std::min(nt, kBwdwBlocks), N.part_elems / n);
-  FVX_CHECK_ARG(G >= 1, "gradient scratch too small");
-  const int np = (Ly.cout / 16) * (Ly.cin / 16);  // (co, ci) block pairs, 1 .. 16
+  const int G = bwdw_slots(Ly, H, W);
+  // Few tiles: a block per 16 output channels (and tile), which leaves each the
+  // x tile, a share of gy and of the products (gradient at 512^2, splitting up to 170,
+  // 256, 512 tiles: 598, 584-595, 594-611 us; never: 674 and up).
+  const int cobn = G <= kBwdwSplit ? 1 : Ly.cout / 16;
+  const int np = cobn * (Ly.cin / 16);  // (co, ci) block pairs of a block, 1 .. 16
 #define FVX_BWDW(PW, RS)                                                          \
-  (ups ? launch_bwdw<PW, RS, true>(N, Ly, x, gyt, G, H, W, tx, nt, s)             \
-       : launch_bwdw<PW, RS, false>(N, Ly, x, gyt, G, H, W, tx, nt, s))
+  (ups ? launch_bwdw<PW, RS, true>(part, Ly, x, gyt, G, cobn, H, W, tx, nt, s)       \
+       : launch_bwdw<PW, RS, false>(part, Ly, x, gyt, G, cobn, H, W, tx, nt, s))
   if (np == 1) FVX_BWDW(1, 4);
   else if (np == 2) FVX_BWDW(1, 2);
   else if (np <= 4) FVX_BWDW(1, 1);
@@ -830,24 +910,15 @@ static int bwdw_launch(UNet& N, int li, const uint16_t* x, const uint16_t* gyt, 
   else if (np <= 12) FVX_BWDW(3, 1);
   else FVX_BWDW(4, 1);
 #undef FVX_BWDW
-  hipLaunchKernelGGL(reduce_slots_kernel, dim3(cdiv((int)n, 64)), dim3(64 * kRedWaves), 0, s,
-                     N.part, G, (int)n, N.g + Ly.off, 1);
-  FVX_LAUNCH_CHECK();
-  return kOk;
+  red_add(N, li, G, red);
 }
 
-static int edge_bwdw(UNet& N, int li, const float* s1, const uint16_t* sc, int C, bool swap,
-                     int H, int W, hipStream_t s) {
-  const Layer& Ly = N.layers[li];
-  const int64_t px = (int64_t)H * W;
-  const int G = (int)std::min<int64_t>((px + 255) / 256, kBwdwBlocks);
-  const size_t n = (size_t)9 * C;
-  hipLaunchKernelGGL(edge_bwdw_kernel, dim3(G), dim3(256), 0, s, s1, sc, C, swap ? -1 : 1, N.part,
-                     H, W);
-  hipLaunchKernelGGL(reduce_slots_kernel, dim3(cdiv((int)n, 64)), dim3(64 * kRedWaves), 0, s,
-                     N.part, G, (int)n, N.g + Ly.off, 1);
-  FVX_LAUNCH_CHECK();
-  return kOk;
+static void edge_bwdw(UNet& N, int li, const float* s1, const uint16_t* sc, int C, bool swap,
+                      int H, int W, RedTable& red, hipStream_t s) {
+  const int G = bwdw_slots(N.layers[li], H, W);
+  hipLaunchKernelGGL(edge_bwdw_kernel, dim3(G), dim3(256), 0, s, s1, sc, C, swap ? -1 : 1,
+                     N.part + N.part_off[li], H, W);
+  red_add(N, li, G, red);
 }
 
 // Backward from N.gy (dLoss/dy, fp32) to weight gradients accumulated in N.g.
@@ -856,21 +927,19 @@ static int unet_backward(UNet& N, int H, int W, hipStream_t s) {
   // output layer
   const Layer& o = N.layers.back();
   const uint16_t* d0 = (L > 1) ? N.dd[0] : N.ee[0];
-  int rc = edge_bwdw(N, (int)N.layers.size() - 1, N.gy, d0, N.ch[0], false, H, W, s);
-  if (rc) return rc;
+  RedTable red;
+  edge_bwdw(N, (int)N.layers.size() - 1, N.gy, d0, N.ch[0], false, H, W, red, s);
   hipLaunchKernelGGL(conv_last_bwd_data_kernel, g2(H, W), dim3(64, 4), 0, s, N.gy, N.w + o.off,
                      N.ch[0], d0, N.gA[0], H, W);
   // decoder levels 0 .. L-2: gA[l] holds the masked gradient into d_l's a2
   for (int l = 0; l <= L - 2; ++l) {
     const int h = H >> l, w = W >> l;
-    rc = bwdw_launch(N, layer_index(N, 'd', l), N.h1d[l], N.gA[l], false, h, w, s);
-    if (rc) return rc;
+    bwdw_launch(N, layer_index(N, 'd', l), N.h1d[l], N.gA[l], false, h, w, red, s);
     // ga1 = conv^T(ga2) * (h1d > 0) -> gB[l]  (also the skip gradient into e_l)
     conv_launch(N, layer_index(N, 'd', l), true, N.gA[l], N.gB[l], nullptr, N.h1d[l], false, false,
                 h, w, s);
     const uint16_t* dnext = (l + 1 == L - 1) ? N.ee[L - 1] : N.dd[l + 1];
-    rc = bwdw_launch(N, layer_index(N, 'u', l), dnext, N.gB[l], true, h, w, s);
-    if (rc) return rc;
+    bwdw_launch(N, layer_index(N, 'u', l), dnext, N.gB[l], true, h, w, red, s);
     // gu (fine, C_{l+1} channels) -> gC[l]; up2 backward + relu mask of d_{l+1} -> gA[l+1]
     conv_launch(N, layer_index(N, 'u', l), true, N.gB[l], N.gC[l], nullptr, nullptr, false, false,
                 h, w, s);
@@ -881,18 +950,15 @@ static int unet_backward(UNet& N, int H, int W, hipStream_t s) {
   // encoder levels L-1 .. 0: gA[l] holds the masked gradient into e_l's a2
   for (int l = L - 1; l >= 0; --l) {
     const int h = H >> l, w = W >> l;
-    rc = bwdw_launch(N, layer_index(N, 'b', l), N.h1e[l], N.gA[l], false, h, w, s);
-    if (rc) return rc;
+    bwdw_launch(N, layer_index(N, 'b', l), N.h1e[l], N.gA[l], false, h, w, red, s);
     // ga1 = conv^T(ga2) * (h1e > 0) -> gC[l]
     conv_launch(N, layer_index(N, 'b', l), true, N.gA[l], N.gC[l], nullptr, N.h1e[l], false, false,
                 h, w, s);
     if (l == 0) {
-      rc = edge_bwdw(N, layer_index(N, 'a', 0), N.rin, N.gC[0], N.ch[0], true, h, w, s);
-      if (rc) return rc;
+      edge_bwdw(N, layer_index(N, 'a', 0), N.rin, N.gC[0], N.ch[0], true, h, w, red, s);
       break;
     }
-    rc = bwdw_launch(N, layer_index(N, 'a', l), N.xin[l], N.gC[l], false, h, w, s);
-    if (rc) return rc;
+    bwdw_launch(N, layer_index(N, 'a', l), N.xin[l], N.gC[l], false, h, w, red, s);
     // gx = conv^T(ga1) (C_{l-1} channels at level l) -> gA[l] (free now)
     conv_launch(N, layer_index(N, 'a', l), true, N.gC[l], N.gA[l], nullptr, nullptr, false, false,
                 h, w, s);
@@ -902,6 +968,7 @@ static int unet_backward(UNet& N, int H, int W, hipStream_t s) {
                        (l - 1 <= L - 2) ? N.gB[l - 1] : nullptr, N.gA[l], N.ee[l - 1],
                        N.gA[l - 1], hf, wf, c);
   }
+  hipLaunchKernelGGL(reduce_slots_kernel, dim3(red.blocks), dim3(64 * kRedWaves), 0, s, red);
   FVX_LAUNCH_CHECK();
   return kOk;
 }
@@ -991,8 +1058,14 @@ int fvx_unet_create(int nlev, const int* channels, int H, int W, void** out) {
   rc |= dev_alloc(*N, &N->yout, npx);
   rc |= dev_alloc(*N, &N->gy, npx);
   rc |= dev_alloc(*N, &N->eref, npx);
-  N->part_elems = (size_t)64 * 9 * 64 * 64;
-  rc |= dev_alloc(*N, &N->part, N->part_elems);
+  size_t slots = 0;
+  for (size_t li = 0; li < N->layers.size(); ++li) {
+    const Layer& Ly = N->layers[li];
+    const int k = (int)li, l = k < 2 * nlev ? k / 2 : (k == (int)N->layers.size() - 1 ? 0 : nlev - 2 - (k - 2 * nlev) / 2);
+    N->part_off.push_back(slots);
+    slots += (size_t)bwdw_slots(Ly, H >> l, W >> l) * 9 * Ly.cout * Ly.cin;
+  }
+  rc |= dev_alloc(*N, &N->part, slots);
   rc |= dev_alloc(*N, &N->rms_part, 4096);
   rc |= dev_alloc(*N, &N->scal, 4);
   rc |= dev_alloc(*N, &N->loss, 1);

@@ -109,6 +109,28 @@ def test_weight_gradients_at_tile_edges(channels, H, W):
         assert err <= tol, (k, err)
 
 
+@pytest.mark.parametrize("channels", [(32,), (16, 48), (64,)])
+def test_weight_gradients_over_many_tiles(channels):
+    """More than 256 tiles on the first level (its blocks hold every output
+    channel), fewer on the second (split over the channels), on a plan for a
+    larger field; the bound of test_weight_gradients_at_tile_edges."""
+    need_gpu()
+    H, W = 70, 1030
+    net = Lm.UNet(channels, H + 6, W + 70, seed=3)
+    Wt = {k: (v if k in ("e0a", "out") else Lm.to_bf16(v).astype(np.float64))
+          for k, v in net.get_weights().items()}
+    rng = np.random.default_rng(5)
+    x = Lm.to_bf16(rng.standard_normal((H, W))).astype(np.float64)
+    gy = Lm.to_bf16(rng.standard_normal((H, W))).astype(np.float64)
+    _, cache = U.forward(Wt, x, channels, bf16=True)
+    ref = U.backward(Wt, cache, gy, channels, bf16=True)
+    got = net.grads(torch.tensor(x, device="cuda"), torch.tensor(gy, device="cuda"))
+    tol = 4 * len(channels) * 2.0**-8
+    for k in ref:
+        err = np.linalg.norm(got[k] - ref[k]) / np.linalg.norm(ref[k])
+        assert err <= tol, (k, err)
+
+
 @pytest.mark.parametrize("cin,cout,ups", [(16, 16, False), (48, 32, True), (64, 48, False),
                                           (32, 64, False)])
 def test_conv_wide_tiles(cin, cout, ups):
