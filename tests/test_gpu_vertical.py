@@ -36,3 +36,19 @@ def test_layer_mode_roundtrip_gpu():
         assert_close_scaled(to_np(modes), fvx.layer_to_mode(f, l2m), tol, "l2m")
         back = fx.mode_to_layer(modes, m2l)
         assert_close_scaled(to_np(back), f, 10 * tol, "roundtrip")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-14), (torch.float32, 1e-6)])
+@pytest.mark.parametrize("nl", [1, 2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("ny,nx,offset", [(1, 1, 0), (7, 9, 0), (8, 33, 0), (8, 36, 0), (8, 36, 1)])
+def test_layer_mix_widths(ny, nx, offset, nl, dtype, tol):
+    """Every layer count, with and without 16-byte accesses (odd sizes, a view
+    that starts off a 16-byte boundary); sums of up to 8 products in FP64."""
+    need_gpu()
+    rng = np.random.default_rng(nl)
+    f, m = rng.standard_normal((nl, ny, nx)), rng.standard_normal((nl, nl))
+    buf = torch.zeros(offset + f.size, dtype=dtype, device="cuda")
+    t = buf[offset:].view(nl, ny, nx)
+    t.copy_(torch.tensor(f))
+    assert_close_scaled(to_np(fx.layer_to_mode(t, m)), fvx.layer_to_mode(f, m), tol, "mix")
