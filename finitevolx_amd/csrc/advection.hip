@@ -337,15 +337,17 @@ __device__ __forceinline__ T weno5_flux(T h0, T h1, T dm2, T dm1, T d0, T d1, T 
                                         bool near, int tier) {
   const bool pos = vel >= T(0);
   const T a1 = pos ? dm2 : d2, a2 = pos ? dm1 : d1, a4 = pos ? d1 : dm1;
+  // (a map may hold the largest stencil that fits, so 6 and above is 6)
+  const bool five = !MASKED || tier >= 6, three = tier == 4;
   T sd = T(0);
-  if (!MASKED || tier == 6) {
+  if (five) {
     if (near) sd = weno3_delta<T, Z>(a2, d0);
     else sd = weno5_delta<T, Z>(a1, a2, d0, a4);
-  } else if (tier == 4) {
+  } else if (three) {
     sd = weno3_delta<T, Z>(a2, d0);
   }
   const T f = ((pos ? h0 : h1) + (pos ? sd : -sd)) * vel;
-  return (!MASKED || tier >= 2) ? f : T(0);
+  return (five || three || tier == 2) ? f : T(0);
 }
 
 // One wavefront per tile of 58 output columns (lanes 3..60; three halo lanes

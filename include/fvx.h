@@ -61,9 +61,9 @@ int fvx_grad_perp_f64(const double* psi, double* u, double* v, int ny, int nx, d
 /* ---- Advection2D.__call__ (advection/advection.py:329-420) -----------------
  * method: FVX_ADV_*; limiter used when method == FVX_ADV_TVD.
  * tier_x / tier_y: NULL for the unmasked path, else per-cell largest usable
- * stencil in {0,2,4,6} (Mask2D.get_adaptive_masks, mask/cartesian.py:495-553)
- * for the mask-dispatchable methods (weno3, weno5, wenoz5, TVD;
- * advection/flux.py:100-253).  mask_h (nullable) multiplies the tendency.   */
+ * stencil in {0,2,4,6} (Mask2D.get_adaptive_masks, mask/cartesian.py:495-553;
+ * larger values count as 6) for the mask-dispatchable methods (weno3, weno5,
+ * wenoz5, TVD; advection/flux.py:100-253).  mask_h (nullable) multiplies the tendency.   */
 enum {
   FVX_ADV_NAIVE = 0, FVX_ADV_UPWIND1 = 1, FVX_ADV_UPWIND2 = 2, FVX_ADV_UPWIND3 = 3,
   FVX_ADV_WENO3 = 4, FVX_ADV_WENOZ3 = 5, FVX_ADV_WENO5 = 6, FVX_ADV_WENOZ5 = 7, FVX_ADV_TVD = 8

@@ -9,7 +9,8 @@ import pytest
 import torch
 
 import finitevolx_amd as fx
-from finitevolx_amd import inputs
+from finitevolx_amd import _lib, inputs
+from finitevolx_amd.advection import method_codes
 from oracle import fvx
 from tests.gpu_util import assert_close_scaled, need_gpu, random_mask, to_np
 
@@ -111,6 +112,41 @@ def test_masked_weno5_fp32_and_fp64(dtype, tol):
     got = fx.Advection2D(g, m)(torch.tensor(h, dtype=dtype), torch.tensor(u, dtype=dtype),
                                torch.tensor(v, dtype=dtype), "weno5")
     assert_close_scaled(to_np(got), ref, tol, f"masked weno5 {dtype}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("method", ["weno3", "weno5", "wenoz5", "van_leer"])
+@pytest.mark.parametrize("ny,nx", [(23, 70), (40, 200)])
+def test_tier_maps_beyond_the_schemes(ny, nx, method, dtype):
+    """Through the C ABI a tier map may hold the largest stencil that fits (8, 10,
+    ...): a scheme takes its own largest below it, so the map acts as its minimum
+    with 6 (bit for bit); no stencil (0) or none of the table (1, 3, 5): no flux.
+    Everywhere 6 is the unmasked scheme."""
+    need_gpu()
+    rng = np.random.default_rng(nx)
+    h, u, v = rng.standard_normal((3, ny, nx))
+    t = [torch.tensor(a, dtype=dtype, device="cuda") for a in (h, u, v)]
+    m, lim = method_codes(method)
+
+    def tend(tier):
+        tx, ty = (torch.tensor(k, dtype=torch.uint8, device="cuda") for k in tier)
+        out = torch.empty_like(t[0])
+        _lib.call(f"fvx_advection2d_{_lib.suffix(out)}", m, lim, *(a.data_ptr() for a in t),
+                  out.data_ptr(), tx.data_ptr(), ty.data_ptr(), None, ny, nx, 0.3, 0.4,
+                  _lib.stream())
+        return out
+
+    six = tend(np.full((2, ny, nx), 6))
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    assert_close_scaled(to_np(six), fvx.advection_2d(h, u, v, 0.3, 0.4, method), tol, method)
+    for k in (7, 8, 10, 255):
+        assert torch.equal(tend(np.full((2, ny, nx), k)), six), k
+    mixed = rng.choice([0, 2, 4, 6, 8, 10], size=(2, ny, nx))
+    assert torch.equal(tend(mixed), tend(np.minimum(mixed, 6)))
+    for k in (0, 1, 3, 5):
+        cap = 6 if method in ("weno5", "wenoz5") else 4
+        if k < cap:
+            assert not tend(np.full((2, ny, nx), k)).any(), k
 
 
 def test_rk3_step_rejects_bad_arguments():
