@@ -146,3 +146,25 @@ def test_conv_wide_tiles(cin, cout, ups):
     refb = Lm.to_bf16(ref)
     ulp = np.abs(refb).astype(np.float64) * 2.0**-7 + 1e-30
     assert np.all(np.abs(got - refb) <= ulp + 1e-6 * np.abs(ref).max())
+
+
+def test_output_layer_gradient_of_a_border_overflow():
+    """An activation that overflowed on the field's border counts for the taps
+    that reach it from inside and for no others: FP32 sums of the plain formula,
+    infinities included.  Activations here are 0 but for one pixel and channel."""
+    need_gpu()
+    C, H, W = 16, 6, 62
+    w = {"e0a": np.zeros((3, 3, C, 1)), "e0b": np.zeros((3, 3, C, C)), "out": np.zeros((3, 3, 1, C))}
+    w["e0a"][1, 1, 0, 0] = 1e20
+    w["e0b"][1, 1, 0, 0] = 1e20
+    for j, i in ((0, 0), (H - 1, W - 1), (0, 30), (2, 31)):
+        x = torch.zeros(H, W, device="cuda")
+        x[j, i] = 1.0
+        net = Lm.UNet((C,), H, W, weights=w)
+        got = net.grads(x, torch.ones(H, W, device="cuda"))["out"][:, :, 0, :]
+        want = np.zeros((3, 3, C))
+        for a in range(3):
+            for b in range(3):  # dW[a, b] = sum_p gy[p] d[p + (a - 1, b - 1)]
+                if 0 <= j - (a - 1) < H and 0 <= i - (b - 1) < W:
+                    want[a, b, 0] = np.inf
+        assert np.array_equal(got, want), (j, i, got[:, :, 0])
