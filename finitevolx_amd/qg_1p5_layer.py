@@ -66,7 +66,9 @@ _lib.extra_signatures({
 
 
 def _unmasked(op, cls) -> bool:
-    return type(op) is cls and op.mask is None
+    """Whether ``op`` is the package's own operator without a mask: no subclass,
+    and nothing set on the instance beyond its grid and mask (a method, say)."""
+    return type(op) is cls and op.mask is None and len(vars(op)) == 2
 
 
 def _gyre(q, psi, wind, grid, beta=0.0, drag=0.0, viscosity=0.0):

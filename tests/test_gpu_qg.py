@@ -279,6 +279,32 @@ def test_gyre_tendency_in_one_pass(ny, nx, dtype):
     assert not psi[0].any() and not psi[-1].any() and not psi[:, 0].any() and not psi[:, -1].any()
 
 
+def test_replaced_operator_methods_are_used():
+    """A method replaced on one of the model's operators takes part in the
+    tendency and in the velocities."""
+    need_gpu()
+    from finitevolx_amd import qg_1p5_layer as Q
+
+    model = Q.QG1p5LayerModel(Q.QuasiGeostrophicConfig(nx=20, ny=16))
+    psi = model.invert_streamfunction(model.q0)
+    plain = model.tendency(model.q0)
+    for name, op in (("laplacian", model.diff), ("diff_y_X_to_U", model.diff),
+                     ("T_to_X", model.interp), ("V_to_T", model.interp)):
+        own = getattr(op, name)
+        calls = []
+        setattr(op, name, lambda f, own=own: calls.append(name) or 2.0 * own(f))
+        changed = model.tendency(model.q0)
+        assert calls and not torch.equal(changed[0], plain[0]), name
+        calls.clear()
+        vel = Q.geostrophic_velocity_from_streamfunction(psi, model.diff, model.interp)
+        assert bool(calls) == (name in ("diff_y_X_to_U", "T_to_X")), name
+        if calls:
+            assert_close_scaled(to_np(vel[0]), 2.0 * to_np(plain[2]), 1e-12, name)
+        delattr(op, name)
+    for got, ref in zip(model.tendency(model.q0), plain):
+        assert torch.equal(got, ref)
+
+
 @pytest.mark.parametrize("nx,ny", [(64, 64), (48, 80)])
 def test_qg_1p5_layer_script_steps_match_oracle(nx, ny):
     """The reference example's composition (upwind1, X-point velocities, DST
