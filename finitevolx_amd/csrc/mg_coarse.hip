@@ -378,10 +378,12 @@ __device__ __forceinline__ void mg_coarse_lds_body(const CoarseArgs<T>& a,
   int low = 0;
   for (int d = 1; d < nd; ++d) low += (ny >> d) * (nx >> d);
   // LDS: scratch, u of level lc, then flat over the lower levels u (a zero
-  // cell after each), b and (no-flux) cx, cy, 1 / diag; wet masks as bytes.
+  // cell after each), b and (no-flux) cx, cy, 1 / diag per cell or (Dirichlet)
+  // 1 / diag per level; wet masks as bytes.
   T* sm = reinterpret_cast<T*>(coarse_smem);
-  T *fu = sm + 2 * (N + 1), *fb = fu + low + nd, *fx = fb + low, *fy = fx + low, *fi = fy + low;
-  uint8_t* wm = reinterpret_cast<uint8_t*>(NF ? fi + low : fx);
+  T *fu = sm + 2 * (N + 1), *fb = fu + low + nd, *fx = fb + low, *fy = fx + low,
+    *fi = NF ? fy + low : fx;
+  uint8_t* wm = reinterpret_cast<uint8_t*>(NF ? fi + low : fi + nd);
   S_ S{sm, L.lam, L.mask != nullptr};
   Geo g0{ny, nx, N, L.idx2, L.idy2, sm + N + 1, wm};
   auto lower = [&](int d, int off) {  // level lc + d, its flat offset
@@ -416,6 +418,9 @@ __device__ __forceinline__ void mg_coarse_lds_body(const CoarseArgs<T>& a,
     S.neighbours(g0, top, q, kc, j, i);
   }
   // ... and the lower levels' coefficients and masks, flat, into LDS.
+  if constexpr (!NF) {
+    if (tid < nd) fi[tid] = a.lv[a.lc + tid].inv_d;
+  }
   if (low > 0 && (NF || S.masked)) {
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
@@ -450,8 +455,8 @@ __device__ __forceinline__ void mg_coarse_lds_body(const CoarseArgs<T>& a,
   }
   __syncthreads();
 
-  // A lower level's cell of this thread, from LDS.
-  auto cell = [&](const Geo& g, int off, typename S_::template Cells<1>& r) {
+  // A cell of level lc + d of this thread, from LDS.
+  auto cell = [&](const Geo& g, int d, int off, typename S_::template Cells<1>& r) {
     const int kc = min(tid, g.N - 1), j = small_div(kc, 1.0f / g.nx), i = kc - j * g.nx;
     r.b[0] = fb[off + kc];
     r.wet = S.masked ? g.wm[kc] != 0 : 1;
@@ -462,8 +467,8 @@ __device__ __forceinline__ void mg_coarse_lds_body(const CoarseArgs<T>& a,
       r.yn[0] = fy[off + kc];
       r.ys[0] = j > 0 ? fy[off + kc - g.nx] : T(0);
     } else {
-      // 1 / diag of the level (the scalar of an all-wet level)
-      r.inv[0] = r.wet ? T(1) / (-T(2) * g.idx2 - T(2) * g.idy2 - S.lam) : T(0);
+      // (the scalar of an all-wet level)
+      r.inv[0] = r.wet ? fi[d] : T(0);
     }
     S.neighbours(g, r, 0, kc, j, i);
   };
@@ -478,7 +483,7 @@ __device__ __forceinline__ void mg_coarse_lds_body(const CoarseArgs<T>& a,
     for (int d = 1; d < nd; ++d) {
       const Geo g = lower(d, off);
       const bool last = d == nd - 1;
-      cell(g, off, r);
+      cell(g, d, off, r);
       S.sweeps(g, last ? a.n_coarse : a.n_pre, true, last ? a.w[2] : a.w[0], r);
       if (!last) {
         S.restrict_to(g, r, lower(d + 1, off + g.N), fb + off + g.N);
@@ -489,7 +494,7 @@ __device__ __forceinline__ void mg_coarse_lds_body(const CoarseArgs<T>& a,
       const Geo h = lower(d + 1, off);
       off -= (ny >> d) * (nx >> d);
       const Geo g = lower(d, off);
-      cell(g, off, r);
+      cell(g, d, off, r);
       S.prolong(g, h, r);
       S.sweeps(g, a.n_post, false, a.w[1], r);
     }
@@ -536,7 +541,7 @@ size_t coarse_lds_bytes(const CoarseArgs<T>& a, bool large) {
   }
   if (large) return 3 * all * sizeof(T);
   const size_t nd = a.nl - a.lc;
-  return (2 * (top + 1) + low + nd + (nf ? 4 : 1) * low) * sizeof(T) + all;
+  return (2 * (top + 1) + low + nd + (nf ? 4 * low : low + nd)) * sizeof(T) + all;
 }
 template size_t coarse_lds_bytes<float>(const CoarseArgs<float>&, bool);
 template size_t coarse_lds_bytes<double>(const CoarseArgs<double>&, bool);

@@ -505,3 +505,24 @@ def test_coarse_kernel_shapes(ny, nx, nl, kind, npre, npost, nco):
             assert_close_scaled(to_np(mg.v_cycle(None, bt)), ref, tol, f"V(0, b) {prec}")
             ref = fvx.v_cycle(levels, u0, b, **kw)
             assert_close_scaled(to_np(mg.v_cycle(ut, bt)), ref, tol, f"V(u0, b) {prec}")
+
+
+@pytest.mark.parametrize("precision", ["float64", "float32"])
+def test_coarse_kernel_inverse_diagonal(precision):
+    """The Dirichlet hierarchy's 1 / diag is an FP64 value rounded once, on the
+    lower levels of the single-workgroup kernel too: with no smoothing on the top
+    level and one bottom sweep of weight 1 from zero, b = 1 arrives below as 1 and
+    the corner cell of the cycle is 9 / 16 of the bottom's 1 / diag, bit for bit
+    (one rounding, of the product with 9)."""
+    need_gpu()
+    T = np.float32 if precision == "float32" else np.float64
+    dt = torch.float32 if precision == "float32" else torch.float64
+    n, m = 64, np.ones((64, 64))
+    for k in range(40):
+        dx, dy, lam = 1.0 / (7 + k), 1.0 / (11 + 0.37 * k), 3.0 + 0.7 * k
+        mg = S.build_multigrid_solver(m, dx, dy, lam, kind="dirichlet", precision=precision,
+                                      n_levels=3, n_pre=0, n_post=0, n_coarse=1, omega=1.0)
+        # level 1 (32^2) is the kernel's top level, level 2 its lower one
+        out = mg.v_cycle(None, torch.ones((n // 2, n // 2), dtype=dt, device="cuda"), level_idx=1)
+        inv = T(1.0 / (-2.0 / (4 * dx) ** 2 - 2.0 / (4 * dy) ** 2 - lam))
+        assert to_np(out)[0, 0] == float(T(9) * inv) / 16, (k, dx, dy, lam)
