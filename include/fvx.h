@@ -386,8 +386,9 @@ int fvx_spectral_helmholtz_f64(void* plan, const double* rhs, int64_t ld_rhs, do
                                void* stream);
 /* nb solves of contiguous (ny, nx) fields back to back, (lap - lambda_[b])
  * out_b = rhs_b (lambda_: host array of nb; pv_inversion's per-layer lambda,
- * solvers/elliptic.py:390-542); out may be rhs.  work: device scratch of
- * 2 nb ny nx elements that the call uses alone (null for bc 2). */
+ * solvers/elliptic.py:390-542); out may be rhs; nb 0 does nothing.  work:
+ * device scratch of 2 nb ny nx elements that the call uses alone (null for
+ * bc 2). */
 int fvx_spectral_helmholtz_batch_f32(void* plan, const float* rhs, float* out, int nb,
                                      const double* lambda_, double dx, double dy, float* work,
                                      void* stream);

@@ -123,3 +123,18 @@ def test_matrix_transforms_match_fft(bc, ny, nx, nb):
     assert_close_scaled(to_np(got), ref, 1e-13, f"{bc} f64")
     got = fx.pv_inversion(torch.tensor(f, dtype=torch.float32, device="cuda"), dx, dy, lam, bc=bc)
     assert_close_scaled(to_np(got), ref, 1e-6, f"{bc} f32")
+
+
+@pytest.mark.parametrize("solve", [fx.solve_helmholtz_dst, fx.solve_helmholtz_dct,
+                                   fx.solve_helmholtz_fft])
+@pytest.mark.parametrize("shape", [(0, 6, 5), (2, 0, 6, 5), (0, 5, 3100)])
+def test_empty_batch_solves_to_an_empty_array(solve, shape):
+    """No slice to solve: an empty result of the same shape, on every route; an
+    axis too short for a transform is refused as in a solve of some slices."""
+    need_gpu()
+    for dtype in (torch.float64, torch.float32):
+        f = torch.zeros(shape, dtype=dtype, device="cuda")
+        got = solve(f, 1.0, 1.0, 0.5)
+        assert got.shape == f.shape and got.dtype == dtype and got.is_cuda
+    with pytest.raises(ValueError):
+        solve(torch.zeros((0, 1, 5), device="cuda"), 1.0, 1.0, 0.5)
