@@ -530,7 +530,8 @@ def _spectral(rhs, dx, dy, lambda_, bc):
     plan = _spec_plan(ny, nx, bc, 64 if b.dtype == torch.float64 else 32)
     nb = b.numel() // (ny * nx) if b.numel() else 0
     out = torch.empty_like(b)
-    # (scratch of this call's stream: solves on several streams share a plan)
+    # (the matrix products' scratch, this call's own: solves on several streams
+    # share a plan; a plan of FFTs orders its uses, which share its scratch)
     work = None if bc == "fft" else torch.empty((2, *b.shape), dtype=b.dtype, device=b.device)
     lam = np.broadcast_to(np.asarray(lambda_, dtype=np.float64), b.shape[:-2]).ravel()
     _lib.call(f"fvx_spectral_helmholtz_batch_{_lib.suffix(b)}", plan.h, b.data_ptr(),

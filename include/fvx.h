@@ -375,7 +375,10 @@ int fvx_mg_batch_status(void* batch, int slot, int n_outer_budget, fvx_cg_info* 
  * outside the array), 1 = DCT-II (no-flux cell-centred Neumann), 2 = FFT
  * (periodic); each is the exact inverse of the matching 5-point operator.
  * The plan owns the transform matrices or hipFFT plans and work buffers of
- * one (ny, nx, bc, dtype). */
+ * one (ny, nx, bc, dtype).  Several threads and streams may share it: calls
+ * that work in its own buffers (all of an FFT plan, fvx_spectral_helmholtz_* of
+ * any) run one after the other on the device.  The replays of a graph that
+ * captured such a call are ordered by the program. */
 int fvx_spectral_plan_create(int ny, int nx, int bc, int precision, void** plan_out);
 int fvx_spectral_plan_destroy(void* plan);
 int fvx_spectral_helmholtz_f32(void* plan, const float* rhs, int64_t ld_rhs, float* out,

@@ -7,6 +7,8 @@ inverse of the 5-point operator it diagonalises (oracle operators), FP64 to
 1e-10 relative and FP32 to 1e-4.
 """
 
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -138,3 +140,56 @@ def test_empty_batch_solves_to_an_empty_array(solve, shape):
         assert got.shape == f.shape and got.dtype == dtype and got.is_cuda
     with pytest.raises(ValueError):
         solve(torch.zeros((0, 1, 5), device="cuda"), 1.0, 1.0, 0.5)
+
+
+@pytest.mark.parametrize("solve,shape,dtype", [
+    (fx.solve_helmholtz_fft, (2, 96, 160), torch.float64),
+    (fx.solve_helmholtz_fft, (700, 900), torch.float32),
+    (fx.solve_helmholtz_dst, (40, 3100), torch.float64),   # FFTs of the odd extension
+    (fx.solve_helmholtz_dct, (3, 300, 200), torch.float64)])  # matrix products
+def test_streams_and_threads_share_a_plan(solve, shape, dtype):
+    """Solves of one shape on several streams, enqueued by one thread and by
+    several, give what they give one at a time."""
+    need_gpu()
+    rng = np.random.default_rng(3)
+    fs = [torch.tensor(rng.standard_normal(shape), dtype=dtype, device="cuda") for _ in range(4)]
+    refs = [solve(f, 0.7, 1.1, 0.5) for f in fs]
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+
+    def run(k, out, rounds):
+        with torch.cuda.stream(streams[k % 3]):  # (two share a stream)
+            out += [(k, solve(fs[k], 0.7, 1.1, 0.5)) for _ in range(rounds)]
+
+    one, many = [], [[] for _ in fs]
+    for _ in range(8):
+        for k in range(4):
+            run(k, one, 1)
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=run, args=(k, many[k], 8)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    done = one + sum(many, [])
+    assert len(done) == 64
+    for k, got in done:
+        assert torch.equal(got, refs[k]), k
+
+
+def test_fft_solve_in_a_graph():
+    """A captured periodic solve replays, with eager solves of the plan between."""
+    need_gpu()
+    rng = np.random.default_rng(4)
+    f, h = (torch.tensor(rng.standard_normal((64, 96)), device="cuda") for _ in range(2))
+    ref, other = fx.solve_helmholtz_fft(f, 0.7, 1.1, 0.5), fx.solve_helmholtz_fft(h, 0.7, 1.1, 0.5)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        out = fx.solve_helmholtz_fft(f, 0.7, 1.1, 0.5)
+    for _ in range(4):
+        out.zero_()
+        g.replay()
+        assert torch.equal(fx.solve_helmholtz_fft(h, 0.7, 1.1, 0.5), other)
+        assert torch.equal(out, ref)
