@@ -626,8 +626,14 @@ static int launch_spec(const SpecGemm<T>& g, int nb, hipStream_t s) {
   return kOk;
 }
 
+// Scratch of a batched solve: two fields a slice of one launch; the FFTs have
+// theirs in the plan.
+static int64_t work_elements(const SpecPlan* P, int nb) {
+  return P->gemm ? (int64_t)2 * std::min(nb, kSpecBatch) * P->ny * P->nx : 0;
+}
+
 // nb solves (right-hand side b at rhs + b bs_rhs, solution at out + b bs_out,
-// its lambda in lam[b]) by matrix products; work: 2 nb ny nx elements.
+// its lambda in lam[b]) by matrix products; work: work_elements(P, nb).
 template <typename T>
 static int gemm_solve(SpecPlan* P, const T* rhs, int64_t ld_rhs, int64_t bs_rhs, T* out,
                       int64_t ld_out, int64_t bs_out, int nb, const double* lam, double dx,
@@ -636,7 +642,7 @@ static int gemm_solve(SpecPlan* P, const T* rhs, int64_t ld_rhs, int64_t bs_rhs,
   const int64_t N = (int64_t)ny * nx;
   for (int b0 = 0; b0 < nb; b0 += kSpecBatch) {
     const int m = std::min(kSpecBatch, nb - b0);
-    T *A = work + 2 * b0 * N, *B = A + m * N;
+    T *A = work, *B = A + m * N;  // (the launches before have read theirs)
     SpecGemm<T> g;
     std::memset(&g, 0, sizeof(g));
     for (int b = 0; b < m; ++b) g.lam[b] = lam[b0 + b];
@@ -801,10 +807,19 @@ int fvx_spectral_helmholtz_f32(void* plan, const float* rhs, int64_t ld_rhs, flo
       spec_solve<float>(P, rhs, ld_rhs, out, ld_out, dx, dy, lambda_, (hipStream_t)stream));
 }
 
+// Elements of the work array of a solve of nb slices.
+int fvx_spectral_work_size(void* plan, int nb, int64_t* elements) {
+  using namespace fvx;
+  FVX_CHECK_ARG(plan && elements, "null argument");
+  FVX_CHECK_ARG(nb >= 0, "negative batch");
+  *elements = work_elements((SpecPlan*)plan, nb);
+  return kOk;
+}
+
 // nb solves of contiguous (ny, nx) fields back to back, (lap - lambda_[b])
-// out_b = rhs_b (lambda_: host array); out may be rhs.  work: device scratch of 2 nb ny nx elements for the call (the caller's, so that calls on
-// several streams or threads do not share any); may be null for the periodic
-// boundary condition.
+// out_b = rhs_b (lambda_: host array); out may be rhs.  work: device scratch of
+// fvx_spectral_work_size elements for the call (the caller's, so that calls on
+// several streams or threads do not share any); may be null where that is 0.
 #define FVX_SPEC_BATCH(SUF, T, PREC)                                                             \
   int fvx_spectral_helmholtz_batch_##SUF(void* plan, const T* rhs, T* out, int nb,               \
                                          const double* lambda_, double dx, double dy, T* work,   \

@@ -481,6 +481,7 @@ def _generic_pcg(matvec, rhs, x0, precond, rtol, atol, max_steps, check_every=8)
 _lib.extra_signatures({
     "fvx_spectral_plan_create": [_i, _i, _i, _i, C.POINTER(_vp)],
     "fvx_spectral_plan_destroy": [_vp],
+    "fvx_spectral_work_size": [_vp, _i, C.POINTER(_i64)],
     "fvx_spectral_helmholtz_f64": [_vp, _vp, _i64, _vp, _i64, _d, _d, _d, _vp],
     "fvx_spectral_helmholtz_f32": [_vp, _vp, _i64, _vp, _i64, _d, _d, _d, _vp],
     "fvx_spectral_helmholtz_field_f64": [_vp, _vp, _vp, _d, _d, _d, _vp, _vp],
@@ -497,6 +498,17 @@ class _SpecPlan:
         h = _vp()
         _lib.call("fvx_spectral_plan_create", ny, nx, _BC[bc], bits, C.byref(h))
         self.h = h
+        # elements of scratch of one slice and, beyond some number, of all
+        one, most = _i64(), _i64()
+        _lib.call("fvx_spectral_work_size", h, 1, C.byref(one))
+        _lib.call("fvx_spectral_work_size", h, 2**31 - 1, C.byref(most))
+        self._work = one.value, most.value
+
+    def work(self, like, nb):
+        """Scratch of a call of ``nb`` slices (the call's own: solves on several
+        streams share a plan), or None where the plan's serves."""
+        n = min(nb * self._work[0], self._work[1])
+        return torch.empty(n, dtype=like.dtype, device=like.device) if n else None
 
     def __del__(self):
         if getattr(self, "h", None):
@@ -530,9 +542,7 @@ def _spectral(rhs, dx, dy, lambda_, bc):
     plan = _spec_plan(ny, nx, bc, 64 if b.dtype == torch.float64 else 32)
     nb = b.numel() // (ny * nx) if b.numel() else 0
     out = torch.empty_like(b)
-    # (the matrix products' scratch, this call's own: solves on several streams
-    # share a plan; a plan of FFTs orders its uses, which share its scratch)
-    work = None if bc == "fft" else torch.empty((2, *b.shape), dtype=b.dtype, device=b.device)
+    work = plan.work(b, nb)
     lam = np.broadcast_to(np.asarray(lambda_, dtype=np.float64), b.shape[:-2]).ravel()
     _lib.call(f"fvx_spectral_helmholtz_batch_{_lib.suffix(b)}", plan.h, b.data_ptr(),
               out.data_ptr(), nb, (_d * nb)(*lam), float(dx), float(dy), _lib.ptr(work),
@@ -547,9 +557,9 @@ def dirichlet_field_solve(field, dx, dy, lambda_):
     ny, nx = b.shape[0] - 2, b.shape[1] - 2
     plan = _spec_plan(ny, nx, "dst", 64 if b.dtype == torch.float64 else 32)
     out = torch.empty_like(b)
-    work = torch.empty((2, ny, nx), dtype=b.dtype, device=b.device)
+    work = plan.work(b, 1)
     _lib.call(f"fvx_spectral_helmholtz_field_{_lib.suffix(b)}", plan.h, b.data_ptr(),
-              out.data_ptr(), float(dx), float(dy), float(lambda_), work.data_ptr(),
+              out.data_ptr(), float(dx), float(dy), float(lambda_), _lib.ptr(work),
               _lib.stream())
     return out
 

@@ -387,11 +387,14 @@ int fvx_spectral_helmholtz_f32(void* plan, const float* rhs, int64_t ld_rhs, flo
 int fvx_spectral_helmholtz_f64(void* plan, const double* rhs, int64_t ld_rhs, double* out,
                                int64_t ld_out, double dx, double dy, double lambda_,
                                void* stream);
+/* Elements of the device scratch of the two solves below: 2 min(nb, 16) ny nx
+ * for a plan of transform matrices, 0 for one of FFTs (its own serves). */
+int fvx_spectral_work_size(void* plan, int nb, int64_t* elements);
 /* nb solves of contiguous (ny, nx) fields back to back, (lap - lambda_[b])
  * out_b = rhs_b (lambda_: host array of nb; pv_inversion's per-layer lambda,
  * solvers/elliptic.py:390-542); out may be rhs; nb 0 does nothing.  work:
- * device scratch of 2 nb ny nx elements that the call uses alone (null for
- * bc 2). */
+ * device scratch of fvx_spectral_work_size elements that the call uses alone
+ * (may be null where that is 0). */
 int fvx_spectral_helmholtz_batch_f32(void* plan, const float* rhs, float* out, int nb,
                                      const double* lambda_, double dx, double dy, float* work,
                                      void* stream);
@@ -400,7 +403,7 @@ int fvx_spectral_helmholtz_batch_f64(void* plan, const double* rhs, double* out,
                                      void* stream);
 /* One solve on the interior of full (ny + 2, nx + 2) fields (ny, nx: the
  * plan's): out's one-cell ring is written zero, rhs' ring is not read; out is
- * another array.  work: 2 ny nx elements, as above. */
+ * another array.  work: as above, of one slice. */
 int fvx_spectral_helmholtz_field_f32(void* plan, const float* rhs, float* out, double dx,
                                      double dy, double lambda_, float* work, void* stream);
 int fvx_spectral_helmholtz_field_f64(void* plan, const double* rhs, double* out, double dx,

@@ -193,3 +193,29 @@ def test_fft_solve_in_a_graph():
         g.replay()
         assert torch.equal(fx.solve_helmholtz_fft(h, 0.7, 1.1, 0.5), other)
         assert torch.equal(out, ref)
+
+
+def _peak_extra(call, *args):
+    """Bytes that a call holds at its peak beyond what it was given."""
+    call(*args)
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    call(*args)
+    return torch.cuda.max_memory_allocated() - base
+
+
+@pytest.mark.parametrize("solve,shape,works", [
+    (fx.solve_helmholtz_dst, (3, 40, 3100), 0), (fx.solve_helmholtz_dct, (2, 40, 3100), 0),
+    (fx.solve_helmholtz_fft, (3, 64, 96), 0),        # the plan's own scratch
+    (fx.solve_helmholtz_dst, (5, 64, 96), 10),
+    (fx.solve_helmholtz_dct, (100, 64, 96), 32)])    # launches of 16 share theirs
+def test_scratch_of_a_solve(solve, shape, works):
+    """A call's peak: its result and the matrix products' two fields a slice of a
+    launch, and nothing where a route has its scratch in the plan (allocations
+    round up to 512 bytes)."""
+    need_gpu()
+    f = torch.zeros(shape, dtype=torch.float64, device="cuda")
+    field = 8 * shape[-2] * shape[-1]
+    extra = _peak_extra(solve, f, 1.0, 1.0, 0.5)
+    assert extra <= f.numel() * 8 + works * field + 2048, (extra, works)
