@@ -765,7 +765,12 @@ struct UNet {
   // activations per level: x (pooled input, l > 0), h1e, e (=h2e), h1d, d
   std::vector<uint16_t*> xin, h1e, ee, h1d, dd, gA, gB, gC;
   float *rin = nullptr, *yout = nullptr, *gy = nullptr, *eref = nullptr;
-  float* part = nullptr;     // weight-gradient slots, each layer's from part_off
+  // Weight-gradient slots: of the layer with most (``widest``) in part, the
+  // others' from part_off in rest, which the first backward pass allocates;
+  // without rest every layer takes part and is summed before the next.
+  float *part = nullptr, *rest = nullptr;
+  size_t rest_elems = 0;
+  int widest = 0;
   std::vector<size_t> part_off;
   double* rms_part = nullptr;
   float* scal = nullptr;
@@ -880,15 +885,39 @@ static int bwdw_slots(const Layer& Ly, int H, int W) {
   const int nt = cdiv(W, kUTw) * cdiv(H, kUTh);
   return (int)std::min<size_t>(std::min(nt, kBwdwBlocks), (size_t)64 * 9 * 64 * 64 / n);
 }
-static void red_add(const UNet& N, int li, int nslot, RedTable& t) {
+static float* layer_part(const UNet& N, int li) {
+  return N.rest && li != N.widest ? N.rest + N.part_off[li] : N.part;
+}
+static void red_flush(RedTable& t, hipStream_t s) {
+  if (t.layers)
+    hipLaunchKernelGGL(reduce_slots_kernel, dim3(t.blocks), dim3(64 * kRedWaves), 0, s, t);
+  t = RedTable();
+}
+static void red_add(const UNet& N, int li, int nslot, RedTable& t, hipStream_t s) {
   const Layer& Ly = N.layers[li];
   auto& e = t.l[t.layers++];
-  e.part = N.part + N.part_off[li];
+  e.part = layer_part(N, li);
   e.out = N.g + Ly.off;
   e.nslot = nslot;
   e.n = 9 * Ly.cout * Ly.cin;
   e.block0 = t.blocks;
   t.blocks += cdiv(e.n, 64);
+  if (!N.rest) red_flush(t, s);
+}
+// The other layers' slots, with the first backward pass (plans that only run
+// forward hold none).  Under capture, where nothing can be allocated, or without
+// the memory, the passes go on layer by layer.
+static void take_slots(UNet& N, hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  void* p = nullptr;
+  if (N.rest) return;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone &&
+      hipMalloc(&p, N.rest_elems * sizeof(float)) == hipSuccess) {
+    N.allocs.push_back(p);
+    N.rest = (float*)p;
+  } else {
+    (void)hipGetLastError();
+  }
 }
 
 template <int PW, int RS, bool UPS>
@@ -904,7 +933,7 @@ static void launch_bwdw(float* part, const Layer& Ly, const uint16_t* x, const u
 static void bwdw_launch(UNet& N, int li, const uint16_t* x, const uint16_t* gyt, bool ups, int H,
                         int W, RedTable& red, hipStream_t s) {
   const Layer& Ly = N.layers[li];
-  float* part = N.part + N.part_off[li];
+  float* part = layer_part(N, li);
   const int tx = cdiv(W, kUTw), ty = cdiv(H, kUTh), nt = tx * ty;
   const int G = bwdw_slots(Ly, H, W);
   // Few tiles: a block per 16 output channels (and tile), which leaves each the
@@ -922,15 +951,15 @@ static void bwdw_launch(UNet& N, int li, const uint16_t* x, const uint16_t* gyt,
   else if (np <= 12) FVX_BWDW(3, 1);
   else FVX_BWDW(4, 1);
 #undef FVX_BWDW
-  red_add(N, li, G, red);
+  red_add(N, li, G, red, s);
 }
 
 static void edge_bwdw(UNet& N, int li, const float* s1, const uint16_t* sc, int C, bool swap,
                       int H, int W, RedTable& red, hipStream_t s) {
   const int G = bwdw_slots(N.layers[li], H, W);
   hipLaunchKernelGGL(edge_bwdw_kernel, dim3(G), dim3(256), 0, s, s1, sc, C, swap ? -1 : 1,
-                     N.part + N.part_off[li], H, W);
-  red_add(N, li, G, red);
+                     layer_part(N, li), H, W);
+  red_add(N, li, G, red, s);
 }
 
 // Backward from N.gy (dLoss/dy, fp32) to weight gradients accumulated in N.g.
@@ -939,6 +968,7 @@ static int unet_backward(UNet& N, int H, int W, hipStream_t s) {
   // output layer
   const Layer& o = N.layers.back();
   const uint16_t* d0 = (L > 1) ? N.dd[0] : N.ee[0];
+  take_slots(N, s);
   RedTable red;
   edge_bwdw(N, (int)N.layers.size() - 1, N.gy, d0, N.ch[0], false, H, W, red, s);
   hipLaunchKernelGGL(conv_last_bwd_data_kernel, g2(H, W), dim3(64, 4), 0, s, N.gy, N.w + o.off,
@@ -980,7 +1010,7 @@ static int unet_backward(UNet& N, int H, int W, hipStream_t s) {
                        (l - 1 <= L - 2) ? N.gB[l - 1] : nullptr, N.gA[l], N.ee[l - 1],
                        N.gA[l - 1], hf, wf, c);
   }
-  hipLaunchKernelGGL(reduce_slots_kernel, dim3(red.blocks), dim3(64 * kRedWaves), 0, s, red);
+  red_flush(red, s);
   FVX_LAUNCH_CHECK();
   return kOk;
 }
@@ -1070,14 +1100,18 @@ int fvx_unet_create(int nlev, const int* channels, int H, int W, void** out) {
   rc |= dev_alloc(*N, &N->yout, npx);
   rc |= dev_alloc(*N, &N->gy, npx);
   rc |= dev_alloc(*N, &N->eref, npx);
-  size_t slots = 0;
+  std::vector<size_t> slots;
   for (size_t li = 0; li < N->layers.size(); ++li) {
     const Layer& Ly = N->layers[li];
     const int k = (int)li, l = k < 2 * nlev ? k / 2 : (k == (int)N->layers.size() - 1 ? 0 : nlev - 2 - (k - 2 * nlev) / 2);
-    N->part_off.push_back(slots);
-    slots += (size_t)bwdw_slots(Ly, H >> l, W >> l) * 9 * Ly.cout * Ly.cin;
+    slots.push_back((size_t)bwdw_slots(Ly, H >> l, W >> l) * 9 * Ly.cout * Ly.cin);
+    if (slots[li] > slots[N->widest]) N->widest = (int)li;
   }
-  rc |= dev_alloc(*N, &N->part, slots);
+  for (size_t li = 0; li < slots.size(); ++li) {
+    N->part_off.push_back(N->rest_elems);
+    if ((int)li != N->widest) N->rest_elems += slots[li];
+  }
+  rc |= dev_alloc(*N, &N->part, slots[N->widest]);
   rc |= dev_alloc(*N, &N->rms_part, 4096);
   rc |= dev_alloc(*N, &N->scal, 4);
   rc |= dev_alloc(*N, &N->loss, 1);

@@ -19,6 +19,7 @@ import numpy as np
 import pytest
 import torch
 
+from finitevolx_amd import _lib
 from finitevolx_amd import learned as Lm
 from oracle import unet as U
 from tests.gpu_util import need_gpu
@@ -168,3 +169,54 @@ def test_output_layer_gradient_of_a_border_overflow():
                 if 0 <= j - (a - 1) < H and 0 <= i - (b - 1) < W:
                     want[a, b, 0] = np.inf
         assert np.array_equal(got, want), (j, i, got[:, :, 0])
+
+
+def test_gradient_slots_come_with_the_first_gradient():
+    """A plan that only runs forward holds no slots beyond one layer's; the first
+    gradient allocates them, further ones nothing."""
+    need_gpu()
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    Lm.UNet((16, 32, 48, 64), 64, 64, seed=0).grads(torch.zeros(64, 64), torch.zeros(64, 64))
+    net = Lm.UNet((16, 32, 48, 64), 512, 512, seed=0)
+    x = torch.randn(512, 512, device="cuda")
+    net.forward(x)
+    f0 = free()
+    first = net.grads(x, x)
+    f1 = free()
+    again = net.grads(x, x)
+    assert f0 - f1 >= 40 << 20, (f0, f1)
+    assert abs(f1 - free()) <= 4 << 20
+    for k in first:
+        assert np.array_equal(first[k], again[k]), k
+
+
+@pytest.mark.parametrize("channels", [(16,), (32, 64, 48)])
+def test_first_gradient_in_a_graph(channels):
+    """A plan's first backward pass may be a captured one (layer by layer in one
+    layer's slots); its replays, and eager passes between them, give what a plan
+    that never saw a capture gives, bit for bit."""
+    need_gpu()
+    H, W = 20, 132
+    x, gy = (torch.randn(H, W, device="cuda") for _ in range(2))
+    ref = Lm.UNet(channels, H, W, seed=1).grads(x, gy)
+    net = Lm.UNet(channels, H, W, seed=1)
+    flat = torch.zeros(sum(r.size for r in ref.values()), device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _lib.call("fvx_unet_backward_raw", net._h, x.data_ptr(), gy.data_ptr(), H, W,
+                  _lib.stream())
+    for k in range(4):
+        graph.replay()
+        _lib.call("fvx_unet_grads", net._h, flat.data_ptr(), 1, _lib.stream())
+        got = net._unflatten(flat.cpu().numpy())
+        for n in ref:
+            assert np.array_equal(got[n], ref[n]), (k, n)
+        if k:
+            got = net.grads(x, gy)
+            for n in ref:
+                assert np.array_equal(got[n], ref[n]), (k, n)
