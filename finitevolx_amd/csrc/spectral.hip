@@ -10,9 +10,9 @@
 //         -4/dx^2 sin^2(pi k / (2 n)); the k = l = 0 mode is set to zero
 //         when the operator is singular)
 //   fft : periodic (eigenvalues -4/dx^2 sin^2(pi k / n))
-// DST / DCT plans up to the sizes of use_gemm transform by matrix products on
+// DST / DCT plans of the sizes of use_gemm transform by matrix products on
 // the FP64 matrix cores (spec_gemm_kernel: four launches for a whole batch of
-// right-hand sides); larger ones by batched real FFTs (hipFFT) of the odd /
+// right-hand sides); others by batched real FFTs (hipFFT) of the odd /
 // even extension of each row, written transposed so the y transform is again a
 // batch of contiguous rows; periodic solves by hipFFT's 2-D real FFT.
 
@@ -198,16 +198,52 @@ static bool fft_smooth(int m) {
     while (m % p == 0) m /= p;
   return m == 1;
 }
-// Matrix products up to the size where the FFTs take less time (us a solve,
-// n^2, matrix / FFT).  FP64: direct lengths 768 110 / 132, 1000 168 / 155;
-// others 1024 160 / 397, 1536 508 / 636.  FP32 (products in FP64): direct 512
-// 52 / 67, 768 115 / 107; others 1024 175 / 230, 1200 300 / 278.
+// Whether a plan transforms by matrix products: where they take less time than
+// the FFTs did, by the two estimates below (us of a solve of one slice).  They
+// fit 451 shapes of 2 to 3000 points an axis, each timed both ways: the products
+// within 8% (FP64; 13% FP32) rms, the FFTs within 15%; the route took at most 1.2
+// times the faster one's time (1.4 with an axis of 2 points), a rule on ny + nx
+// alone up to 1.7.  Measured, products / FFTs:
+//            FP64                         FP32
+//   DCT  500 x  900    76 / 103      500 x 500    64 /  73     (direct lengths)
+//        800 x  900   150 / 133      128 x 1100   81 /  69
+//   DST  500 x  900    76 / 165      500 x 900    96 / 133     (others)
+//       1023 x 1800   449 / 349     1023 x 1100  299 / 186
+//         64 x 2900   135 / 158       64 x 1800  116 /  78
+static double products_us(int ny, int nx, int bits) {
+  double slabs = 0, second = 0, rounds = 0;  // of 64 points: all, > 256 blocks, > 512
+  const auto launch = [&](int k, int blocks) {
+    slabs += k;
+    second += blocks > 256 ? k : 0;
+    rounds += (double)k * (cdiv(blocks, 512) - 1);
+  };
+  const auto axis = [&](int n, int other) {
+    const int h = (n + 1) / 2, n1 = n / 2, o = cdiv(other, 32);
+    launch(cdiv(h, 64), o * (cdiv(h, 32) + cdiv(n1, 32)));
+    launch(cdiv(h, 64) + cdiv(n1, 64), o * cdiv(h, 32));
+  };
+  axis(nx, ny);
+  axis(ny, nx);
+  const double cells = (double)ny * nx;
+  return bits == 64 ? 9.3 + 1.43 * slabs + 0.4 * second + 1.78 * rounds + 4.24e-5 * cells
+                    : 10.8 + 1.71 * slabs + 1.76 * rounds + 7.58e-5 * cells;
+}
+static double ffts_us(int ny, int nx, int slow, int bits) {
+  // by the axes without a direct FFT (none, one, two; the last two again with an
+  // axis over 2047 points): us, ns a cell
+  static const double cost[2][5][2] = {
+      {{53, 0.101}, {68, 0.132}, {82, 0.2}, {115, 0.184}, {131, 0.206}},  // FP64
+      {{57, 0.06}, {68, 0.085}, {81, 0.13}, {95, 0.089}, {100, 0.13}}};   // FP32
+  const double* c = cost[bits == 64 ? 0 : 1][slow + (slow && std::max(ny, nx) > 2047 ? 2 : 0)];
+  return c[0] + 1e-3 * c[1] * ny * nx;
+}
 static bool use_gemm(int ny, int nx, int bc, int bits) {
   if (bc == kFft) return false;
   const int ext = bc == kDst ? 2 : 0;
-  const bool direct = fft_smooth(2 * nx + ext) && fft_smooth(2 * ny + ext);
-  const int most = bits == 64 ? (direct ? 1800 : 3072) : (direct ? 1400 : 2200);
-  return ny + nx <= most;
+  const int slow = !fft_smooth(2 * nx + ext) + !fft_smooth(2 * ny + ext);
+  // (nothing beyond these sums was timed)
+  const int most = bits == 64 ? (slow ? 3072 : 1800) : (slow ? 2200 : 1400);
+  return ny + nx <= most && products_us(ny, nx, bits) <= ffts_us(ny, nx, slow, bits);
 }
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 

@@ -14,6 +14,7 @@ import pytest
 import torch
 
 import finitevolx_amd as fx
+from finitevolx_amd import solvers
 from oracle import fvx
 from tests.gpu_util import assert_close_scaled, need_gpu, to_np
 
@@ -219,3 +220,19 @@ def test_scratch_of_a_solve(solve, shape, works):
     field = 8 * shape[-2] * shape[-1]
     extra = _peak_extra(solve, f, 1.0, 1.0, 0.5)
     assert extra <= f.numel() * 8 + works * field + 2048, (extra, works)
+
+
+@pytest.mark.parametrize("bc,ny,nx,bits,products", [
+    ("dst", 512, 768, 64, True), ("dct", 256, 700, 64, True), ("dst", 500, 900, 32, True),
+    ("dct", 300, 32, 32, True), ("dst", 128, 2150, 64, True), ("dst", 2, 300, 32, True),
+    ("dct", 1023, 1100, 32, False), ("dst", 1100, 1023, 32, False), ("dst", 64, 1800, 32, False),
+    ("dct", 2047, 32, 32, False), ("dst", 800, 2047, 64, False), ("dct", 1023, 1800, 64, False),
+    ("fft", 64, 64, 64, False)])
+def test_route_takes_the_faster_transform(bc, ny, nx, bits, products):
+    """Shapes at which one side was measured at least 1.25 times as fast."""
+    need_gpu()
+    plan = solvers._SpecPlan(ny, nx, bc, bits)
+    like = torch.zeros(1, dtype=torch.float64 if bits == 64 else torch.float32, device="cuda")
+    work = plan.work(like, 1)
+    assert (work is not None) == products
+    assert work is None or work.numel() == 2 * ny * nx
