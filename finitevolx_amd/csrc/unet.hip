@@ -71,8 +71,8 @@ __global__ void pack_weights_kernel(const float* __restrict__ w, uint16_t* __res
 // rows x NB pixel blocks) and its share of the input tile together, then the
 // tile goes to LDS (pixel pitch Cin + 8: the 16 pixels of a fragment read lie
 // on different banks) and the matrix instructions run from registers and LDS.
-// NB = 1 where NB = 4 would leave CUs idle (conv_launch).  Measured: 64 -> 64
-// channels at 64^2 7.8 us, 48 -> 48 at 128^2 6.7 us, 16 -> 16 at 512^2 9.9 us
+// NB = 1 or 2 (conv_launch).  Measured: 64 -> 64
+// channels at 64^2 7.8 us, 48 -> 48 at 128^2 6.7 us, 16 -> 16 at 512^2 9.0 us
 // (one wave per row with the weights fetched between the matrix instructions:
 // 31.5, 23.8 and 14.5 us).
 // ---------------------------------------------------------------------------
@@ -804,15 +804,25 @@ static void conv_launch(const UNet& N, int li, bool transposed, const uint16_t* 
   const Layer& Ly = N.layers[li];
   const int cout = transposed ? Ly.cin : Ly.cout, cin = transposed ? Ly.cout : Ly.cin;
   const bf16x4* wp = (const bf16x4*)((transposed ? N.wpkT : N.wpk) + N.pk_off[li]);
-  // Tiles 64 pixels wide (halo 1.5x) where they fill the chip with several
-  // workgroups per CU, else 16 wide (halo 1.7x) for four times the workgroups.
-  const bool wide = cdiv(W, 64) * cdiv(H, kUTh) >= 1024;
-  const int tx = cdiv(W, wide ? 64 : 16), nt = tx * cdiv(H, kUTh);
+  // Tiles 16 pixels wide (halo 1.7x): many workgroups, which hide each other's
+  // loads.  32 wide (halo 1.6x) on large fields with few output channels, which
+  // are nearer the memory than the matrix cores.  us, 16 / 32 / 64 wide:
+  //   16 -> 16 channels  256 x 512  7.5 /  7.5 /  7.8   512^2 10.4 /  9.0 /  9.8
+  //                         1024^2 25.0 / 19.3 / 20.6  2048^2   83 /   61 /   59
+  //   48 -> 32           256 x 512 13.9 / 13.3 / 14.6  1024^2 68.6 / 59.5 / 81.4
+  //   32 -> 48              512^2  20.3 / 21.6 / 27.1  2048^2  286 /  241 /  318
+  //   48 -> 48              512^2  24.7 / 34.7 / 50.2  2048^2  359 /  473 /  740
+  //   64 -> 64              512^2  40.7 / 44.6 / 57.1  2048^2  598 /  590 /  844
+  // (64 wide: one wave a SIMD with 48 and 64 channels, whose weights, accumulators
+  // and staging fill its registers).
+  const bool wide = cout <= 32 && cdiv(W, 64) * cdiv(H, kUTh) >= 1024;
+  const int tx = cdiv(W, wide ? 32 : 16), nt = tx * cdiv(H, kUTh);
 #define FVX_CONV_NB(COB, CIB, NB)                                                              \
   hipLaunchKernelGGL((conv_mfma_kernel<COB, CIB, NB>), dim3(nt), dim3(conv_threads(COB)), 0, s, x, \
                      wp, out, skip, maskt, relu ? 1 : 0, ups ? 1 : 0, H, W, tx, nt, N.guard)
 #define FVX_CONV(COB, CIB)                   \
-  if (wide) FVX_CONV_NB(COB, CIB, 4);        \
+  if constexpr (COB > 2) FVX_CONV_NB(COB, CIB, 1); \
+  else if (wide) FVX_CONV_NB(COB, CIB, 2);   \
   else FVX_CONV_NB(COB, CIB, 1)
 #define FVX_CONV_CI(COB)                     \
   switch (cin / 16) {                        \

@@ -135,8 +135,9 @@ def test_weight_gradients_over_many_tiles(channels):
 @pytest.mark.parametrize("cin,cout,ups", [(16, 16, False), (48, 32, True), (64, 48, False),
                                           (32, 64, False)])
 def test_conv_wide_tiles(cin, cout, ups):
-    """Enough rows for the 64-pixel tiles, whose last column holds 2 pixels
-    and whose last row of tiles 2 rows; the bound of test_single_conv_mfma."""
+    """Enough rows for the wide tiles (up to 32 output channels; the others take
+    16 pixels), whose last column holds 2 pixels and whose last row of tiles 2
+    rows; the bound of test_single_conv_mfma."""
     need_gpu()
     rng = np.random.default_rng(1)
     Hx, Wx = (685, 65) if ups else (1370, 130)
