@@ -1,8 +1,8 @@
 """Flux-form advection (drop-in for ``Advection2D``, ``advection/advection.py:283-420``).
 
-Every method runs as one fused HIP kernel: LDS-staged tracer tile,
-one upwind-selected reconstruction per face, flux divergence, mask and the
-zero 2-cell output ring in the same pass.  With a mask, the WENO3/WENO5/
+Every method runs as one fused HIP kernel: a tracer tile per wavefront in
+registers, one upwind-selected reconstruction per face, flux divergence, mask
+and the zero 2-cell output ring in the same pass.  With a mask, the WENO3/WENO5/
 WENO-Z5/TVD methods dispatch per face on the upwind cell's stencil tier
 (``advection/flux.py:100-253``); other methods run unmasked and the result
 is multiplied by ``mask.h`` (``advection.py:363-419``).

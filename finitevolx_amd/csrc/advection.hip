@@ -281,17 +281,14 @@ struct StageCoef {
   int ng = 0, images = 0;
 };
 
-// Face value from the stencil mirrored to the upwind side of the face:
-// m[k + 2] = h[i + k] for flow towards +x (k = -2 .. 2, the face between
-// cells i and i+1) and h[i + 1 - k] for flow towards -x.  Every scheme's
-// negative-flow formula is its positive-flow formula on the mirrored stencil
-// (weno.py:413-491 against :297-410, reconstruction.py:636-1050), so one
-// branch-free evaluation serves both signs.  ``near``: the face next to the
-// array edge on the upwind side (face 1 for positive, n-3 for negative flow),
-// where the 5-point schemes fall back to the 3-point ones.
+// Face value of the schemes of up to three points from the stencil mirrored to
+// the upwind side of the face: (hm1, h0, h1) = h[i - 1], h[i], h[i + 1] for flow
+// towards +x through the face between cells i and i+1, h[i + 2], h[i + 1], h[i]
+// for flow towards -x.  Every scheme's negative-flow formula is its positive-flow
+// formula on the mirrored stencil (weno.py:413-459 against :297-347,
+// reconstruction.py:636-1050), so one branch-free evaluation serves both signs.
 template <typename T, int M, int L>
-__device__ __forceinline__ T upwind_value(const T (&m)[5], bool near) {
-  const T hm1 = m[1], h0 = m[2], h1 = m[3];
+__device__ __forceinline__ T upwind_value(T hm1, T h0, T h1) {
   if constexpr (M == kNaive) return T(0.5) * (h0 + h1);
   if constexpr (M == kUpwind1) return h0;
   if constexpr (M == kUpwind2) return T(1.5) * h0 - T(0.5) * hm1;
@@ -299,11 +296,6 @@ __device__ __forceinline__ T upwind_value(const T (&m)[5], bool near) {
     return T(-1.0 / 6.0) * hm1 + T(5.0 / 6.0) * h0 + T(1.0 / 3.0) * h1;
   if constexpr (M == kWeno3) return weno3_left(hm1, h0, h1);
   if constexpr (M == kWenoZ3) return wenoz3_left(hm1, h0, h1);
-  if constexpr (M == kWeno5 || M == kWenoZ5) {
-    constexpr bool Z = (M == kWenoZ5);
-    if (near) return Z ? wenoz3_left(hm1, h0, h1) : weno3_left(hm1, h0, h1);
-    return weno5_upwind<T, Z>(m[0], hm1, h0, h1, m[4]);
-  }
   if constexpr (M == kTvd) {
     const T eps = T(1e-8);
     const T dfwd = h1 - h0, dbwd = h0 - hm1;
@@ -314,16 +306,13 @@ __device__ __forceinline__ T upwind_value(const T (&m)[5], bool near) {
 
 // The masked tier dispatch of face_flux on the mirrored stencil.
 template <typename T, int M, int L, bool MASKED>
-__device__ __forceinline__ T upwind_face(const T (&m)[5], bool near, int tier) {
+__device__ __forceinline__ T upwind_face(T hm1, T h0, T h1, int tier) {
   if constexpr (!MASKED) {
-    return upwind_value<T, M, L>(m, near);
+    return upwind_value<T, M, L>(hm1, h0, h1);
   } else {
-    constexpr int cap = (M == kWeno5 || M == kWenoZ5) ? 6 : 4;
-    constexpr int M4 = (M == kWenoZ5) ? kWenoZ3 : (M == kTvd ? kTvd : kWeno3);
-    const int t = tier < cap ? tier : cap;
-    if (t == 2) return upwind_value<T, kUpwind1, L>(m, near);
-    if (t == 4) return upwind_value<T, M4, L>(m, near);
-    if (t == 6) return upwind_value<T, M, L>(m, near);
+    constexpr int M4 = M == kTvd ? kTvd : kWeno3;
+    if (tier == 2) return h0;
+    if (tier >= 4) return upwind_value<T, M4, L>(hm1, h0, h1);
     return T(0);
   }
 }
@@ -331,7 +320,9 @@ __device__ __forceinline__ T upwind_face(const T (&m)[5], bool near, int tier) {
 // WENO5 / WENO-Z5 flux through the face between values h0 and h1, from the
 // differences around it (dk between cells k and k + 1 of the face's cell 0):
 // the upwind cell's value plus or minus the oriented weno5_delta; the masked
-// tier dispatch as upwind_face.
+// tier dispatch of face_flux.  ``near``: the face next to the array edge on the
+// upwind side (face 1 for positive, n - 3 for negative flow), where these schemes
+// fall back to the 3-point ones.
 template <typename T, bool Z, bool MASKED>
 __device__ __forceinline__ T weno5_flux(T h0, T h1, T dm2, T dm1, T d0, T d1, T d2, T vel,
                                         bool near, int tier) {
@@ -478,10 +469,8 @@ __device__ __forceinline__ void advection_tile(const AdvArgs<T>& a, int i0, int 
       f = weno5_flux<T, Z, MASKED>(hr[r], hr[r + 1], dy_[r - 2], dy_[r - 1], dy_[r], dy_[r + 1],
                                    dy_[r + 2], vel, near, tier);
     } else {
-      const T m[5] = {pos ? hr[r - 2] : hr[r + 3], pos ? hr[r - 1] : hr[r + 2],
-                      pos ? hr[r] : hr[r + 1], pos ? hr[r + 1] : hr[r],
-                      pos ? hr[r + 2] : hr[r - 1]};
-      f = upwind_face<T, M, L, MASKED>(m, near, tier) * vel;
+      f = upwind_face<T, M, L, MASKED>(pos ? hr[r - 1] : hr[r + 2], pos ? hr[r] : hr[r + 1],
+                                       pos ? hr[r + 1] : hr[r], tier) * vel;
     }
     fn[t] = INNER || (colin && gi >= 2 && gi <= nx - 3 && fj >= 1 && fj <= ny - 3) ? f : T(0);
   }
@@ -505,9 +494,8 @@ __device__ __forceinline__ void advection_tile(const AdvArgs<T>& a, int i0, int 
       const T d0 = e1 - hc, dm1 = adv_w(d0), dm2 = adv_w(dm1), d1 = adv_e(d0), d2 = adv_e(d1);
       fe = weno5_flux<T, Z, MASKED>(hc, e1, dm2, dm1, d0, d1, d2, vel, near, tier);
     } else {
-      const T e2 = adv_e(e1), e3 = adv_e(e2), w1 = adv_w(hc), w2 = adv_w(w1);
-      const T m[5] = {pos ? w2 : e3, pos ? w1 : e2, pos ? hc : e1, pos ? e1 : hc, pos ? e2 : w1};
-      fe = upwind_face<T, M, L, MASKED>(m, near, tier) * vel;
+      const T e2 = adv_e(e1), w1 = adv_w(hc);
+      fe = upwind_face<T, M, L, MASKED>(pos ? w1 : e2, pos ? hc : e1, pos ? e1 : hc, tier) * vel;
     }
     if constexpr (!INNER)
       fe = colin && gj >= 2 && gj <= ny - 3 && gi >= 1 && gi <= nx - 3 ? fe : T(0);

@@ -1867,8 +1867,7 @@ constexpr bool strip_levels() {
 template <typename T, int MODE>
 static void tile_weights(const Plan& P, TileArgs<T>& a, bool uniform) {
   constexpr int role = (MODE == kDown || MODE == kDownUpd) ? 0 : (MODE == kSmooth ? 2 : 1);
-  a.omega = (T)P.omega;
-  for (int k = 0; k < 3; ++k) a.omw[k] = uniform ? a.omega : (T)P.omw[role][k];
+  for (int k = 0; k < 3; ++k) a.omw[k] = uniform ? (T)P.omega : (T)P.omw[role][k];
 }
 
 template <typename T, int KIND, int NS, int MODE, bool ZERO>
@@ -2060,8 +2059,9 @@ static T* smooth_chunks(const Plan& P, const LevelDev<T>& L, const T* u_in, bool
 // One V-cycle z = V(u0 or 0, rhs) from level l0 (rhs, u0 and out have that
 // level's shape; MultigridSolver.v_cycle(u, rhs, level_idx), multigrid.py:
 // 808-883).  With ``az`` given (level 0 only), the last kernel also writes
-// az = A z and the PCG dots against rhs and w (kUpCG) when it can (two or
-// fewer post-sweeps on a tiled level 0); *fused says whether it did.
+// az = A z and the PCG dots against rhs and w (kUpCG) when it can (a level 0
+// above the coarse kernel whose post-sweeps fit one launch); *fused says whether
+// it did.
 // The coarse kernel's sweep weights (omega, or the plan's Chebyshev weights).
 template <typename T>
 static void coarse_weights(const Plan& P, CoarseArgs<T>& ca) {
@@ -2102,7 +2102,6 @@ static int v_cycle_impl(Plan& P, const T* u0, const T* rhs, T* out, T* az, const
     ca.n_post = P.n_post;
     ca.n_coarse = P.n_coarse;
     ca.nonzero_init = u0 != nullptr;
-    ca.omega = (T)P.omega;
     coarse_weights(P, ca);
     ca.done = sc ? &sc->done : nullptr;
     launch_coarse<T, KIND>(ca, s);
@@ -2148,7 +2147,6 @@ static int v_cycle_impl(Plan& P, const T* u0, const T* rhs, T* out, T* az, const
     ca.n_pre = P.n_pre;
     ca.n_post = P.n_post;
     ca.n_coarse = P.n_coarse;
-    ca.omega = (T)P.omega;
     coarse_weights(P, ca);
     ca.done = sc ? &sc->done : nullptr;
     launch_coarse<T, KIND>(ca, s);
@@ -2968,7 +2966,8 @@ int fvx_mg_plan_create(const double* mask, const double* coeff, int ny, int nx, 
       P->lc = l;
       break;
     }
-  // The bottom level is always the coarse kernel's (even when it is large).
+  // The bottom level is lc at the latest: the coarse kernel runs it where it has
+  // at most kCoarseCells cells, the level kernels' sweeps where it is larger.
   if (P->lc > nl - 1) P->lc = nl - 1;
   if (nl == 1) P->lc = 0;
   else if (P->lc == 0) P->lc = 1;
@@ -3480,7 +3479,6 @@ static int batch_build_slot(MgBatch& B, int s) {
       std::memset(&a, 0, sizeof(a));
       a.L = L;
       a.C = H.lv[l + 1];
-      a.omega = (float)Pm.omega;
       a.partials = Pm.partials;
       a.sc = sc;
       a.tiles_x = cdiv(L.nx, kTx);
@@ -3555,7 +3553,6 @@ static int batch_build_slot(MgBatch& B, int s) {
         std::memset(&a, 0, sizeof(a));
         a.L = L;
         a.C = H.lv[1];
-        a.omega = (float)Pm.omega;
         a.partials = Pm.partials;
         a.sc = &Pm.sc[2 * s];
         // down leg after the step that takes (rc, qc) to (rn, qn)
@@ -3606,7 +3603,6 @@ static int batch_build_slot(MgBatch& B, int s) {
       c.n_post = Pm.n_post;
       c.n_coarse = Pm.n_coarse;
       c.nonzero_init = 0;
-      c.omega = (float)Pm.omega;
       coarse_weights(Pm, c);
       c.done = &sc->done;
       S.coarse_cells = std::max(S.coarse_cells, (int64_t)c.lv[c.lc].ny * c.lv[c.lc].nx);

@@ -21,7 +21,6 @@ struct CoarseArgs {
   LevelDev<T> lv[16];
   int lc, nl, n_pre, n_post, n_coarse;
   int nonzero_init;  // level lc starts from lv[lc].u instead of zero
-  T omega;
   T w[3][kMaxW];  // sweep weights: pre-smoothing, post-smoothing, bottom
   const int* done;
 };

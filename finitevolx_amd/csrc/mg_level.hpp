@@ -20,8 +20,8 @@ struct LevelDev {
   const T* inv;            // noflux inverse diagonal
   T* u;                    // iterate (coarse levels: error)
   T* b;                    // right-hand side (coarse levels: restricted residual)
-  T* t;                    // scratch (ping-pong for single-workgroup sweeps)
-  T* t2;                   // scratch for tiled sweep chains
+  T* t;                    // scratch of the level kernels: sweep chains, the up leg's result
+  T* t2;
   T* t3;
   // Dirichlet coarse levels with the wall correction: each dry or outside
   // neighbour adds wall_g / h^2 to the diagonal (a ghost value wall_g u_c
@@ -117,9 +117,8 @@ struct TileArgs {
   T* u_out;
   const T* w;
   T* az_out;
-  T omega;
-  T omw[3];  // wave-tile kernels: the weight of sweep k (= omega unless the
-             // plan smooths with Chebyshev weights)
+  T omw[3];  // the weight of sweep k (the plan's omega unless it smooths with
+             // Chebyshev weights)
   double* partials;
   PcgScalars* sc;
   int tiles_x, ntiles;

@@ -3,9 +3,9 @@
 // masked_laplacian and the periodic ghost fill.
 //
 // All kernels are HBM-bandwidth bound; each output element is written once
-// and each input element is read from HBM once (neighbour reuse comes from
-// L1/LDS).  Point ops use one thread per output on a 64 x 4 workgroup so a
-// wavefront covers 64 contiguous elements of a row.
+// and each input element is read from HBM once (neighbour reuse comes from L1,
+// registers and lane moves).  A wavefront covers 60 to 64 contiguous columns of
+// one or several rows.
 
 #include "fvx_common.hpp"
 
