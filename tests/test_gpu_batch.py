@@ -101,3 +101,39 @@ def test_batch_with_a_large_bottom_level():
         assert info.converged
         r = to_np(b) - fvx.apply_operator(to_np(x), lev)
         assert np.linalg.norm(r) <= 1.0001e-8 * np.linalg.norm(to_np(b))
+
+
+@pytest.mark.parametrize("kind", ["noflux", "dirichlet"])
+@pytest.mark.parametrize("shapes", [
+    ((48, 64), (64, 60), (40, 96)),            # every coarse level has at most 1024 cells
+    ((128, 128), (48, 64), (96, 160)),         # up to 4096
+    ((250, 130), (64, 96), (128, 128))])       # a bottom level over 4096
+def test_coarse_kernels_of_a_batch(shapes, kind):
+    """The coarse kernels by the size of their largest level, both operators,
+    masked (no-flux: variable coefficients).  Batch and the member's own solver
+    certify ||b - A x|| <= 1e-10 ||b||, checked with the oracle's operator; all
+    eigenvalues of A are at least lambda in magnitude, so the two solutions differ
+    by at most 2e-10 ||b|| / lambda on the wet cells."""
+    need_gpu()
+    rng = np.random.default_rng(9)
+    lam, mem = 0.5, []
+    for k, (ny, nx) in enumerate(shapes):
+        m = inputs.basin_mask(ny, nx, 30 + k).astype(np.float64)
+        coeff = rng.uniform(0.5, 2.0, (ny, nx)) if kind == "noflux" else None
+        own = S.build_multigrid_solver(m, 1.0, 1.0, lam, coeff, kind=kind, precision="mixed",
+                                       n_pre=2, n_post=2, n_coarse=8, omega=0.85)
+        lev = fvx.build_multigrid(m, 1.0, 1.0, lam, coeff, n_levels=1, kind=kind)[0]
+        mem.append((m, own, lev, rng.standard_normal((ny, nx)) * m))
+    batch = S.MultigridBatch([own for _, own, _, _ in mem])
+    bs = [torch.tensor(b, device="cuda") for *_, b in mem]
+    xs = [torch.zeros_like(b) for b in bs]
+    batch.enqueue(bs, xs, rtol=1e-10, n_outer=6, n_inner=(20,) * 6)
+    for (m, own, lev, b), bt, x, (info, _, _) in zip(mem, bs, xs, batch.status(n_outer=6)):
+        assert info.converged, (m.shape, info)
+        other, oi = own.pcg(bt, rtol=1e-10, atol=0.0, max_steps=200)
+        assert oi.converged
+        for sol in (x, other):
+            r = (b - fvx.apply_operator(to_np(sol), lev)) * m
+            assert np.linalg.norm(r) <= 1.0001e-10 * np.linalg.norm(b), m.shape
+        d = np.linalg.norm((to_np(x) - to_np(other)) * m)
+        assert d <= 2.0002e-10 * np.linalg.norm(b) / lam, (m.shape, d)
