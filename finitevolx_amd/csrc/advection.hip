@@ -351,8 +351,9 @@ __device__ __forceinline__ T weno5_flux(T h0, T h1, T dm2, T dm1, T d0, T d1, T 
 // Grids up to 512^2 take tiles of 2 rows: more wavefronts for the chip, a
 // shorter chain of loads and arithmetic per wavefront.
 //
-// Bound by issue slots (FP64 also by the FP64 pipe) and by the loads' latency,
-// so: differences instead of values (weno5_delta); every array of the tile
+// Bound by issue slots and by the loads' latency (2048^2 FP64 0.54 of the VALU's
+// issue peak and 0.47 of the bandwidth, FP32 0.68 and 0.38; masked 0.42 / 0.39 and
+// 0.54 / 0.35), so: differences instead of values (weno5_delta); every array of the tile
 // requested before the first flux (a stage's output may alias its h_n, so the
 // compiler does not move those loads up itself); and a tile away from every
 // edge (INNER: all but the outermost ring) runs without the clamps, zero

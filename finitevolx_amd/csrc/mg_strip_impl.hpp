@@ -13,9 +13,13 @@
 // arrive in chunks of four, the next chunk's loads issued before the current
 // chunk is swept.
 //
-// Bound: at 2048^2 (FP64, no-flux) the ~6 arrays of 33.5 MB a pass moves; the
-// LDS tiles this replaces spent their time on LDS traffic and barriers
-// (10 LDS accesses a cell and sweep) with too few waves to hide either.
+// Bound: at 2048^2 (FP64, no-flux) the ~6 arrays of 33.5 MB a pass moves (the up
+// leg with the dots 71 us, 4.6 TB/s); below, the march itself: at 1024^2 with six
+// sweeps 2.5 wavefronts a SIMD keep the VALU at 0.45 of its issue peak and the
+// memory at 0.29 (28 us), from 512^2 down a launch is one wavefront's rows one
+// after the other (8-16 us).  The LDS tiles this replaces spent their time on LDS
+// traffic and barriers (10 LDS accesses a cell and sweep) with too few waves to
+// hide either.
 // Halo: rows cost (len + 2H) / len, columns 64 / (64 - 2H); strip_rows picks
 // len, long strips where the level fills the chip with them.
 #pragma once
@@ -389,7 +393,16 @@ __global__ __launch_bounds__(256) void mg_strip_kernel(TileArgs<T> a, int len) {
 }
 
 // Rows per strip: as many as leave two wavefronts per SIMD (2048), at most 32
-// (the mask windows hold 64 rows with the halo), at least 4.
+// (the mask windows hold 64 rows with the halo), at least 4.  Short strips sweep
+// more halo rows than they keep, and are still the fastest where long ones would
+// leave SIMDs empty: us of a V-cycle with 3 (6) sweeps a leg, no-flux FP64, by
+// this rule / all levels with 4, 8, 16, 32 rows:
+//   256^2      52 (74)   / 52 (74)   58 (81)   70 (95)   92 (123)
+//   512^2      70 (101)  / 70 (101)  75 (105)  93 (127) 128 (169)
+//   1024^2    105 (149)  / 109 (161) 109 (153) 126 (171) 166 (217)
+//   600x1000   68 (155)  / 68 (155)  74 (169)  92 (205) 137 (295)
+//   2048^2    192 (253)  / 226 (370) 199 (292) 212 (278) 255 (319)
+// (FP32 and the Dirichlet operator likewise.)
 inline int strip_rows(int tiles_x, int ny) {
   int len = 32;
   while (len > 4 && (int64_t)tiles_x * cdiv(ny, len) < 2048) len /= 2;

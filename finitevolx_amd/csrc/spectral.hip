@@ -183,10 +183,12 @@ struct FftTypes<float> {
 // Why: for the extended lengths 2 (n + 1) hipFFT falls to Bluestein's method
 // at most n (n = 512: 1026 = 2 3^3 19), and each transform took an extension,
 // 3-4 FFT kernels and an extraction per right-hand side.  Arithmetic is FP64
-// for both precisions, each sum in chunks of 16 products.  Bound: FP64 matrix
-// cores (45 TFLOP/s with v_mfma_f64_16x16x4 alone; 64 TFLOP/s of plain FMAs
-// would need four times the LDS reads).  Measured: 3 x 512 x 768 DST 151 us a
-// solve (20 TFLOP/s) against 535 through hipFFT; error against long double
+// for both precisions, each sum in chunks of 16 products.  Bound: the chain of a
+// slab (two barriers, staging, both operands of every matrix instruction from
+// LDS): the matrix cores are busy 0.20 to 0.28 of the time, the VALU 0.13 to
+// 0.25, the memory 0.1 (v_mfma_f64_16x16x4 alone reaches 45 TFLOP/s; 64 TFLOP/s
+// of plain FMAs would need four times the LDS reads).  Measured: 3 x 512 x 768
+// DST 149 us a solve (20 TFLOP/s) against 535 through hipFFT; error against long double
 // 3.2e-16 to 4.4e-16 (FP32 data 3.6e-8 to 6.1e-8) from 64 to 512 points, hipFFT
 // 3.1e-16 to 7.6e-16 (1.4e-7 to 3.1e-7).
 // ---------------------------------------------------------------------------

@@ -64,16 +64,17 @@ __global__ void pack_weights_kernel(const float* __restrict__ w, uint16_t* __res
 // * (maskt > 0).  ups: x is (H/2, W/2) and read through nearest upsampling.
 //
 // A workgroup owns a tile of 16 NB x 4 pixels; its COB * RG waves take one
-// block of 16 output channels and 4 / RG rows each.  The layers hold too little
+// block of 16 output channels and 4 / RG rows each.  Most layers hold too little
 // work to be bound by anything but latency (64 -> 64 channels at 64^2: 36
-// matrix instructions per SIMD), so a launch is arranged as one round of
-// loads: every wave requests its 9 CIB weight fragments (each reused on its
+// matrix instructions per SIMD; large fields come to the VALU, 16 -> 16 at 1024^2
+// 0.68 of its issue peak, matrix cores 0.18), so a launch is arranged as one round
+// of loads: every wave requests its 9 CIB weight fragments (each reused on its
 // rows x NB pixel blocks) and its share of the input tile together, then the
 // tile goes to LDS (pixel pitch Cin + 8: the 16 pixels of a fragment read lie
-// on different banks) and the matrix instructions run from registers and LDS.
-// NB = 1 or 2 (conv_launch).  Measured: 64 -> 64
-// channels at 64^2 7.8 us, 48 -> 48 at 128^2 6.7 us, 16 -> 16 at 512^2 9.0 us
-// (one wave per row with the weights fetched between the matrix instructions:
+// on different banks; the four channel groups still meet, conflicts take 0.1 to
+// 0.2 of the cycles below 64 channels) and the matrix instructions run from
+// registers and LDS.  NB = 1 or 2 (conv_launch).  Measured: 64 -> 64 channels at
+// 64^2 7.5 us, 48 -> 48 at 128^2 6.5 us, 16 -> 16 at 512^2 9.0 us (one wave per row with the weights fetched between the matrix instructions:
 // 31.5, 23.8 and 14.5 us).
 // ---------------------------------------------------------------------------
 constexpr int conv_row_groups(int cob) { return cob == 1 ? 4 : cob == 2 ? 2 : 1; }
@@ -947,8 +948,10 @@ static void bwdw_launch(UNet& N, int li, const uint16_t* x, const uint16_t* gyt,
   const int tx = cdiv(W, kUTw), ty = cdiv(H, kUTh), nt = tx * ty;
   const int G = bwdw_slots(Ly, H, W);
   // Few tiles: a block per 16 output channels (and tile), which leaves each the
-  // x tile, a share of gy and of the products (gradient at 512^2, splitting up to 170,
-  // 256, 512 tiles: 598, 584-595, 594-611 us; never: 674 and up).
+  // x tile, a share of gy and of the products.  Gradient, us, splitting never / up
+  // to 64, 128, 256, 512 tiles: default network 128^2 475 / 422 426 420 430, 512^2
+  // 631 / 588 588 587 583, 1024^2 1366 / 1350 1293 1266 1267; channels (32, 48)
+  // 512^2 561 / 560 546 523 523, 1024^2 1786 / 1787 1733 1644 1643.
   const int cobn = G <= kBwdwSplit ? 1 : Ly.cout / 16;
   const int np = cobn * (Ly.cin / 16);  // (co, ci) block pairs of a block, 1 .. 16
 #define FVX_BWDW(PW, RS)                                                          \
