@@ -92,6 +92,8 @@ class Advection2D:
         ny, nx = h.shape
         tx = ty = mh = None
         if self.mask is not None:
+            if tuple(self.mask.shape) != (ny, nx):
+                raise ValueError(f"mask shape {self.mask.shape} != field shape {(ny, nx)}")
             mh = self.mask.device("h")
             if method in _MASK_DISPATCHABLE:
                 tx, ty = self.mask.device("tier_x"), self.mask.device("tier_y")

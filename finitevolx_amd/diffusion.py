@@ -112,9 +112,7 @@ class MomentumAdvection2D:
         if u.dim() != 2 or u.shape != v.shape:
             raise ValueError("u and v must share one 2-D shape")
         ny, nx = u.shape
-        m = [None] * 4
-        if self.mask is not None:
-            m = [self.mask.device(k) for k in ("h", "u", "v", "xy_corner_strict")]
+        m = _masks(self.mask, ("h", "u", "v", "xy_corner_strict"), u.shape)
         du, dv = torch.empty_like(u), torch.empty_like(u)
         _lib.call(f"fvx_momentum_advection2d_{_lib.suffix(u)}", u.data_ptr(), v.data_ptr(),
                   du.data_ptr(), dv.data_ptr(), _SCHEMES[scheme], *[_lib.ptr(t) for t in m],

@@ -159,6 +159,22 @@ def test_rk3_step_rejects_bad_arguments():
         adv.rk3_step(h, h, h, 0.1, "bogus")
 
 
+@pytest.mark.parametrize("shape", [(11, 12), (12, 13), (20, 30)])
+def test_masks_of_another_shape_are_refused(shape):
+    """Every masked tendency: its kernel reads the mask by the field's indices."""
+    need_gpu()
+    h = torch.zeros(12, 12, dtype=torch.float64, device="cuda")
+    g = fx.CartesianGrid2D.from_interior(10, 10, 1.0, 1.0)
+    m = fx.Mask2D(np.ones(shape, bool))
+    for call in (lambda: fx.Advection2D(g, m)(h, h, h, "weno5"),
+                 lambda: fx.Advection2D(g, m).rk3_step(h, h, h, 0.1, "weno5", ng=3),
+                 lambda: fx.MomentumAdvection2D(g, m)(h, h, "al"),
+                 lambda: fx.Diffusion2D(g, m)(h, 1.0), lambda: fx.Difference2D(g, m).grad_perp(h)):
+        with pytest.raises(ValueError, match="mask shape"):
+            call()
+
+
+
 RECON = ["naive", "upwind1", "upwind2", "upwind3", "weno3", "wenoz3", "weno5", "wenoz5"]
 
 
