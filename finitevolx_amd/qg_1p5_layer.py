@@ -65,10 +65,18 @@ _lib.extra_signatures({
 })
 
 
+# The methods that the one-kernel path stands for, as this package defines them.
+_METHODS = {cls: tuple((n, getattr(cls, n)) for n in names) for cls, names in (
+    (Difference2D, ("diff_y_X_to_U", "diff_x_X_to_V", "laplacian", "_op")),
+    (Interpolation2D, ("T_to_X", "V_to_T")), (Advection2D, ("__call__",)))}
+
+
 def _unmasked(op, cls) -> bool:
-    """Whether ``op`` is the package's own operator without a mask: no subclass,
-    and nothing set on the instance beyond its grid and mask (a method, say)."""
-    return type(op) is cls and op.mask is None and len(vars(op)) == 2
+    """Whether ``op`` is the package's own operator without a mask: no subclass, no
+    method replaced on the class, and nothing set on the instance beyond its grid
+    and mask (a method, say)."""
+    return (type(op) is cls and op.mask is None and len(vars(op)) == 2
+            and all(getattr(cls, n) is f for n, f in _METHODS[cls]))
 
 
 def _gyre(q, psi, wind, grid, beta=0.0, drag=0.0, viscosity=0.0):

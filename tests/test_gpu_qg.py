@@ -279,9 +279,10 @@ def test_gyre_tendency_in_one_pass(ny, nx, dtype):
     assert not psi[0].any() and not psi[-1].any() and not psi[:, 0].any() and not psi[:, -1].any()
 
 
-def test_replaced_operator_methods_are_used():
-    """A method replaced on one of the model's operators takes part in the
-    tendency and in the velocities."""
+@pytest.mark.parametrize("on_class", [False, True])
+def test_replaced_operator_methods_are_used(on_class, monkeypatch):
+    """A method replaced on one of the model's operators, or on its class, takes
+    part in the tendency and in the velocities."""
     need_gpu()
     from finitevolx_amd import qg_1p5_layer as Q
 
@@ -292,7 +293,11 @@ def test_replaced_operator_methods_are_used():
                      ("T_to_X", model.interp), ("V_to_T", model.interp)):
         own = getattr(op, name)
         calls = []
-        setattr(op, name, lambda f, own=own: calls.append(name) or 2.0 * own(f))
+        if on_class:
+            monkeypatch.setattr(type(op), name,
+                                lambda self, f, own=own: calls.append(name) or 2.0 * own(f))
+        else:
+            setattr(op, name, lambda f, own=own: calls.append(name) or 2.0 * own(f))
         changed = model.tendency(model.q0)
         assert calls and not torch.equal(changed[0], plain[0]), name
         calls.clear()
@@ -300,7 +305,10 @@ def test_replaced_operator_methods_are_used():
         assert bool(calls) == (name in ("diff_y_X_to_U", "T_to_X")), name
         if calls:
             assert_close_scaled(to_np(vel[0]), 2.0 * to_np(plain[2]), 1e-12, name)
-        delattr(op, name)
+        if on_class:
+            monkeypatch.undo()
+        else:
+            delattr(op, name)
     for got, ref in zip(model.tendency(model.q0), plain):
         assert torch.equal(got, ref)
 
